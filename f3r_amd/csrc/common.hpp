@@ -77,6 +77,11 @@ struct Context {
   int num_cu = 256;
   Reducer red;
   double *pinned = nullptr;  // host-pinned landing buffer for small reads
+  // scratch of the calls that need some between launches on this stream (the
+  // largest size asked for so far; a call uses it only until it returns, and
+  // calls on one context run one after another)
+  DevPtr work;
+  void *workspace(size_t bytes);
   void *na_scratch = nullptr;  // device address of f3r_vec_dot_noalloc's scratch on this device
 };
 

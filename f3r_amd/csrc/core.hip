@@ -329,8 +329,18 @@ std::shared_ptr<Context> ctx_create(int device) {
 Context::~Context() {
   if (stream) (void)hipStreamSynchronize(stream);
   red = Reducer();
+  work.reset();
   if (pinned) (void)hipHostFree(pinned);
   if (stream) (void)hipStreamDestroy(stream);
+}
+
+void *Context::workspace(size_t bytes) {
+  if (!work || work->bytes < bytes) {
+    F3R_HIP(hipStreamSynchronize(stream));  // the old buffer's last reader
+    work.reset();
+    work = dev_alloc(bytes);
+  }
+  return work->p;
 }
 
 double read_scalar(Context *c, const double *dev) {

@@ -61,10 +61,19 @@ struct MLPShared {  // 16-byte aligned rows: the MFMA operands are read as 8- an
 };
 
 __device__ void load_mlp(const MLPDev &m, MLPShared &sm, bool transpose) {
-  for (int t = threadIdx.x; t < kH * kNin; t += blockDim.x) sm.w1[t] = m.w1[t];
-  for (int t = threadIdx.x; t < kH * kH; t += blockDim.x) {
-    sm.w2[t] = m.w2[t];
-    if (transpose) sm.w2t[(t % kH) * kH + t / kH] = m.w2[t];
+  // 8 weights per load (the device copies are 256-byte aligned allocations)
+  for (int t = threadIdx.x; t < kH * kNin / 8; t += blockDim.x)
+    reinterpret_cast<u32x4 *>(sm.w1)[t] = reinterpret_cast<const u32x4 *>(m.w1)[t];
+  for (int t = threadIdx.x; t < kH * kH / 8; t += blockDim.x) {
+    const u32x4 w = reinterpret_cast<const u32x4 *>(m.w2)[t];
+    reinterpret_cast<u32x4 *>(sm.w2)[t] = w;
+    if (transpose) {
+      uint16_t e[8];
+      __builtin_memcpy(e, &w, 16);
+      const int o = t * 8 / kH, k0 = t * 8 % kH;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sm.w2t[(k0 + k) * kH + o] = e[k];
+    }
   }
   for (int t = threadIdx.x; t < kH; t += blockDim.x) {
     sm.b1[t] = m.p[kOffB1 + t];
@@ -124,9 +133,9 @@ __device__ __forceinline__ void mlp_rows(const MLPShared &sm, uint16_t *h1t, con
     for (int q = 0; q < 4; ++q) acc[nt][q] += sm.b2[nt * 16 + i];
 }
 
-// y[r] = MLP(features[r]) for every row
+// y[r] = MLP(features[r]) for every row, and with `s` the scale exp(clamp(y))
 __global__ __launch_bounds__(256) void k_mlp_forward(MLPDev m, const uint16_t *__restrict__ feat, int64_t n,
-                                                     float *__restrict__ y) {
+                                                     float *__restrict__ y, float *__restrict__ s) {
   __shared__ MLPShared sm;
   load_mlp(m, sm, false);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
@@ -150,7 +159,11 @@ __global__ __launch_bounds__(256) void k_mlp_forward(MLPDev m, const uint16_t *_
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int64_t r = r0 + 4 * g + q;
-        if (r < n) y[r] = part[q] + sm.b3;
+        if (r < n) {
+          const float v = part[q] + sm.b3;
+          y[r] = v;
+          if (s) s[r] = expf(fminf(fmaxf(v, -kYClamp), kYClamp));
+        }
       }
     }
     __syncthreads();
@@ -158,8 +171,12 @@ __global__ __launch_bounds__(256) void k_mlp_forward(MLPDev m, const uint16_t *_
 }
 
 // Backward: given gy[r] = dL/dy_r, every wave accumulates its share of the
-// parameter gradient and writes it to part[(block * 4 + wave) * kNParams + .];
+// parameter gradient in registers; the block adds its four waves' shares in
+// LDS, in wave order, and writes one slice part[block * kNParams + .];
 // k_grad_reduce then adds the slices in a fixed order.
+// Bound by the chain of MFMA and LDS steps of a 64-row tile (about 4.7 us at
+// one wave per SIMD, 75 us for 64^3 rows on 256 blocks), so two blocks run
+// per CU.
 __global__ __launch_bounds__(256) void k_mlp_backward(MLPDev m, const uint16_t *__restrict__ feat, int64_t n,
                                                       const float *__restrict__ gy, float *__restrict__ part) {
   __shared__ MLPShared sm;
@@ -270,35 +287,71 @@ __global__ __launch_bounds__(256) void k_mlp_backward(MLPDev m, const uint16_t *
   }
   gb3 += __shfl_xor(gb3, 16, 64);
   gb3 += __shfl_xor(gb3, 32, 64);
-  float *out = part + (int64_t)(blockIdx.x * 4 + wave) * kNParams;
+  // the four waves' shares, added in wave order in LDS (the weights and tiles
+  // are no longer read)
+  static_assert(sizeof(float) * kNParams <= sizeof(MLPShared), "the gradient slice reuses the block's LDS");
+  float *acc_s = reinterpret_cast<float *>(&sm);
+  for (int w = 0; w < 4; ++w) {
+    __syncthreads();
+    if (wave != w) continue;
+    auto put = [&](int k, float v) { acc_s[k] = w == 0 ? v : acc_s[k] + v; };
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
+    for (int mt = 0; mt < 4; ++mt) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int o = mt * 16 + 4 * g + q;
-      out[kOffW1 + o * kNin + i] = gw1[mt][q];
+      for (int q = 0; q < 4; ++q) {
+        const int o = mt * 16 + 4 * g + q;
+        put(kOffW1 + o * kNin + i, gw1[mt][q]);
 #pragma unroll
-      for (int it = 0; it < 4; ++it) out[kOffW2 + o * kH + it * 16 + i] = gw2[mt][it][q];
+        for (int it = 0; it < 4; ++it) put(kOffW2 + o * kH + it * 16 + i, gw2[mt][it][q]);
+      }
+    }
+    if (g == 0) {
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) {
+        put(kOffB1 + nt * 16 + i, gb1[nt]);
+        put(kOffB2 + nt * 16 + i, gb2[nt]);
+        put(kOffW3 + nt * 16 + i, gw3[nt]);
+      }
+      if (i == 0) put(kOffB3, gb3);
     }
   }
-  if (g == 0) {
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      out[kOffB1 + nt * 16 + i] = gb1[nt];
-      out[kOffB2 + nt * 16 + i] = gb2[nt];
-      out[kOffW3 + nt * 16 + i] = gw3[nt];
-    }
-    if (i == 0) out[kOffB3] = gb3;
-  }
+  __syncthreads();
+  float *out = part + (int64_t)blockIdx.x * kNParams;
+  for (int k = threadIdx.x; k < kNParams; k += blockDim.x) out[k] = acc_s[k];
 }
 
-// grad[k] += sum over slices s of part[s * kNParams + k], slices in order
-__global__ void k_grad_reduce(const float *__restrict__ part, int nslices, float *__restrict__ grad) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= kNParams) return;
+// grad[k] += sum over slices s of part[s * kNParams + k].  A block takes 64
+// parameters; wave w of its 16 sums slices w, w + 16, ... in order (every
+// load of a round of 8 in flight at once), then the 16 sums are added in wave
+// order.  One thread per parameter adding 1024 slices one after another was a
+// chain of 1024 loads, 243 us; this reads the same slices in 8 us (512 of them).
+constexpr int kGradWaves = 16;
+__global__ __launch_bounds__(64 * kGradWaves) void k_grad_reduce(const float *__restrict__ part, int nslices,
+                                                                 float *__restrict__ grad) {
+  __shared__ float lds[kGradWaves][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int k = blockIdx.x * 64 + lane;
   float s = 0.f;
-  for (int j = 0; j < nslices; ++j) s += part[(int64_t)j * kNParams + k];
-  grad[k] += s;
+  if (k < kNParams) {
+    for (int j0 = w; j0 < nslices; j0 += 8 * kGradWaves) {
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int j = j0 + q * kGradWaves;
+        v[q] = j < nslices ? part[(int64_t)j * kNParams + k] : 0.f;
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s += v[q];
+    }
+  }
+  lds[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && k < kNParams) {
+    float u = lds[0][lane];
+#pragma unroll
+    for (int q = 1; q < kGradWaves; ++q) u += lds[q][lane];
+    grad[k] += u;
+  }
 }
 
 // Adam on the fp32 master parameters, then refresh the bf16 copies
@@ -325,66 +378,121 @@ __global__ void k_refresh_bf16(const float *__restrict__ p, uint16_t *__restrict
   if (k < kH * kH) w2b[k] = f2bf(p[kOffW2 + k]);
 }
 
-// s = exp(clamp(y)); v = s * u
-__global__ void k_scale_from_y(int64_t n, const float *__restrict__ y, float *__restrict__ s) {
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-    s[i] = expf(fminf(fmaxf(y[i], -kYClamp), kYClamp));
+// ------------------------------------------- products over the probes ---
+// The loss applies five sparse products to every probe vector.  One launch
+// runs a product for a group of up to kProbeGroup probes (blockIdx.y = probe),
+// with what follows it in the epilogue: 8 probes on a 64^3 system are 7
+// launches of 2 M rows in place of 72 of 262 K rows, which took 4 to 6.5 us
+// each, most of it launch and drain.
+constexpr int kProbeGroup = 8;
+
+template <int K, class Epi>
+__global__ __launch_bounds__(kBlock) void k_probe_sell(SellArgs a, const float *__restrict__ val,
+                                                       const float *__restrict__ x, Epi epi) {
+  const int64_t off = (int64_t)blockIdx.y * a.n;
+  typename Epi::State st{};
+  for (int r = xcd_block() * kBlock + threadIdx.x; r < a.n; r += gridDim.x * kBlock)
+    epi.row(r, off + r, sell_row<float, float, float, K>(a, val, x + off, r), st);
+  epi.finish(st);
 }
-__global__ void k_mul(int64_t n, const float *__restrict__ a, const float *__restrict__ b, float *__restrict__ c) {
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-    c[i] = a[i] * b[i];
-}
-// r = z - q and ||r||^2, ||z||^2 (single-pass grid reduction)
-__global__ __launch_bounds__(kBlock) void k_resid_norms(int64_t n, const float *__restrict__ z,
-                                                        const float *__restrict__ q, float *__restrict__ r,
-                                                        float *partial, unsigned *counters, float *out) {
-  __shared__ float lds[2 * kWavesPerBlock];
-  float v[2] = {0.f, 0.f};
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const float ri = z[i] - q[i];
-    r[i] = ri;
-    v[0] = __builtin_fmaf(ri, ri, v[0]);
-    v[1] = __builtin_fmaf(z[i], z[i], v[1]);
+
+// y = A x
+struct EpiProbeStore {
+  using State = NoState;
+  float *__restrict__ y;
+  __device__ void row(int, int64_t at, float acc, State &) const { y[at] = acc; }
+  __device__ void finish(State &) const {}
+};
+// u = W^T z and v = s u
+struct EpiProbeScale {
+  using State = NoState;
+  float *__restrict__ u;
+  float *__restrict__ v;
+  const float *__restrict__ s;
+  __device__ void row(int r, int64_t at, float acc, State &) const {
+    u[at] = acc;
+    v[at] = s[r] * acc;
   }
-  if (grid_sum<float, 2>(v, partial, counters, lds) && threadIdx.x == 0) {
-    out[0] = v[0];
-    out[1] = v[1];
+  __device__ void finish(State &) const {}
+};
+// q = A M z.  kind 0: r = z - q and the sums ||r||^2, ||z||^2; kind 1: q and
+// the sums <z,q>, <q,q>, <z,z>.  Block sums into partial[(probe * 3 + sum) *
+// gridDim.x + block]; k_probe_norms adds them in the next launch.
+struct EpiProbeResid {
+  struct State {
+    float v[3];
+  };
+  float *__restrict__ out;
+  const float *__restrict__ z;
+  float *__restrict__ partial;
+  int kind;
+  __device__ void row(int, int64_t at, float acc, State &s) const {
+    const float zi = z[at];
+    const float o = kind == 0 ? zi - acc : acc;
+    out[at] = o;
+    s.v[0] = __builtin_fmaf(kind == 0 ? o : zi, o, s.v[0]);
+    s.v[1] = __builtin_fmaf(kind == 0 ? zi : o, kind == 0 ? zi : o, s.v[1]);
+    s.v[2] = __builtin_fmaf(zi, zi, s.v[2]);
   }
-}
-// <z, q>, <q, q>, <z, z> (single-pass grid reduction)
-__global__ __launch_bounds__(kBlock) void k_qdots(int64_t n, const float *__restrict__ z,
-                                                  const float *__restrict__ q, float *partial, unsigned *counters,
-                                                  float *out) {
-  __shared__ float lds[3 * kWavesPerBlock];
+  __device__ void finish(State &s) const {
+    __shared__ float lds[3 * kWavesPerBlock];
+    block_sum<float, 3>(s.v, lds);
+    if (threadIdx.x == 0)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) partial[((int64_t)blockIdx.y * 3 + k) * gridDim.x + blockIdx.x] = s.v[k];
+  }
+};
+// norms[4 probe + k] = the G block sums of sum k (block = probe, fixed order)
+__global__ __launch_bounds__(1024) void k_probe_norms(const float *__restrict__ partial, int G,
+                                                      float *__restrict__ norms) {
+  __shared__ float lds[3][16];
+  const float *__restrict__ p = partial + (int64_t)blockIdx.x * 3 * G;
   float v[3] = {0.f, 0.f, 0.f};
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    v[0] = __builtin_fmaf(z[i], q[i], v[0]);
-    v[1] = __builtin_fmaf(q[i], q[i], v[1]);
-    v[2] = __builtin_fmaf(z[i], z[i], v[2]);
+  for (int b = threadIdx.x; b < G; b += 1024)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[k] += p[(int64_t)k * G + b];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    v[k] = wave_sum(v[k]);
+    if ((threadIdx.x & (kWave - 1)) == 0) lds[k][threadIdx.x / kWave] = v[k];
   }
-  if (grid_sum<float, 3>(v, partial, counters, lds) && threadIdx.x == 0) {
-    out[0] = v[0];
-    out[1] = v[1];
-    out[2] = v[2];
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    float t = lds[threadIdx.x][0];
+    for (int w = 1; w < 16; ++w) t += lds[threadIdx.x][w];
+    norms[4 * blockIdx.x + threadIdx.x] = t;
   }
 }
-// r = <q,q> z - <z,q> q: minus the q-gradient of 1 - <z,q>^2 / (<z,z><q,q>),
-// up to the factor 2 <z,q> / (<z,z> <q,q>^2)
-__global__ void k_rscaled(int64_t n, const float *__restrict__ z, const float *__restrict__ q,
-                          const float *__restrict__ d, float *__restrict__ r) {
-  const float a = d[0], b = d[1];
+// r = <q,q> z - <z,q> q in place of q (blockIdx.y = probe): minus the
+// q-gradient of 1 - <z,q>^2 / (<z,z><q,q>), up to the factor
+// 2 <z,q> / (<z,z> <q,q>^2)
+__global__ void k_rscaled(int64_t n, const float *__restrict__ z, float *__restrict__ q,
+                          const float *__restrict__ norms) {
+  const float a = norms[4 * blockIdx.y], b = norms[4 * blockIdx.y + 1];
+  const int64_t off = (int64_t)blockIdx.y * n;
   for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-    r[i] = b * z[i] - a * q[i];
+    q[off + i] = b * z[off + i] - a * q[off + i];
 }
-// gy += c * g2 * u * s, zero where the clamp is active; c = -2 wgt / ||z||^2
-// (kind 0) or -2 wgt <z,q> / (<z,z> <q,q>^2) (kind 1)
-__global__ void k_gy(int64_t n, const float *__restrict__ g2, const float *__restrict__ u,
-                     const float *__restrict__ s, const float *__restrict__ y, const float *__restrict__ norms,
-                     int kind, float wgt, float *__restrict__ gy) {
-  const float c = kind == 0 ? -2.f * wgt / norms[1] : -2.f * wgt * norms[0] / (norms[2] * norms[1] * norms[1]);
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const bool live = fabsf(y[i]) < kYClamp;
-    gy[i] += live ? c * g2[i] * u[i] * s[i] : 0.f;
+// gy (+)= sum over the group's probes of c g2 u s with g2 = Z^T g1, zero where
+// the clamp is active; c = -2 wgt / ||z||^2 (kind 0) or
+// -2 wgt <z,q> / (<z,z> <q,q>^2) (kind 1)
+template <int K>
+__global__ __launch_bounds__(kBlock) void k_probe_gy(SellArgs a, const float *__restrict__ val,
+                                                     const float *__restrict__ g1, const float *__restrict__ u,
+                                                     const float *__restrict__ s, const float *__restrict__ y,
+                                                     const float *__restrict__ norms, int probes, int kind, float wgt,
+                                                     int first, float *__restrict__ gy) {
+  for (int r = xcd_block() * kBlock + threadIdx.x; r < a.n; r += gridDim.x * kBlock) {
+    const bool live = fabsf(y[r]) < kYClamp;
+    float t = first ? 0.f : gy[r];
+    for (int k = 0; k < probes; ++k) {
+      const float *__restrict__ nk = norms + 4 * k;
+      const float c = kind == 0 ? -2.f * wgt / nk[1] : -2.f * wgt * nk[0] / (nk[2] * nk[1] * nk[1]);
+      const int64_t off = (int64_t)k * a.n;
+      const float g2 = sell_row<float, float, float, K>(a, val, g1 + off, r);
+      t += live ? c * g2 * u[off + r] * s[r] : 0.f;
+    }
+    gy[r] = t;
   }
 }
 
@@ -396,7 +504,7 @@ namespace f3r {
 struct MLP {
   std::shared_ptr<Context> ctx;
   DevPtr p, mom, vel, w1b, w2b, part, grad;
-  int grid = 256;
+  int grid = 512;  // blocks of the backward pass: two per CU
   int64_t step = 0;
   MLPDev dev() const { return MLPDev{w1b->as<uint16_t>(), w2b->as<uint16_t>(), p->as<float>()}; }
 };
@@ -410,21 +518,25 @@ struct LSys {
     std::shared_ptr<SellShared> sh;
     DevPtr val;
   } A, At, Z, Zt, Wt;
-  DevPtr feat, y, s, u, v, pz, q, r, g1, g2, gy, norms, probes;
+  DevPtr feat, norms, probes;
   int32_t nprobes = 0;
 };
 
+// K = 4 slots per load for matrices of several entries per row, 1 for the
+// near-diagonal factors
 static LSys::M upload_f32(Context *c, const HostCSR &M) {
-  HostSell hs = build_sell(M, 64, 1, 1, nullptr, false, true);
+  HostSell hs = build_sell(M, 64, 1, M.nnz() >= (int64_t)3 * M.n ? 4 : 1, nullptr, false, true);
   LSys::M m;
   m.sh = upload_sell_shared(c, hs, false);
   m.val = upload_sell_values(c, hs, F3R_F32);
   return m;
 }
 
-static void spmv32(const LSys::M &m, const float *x, float *y, hipStream_t st) {
+template <class Epi>
+static void probe_sell(const LSys::M &m, const float *x, int probes, const Epi &epi, int grid, hipStream_t st) {
   SellArgs a = sell_args(*m.sh, false);
-  launch_sell<float, float, float>(m.sh->K, a, m.val->as<float>(), x, EpiStore<float, float>{y, nullptr}, st);
+  auto kern = m.sh->K == 4 ? k_probe_sell<4, Epi> : k_probe_sell<1, Epi>;
+  hipLaunchKernelGGL(kern, dim3(grid, probes), dim3(kBlock), 0, st, a, m.val->as<float>(), x, epi);
 }
 
 static HostCSR transpose_csr(const HostCSR &A) {
@@ -521,7 +633,7 @@ MLP *mlp_create(std::shared_ptr<Context> ctx, uint64_t seed) {
   m->grad = dev_alloc(4 * kNParams);
   m->w1b = dev_alloc(2 * kH * kNin);
   m->w2b = dev_alloc(2 * kH * kH);
-  m->part = dev_alloc((size_t)4 * kNParams * m->grid * 4);
+  m->part = dev_alloc((size_t)4 * kNParams * m->grid);
   hipStream_t st = ctx->stream;
   F3R_HIP(hipMemcpyAsync(m->p->p, p.data(), 4 * kNParams, hipMemcpyHostToDevice, st));
   F3R_HIP(hipMemsetAsync(m->mom->p, 0, 4 * kNParams, st));
@@ -538,15 +650,15 @@ static int fwd_grid(Context *c, int64_t n) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(t, (int64_t)c->num_cu * 4));
 }
 
-void mlp_forward_dev(MLP *m, const uint16_t *feat, int64_t n, float *y, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_forward, dim3(fwd_grid(m->ctx.get(), n)), dim3(256), 0, st, m->dev(), feat, n, y);
+void mlp_forward_dev(MLP *m, const uint16_t *feat, int64_t n, float *y, float *s, hipStream_t st) {
+  hipLaunchKernelGGL(k_mlp_forward, dim3(fwd_grid(m->ctx.get(), n)), dim3(256), 0, st, m->dev(), feat, n, y, s);
 }
 
 void mlp_backward_dev(MLP *m, const uint16_t *feat, int64_t n, const float *gy, hipStream_t st) {
   const int grid = std::min<int>(m->grid, (int)std::max<int64_t>(1, (n + 63) / 64));
   hipLaunchKernelGGL(k_mlp_backward, dim3(grid), dim3(256), 0, st, m->dev(), feat, n, gy, m->part->as<float>());
-  hipLaunchKernelGGL(k_grad_reduce, dim3((kNParams + 255) / 256), dim3(256), 0, st,
-                     (const float *)m->part->as<float>(), grid * 4, m->grad->as<float>());
+  hipLaunchKernelGGL(k_grad_reduce, dim3((kNParams + 63) / 64), dim3(64 * kGradWaves), 0, st,
+                     (const float *)m->part->as<float>(), grid, m->grad->as<float>());
 }
 
 LSys *lsys_create(std::shared_ptr<Context> ctx, const HostCSR &A, const HostFactors &F, const float *feat) {
@@ -564,7 +676,6 @@ LSys *lsys_create(std::shared_ptr<Context> ctx, const HostCSR &A, const HostFact
   for (size_t k = 0; k < fb.size(); ++k) fb[k] = f2bf_host(feat[k]);
   L->feat = dev_alloc(2 * fb.size());
   F3R_HIP(hipMemcpyAsync(L->feat->p, fb.data(), 2 * fb.size(), hipMemcpyHostToDevice, c->stream));
-  for (DevPtr *v : {&L->y, &L->s, &L->u, &L->v, &L->pz, &L->q, &L->r, &L->g1, &L->g2, &L->gy}) *v = dev_alloc(4 * n);
   F3R_HIP(hipStreamSynchronize(c->stream));
   return L.release();
 }
@@ -579,40 +690,37 @@ double lsys_loss(LSys *L, MLP *m, int kind, bool grad) {
   Context *c = L->ctx.get();
   hipStream_t st = c->stream;
   const int64_t n = L->n;
-  const dim3 g((unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, (int64_t)c->num_cu * 16)), b(kBlock);
+  const dim3 b(kBlock);
   const uint16_t *feat = L->feat->as<uint16_t>();
-  float *y = L->y->as<float>(), *s = L->s->as<float>(), *u = L->u->as<float>(), *v = L->v->as<float>();
-  float *pz = L->pz->as<float>(), *q = L->q->as<float>(), *r = L->r->as<float>();
-  float *g1 = L->g1->as<float>(), *g2 = L->g2->as<float>(), *gy = L->gy->as<float>();
+  // y, s, gy and, per probe of a group, u, v and pz (v and pz are then reused
+  // for g1 and q or r): the context's workspace, shared by all its systems
+  const int group = std::min(L->nprobes, kProbeGroup);
+  float *ws = static_cast<float *>(c->workspace(4 * n * (3 + 3 * (int64_t)group)));
+  float *y = ws, *s = y + n, *gy = s + n, *u = gy + n, *v = u + group * n, *pz = v + group * n;
   float *norms = L->norms->as<float>();
-  mlp_forward_dev(m, feat, n, y, st);
-  hipLaunchKernelGGL(k_scale_from_y, g, b, 0, st, n, (const float *)y, s);
-  if (grad) F3R_HIP(hipMemsetAsync(gy, 0, 4 * n, st));
-  const int rgrid = (int)std::min<int64_t>((n + kBlock - 1) / kBlock, kMaxReduceGrid);
-  for (int k = 0; k < L->nprobes; ++k) {
-    const float *z = L->probes->as<float>() + (int64_t)k * n;
-    float *nk = norms + 4 * k;
-    spmv32(L->Wt, z, u, st);
-    hipLaunchKernelGGL(k_mul, g, b, 0, st, n, (const float *)s, (const float *)u, v);
-    spmv32(L->Z, v, pz, st);
-    spmv32(L->A, pz, q, st);
-    unsigned *cnt = c->red.counters->as<unsigned>() + 20 * kCounterSlot;
-    if (kind == 0) {
-      hipLaunchKernelGGL(k_resid_norms, dim3(rgrid), b, 0, st, n, z, (const float *)q, r,
-                         c->red.partial->as<float>(), cnt, nk);
-    } else {
-      hipLaunchKernelGGL(k_qdots, dim3(rgrid), b, 0, st, n, z, (const float *)q, c->red.partial->as<float>(), cnt,
-                         nk);
-      if (grad) hipLaunchKernelGGL(k_rscaled, g, b, 0, st, n, z, (const float *)q, (const float *)nk, r);
-    }
+  mlp_forward_dev(m, feat, n, y, s, st);
+  // block sums: 3 per probe and block
+  const int G = (int)std::min<int64_t>((n + kBlock - 1) / kBlock,
+                                       2 * Reducer::kPartialDoubles / (3 * kProbeGroup));
+  for (int k0 = 0; k0 < L->nprobes; k0 += group) {
+    const int np = std::min(group, L->nprobes - k0);
+    const float *z = L->probes->as<float>() + (int64_t)k0 * n;
+    float *nk = norms + 4 * k0, *q = v, *g1 = pz;
+    probe_sell(L->Wt, z, np, EpiProbeScale{u, v, s}, G, st);
+    probe_sell(L->Z, v, np, EpiProbeStore{pz}, G, st);
+    probe_sell(L->A, pz, np, EpiProbeResid{q, z, c->red.partial->as<float>(), kind}, G, st);
+    hipLaunchKernelGGL(k_probe_norms, dim3(np), dim3(1024), 0, st, (const float *)c->red.partial->as<float>(), G, nk);
     if (grad) {
-      spmv32(L->At, r, g1, st);
-      spmv32(L->Zt, g1, g2, st);
-      hipLaunchKernelGGL(k_gy, g, b, 0, st, n, (const float *)g2, (const float *)u, (const float *)s,
-                         (const float *)y, (const float *)nk, kind, 1.f / (float)L->nprobes, gy);
+      if (kind == 1)
+        hipLaunchKernelGGL(k_rscaled, dim3(std::min(G, 4 * c->num_cu), np), b, 0, st, n, z, q, (const float *)nk);
+      probe_sell(L->At, q, np, EpiProbeStore{g1}, G, st);
+      auto kern = L->Zt.sh->K == 4 ? k_probe_gy<4> : k_probe_gy<1>;
+      hipLaunchKernelGGL(kern, dim3(G), b, 0, st, sell_args(*L->Zt.sh, false), L->Zt.val->as<float>(),
+                         (const float *)g1, (const float *)u, (const float *)s, (const float *)y, (const float *)nk, np,
+                         kind, 1.f / (float)L->nprobes, k0 == 0 ? 1 : 0, gy);
     }
   }
-  if (grad && L->nprobes > 0) mlp_backward_dev(m, feat, n, gy, st);
+  if (grad) mlp_backward_dev(m, feat, n, gy, st);
   F3R_HIP(hipGetLastError());
   std::vector<float> h(4 * (size_t)L->nprobes);
   F3R_HIP(hipMemcpyAsync(h.data(), norms, 4 * h.size(), hipMemcpyDeviceToHost, st));
@@ -623,7 +731,7 @@ double lsys_loss(LSys *L, MLP *m, int kind, bool grad) {
     total += kind == 0 ? (double)e[0] / (double)e[1]
                        : 1.0 - (double)e[0] * (double)e[0] / ((double)e[2] * (double)e[1]);
   }
-  return L->nprobes > 0 ? total / L->nprobes : 0.0;
+  return total / L->nprobes;
 }
 
 }  // namespace f3r
@@ -722,7 +830,7 @@ int f3r_mlp_forward(f3r_mlp m, int64_t n, const float *feat, float *y) {
   Context *c = m->m->ctx.get();
   DevPtr f = upload_features(c, n, feat);
   DevPtr dy = dev_alloc(4 * n);
-  mlp_forward_dev(m->m.get(), f->as<uint16_t>(), n, dy->as<float>(), c->stream);
+  mlp_forward_dev(m->m.get(), f->as<uint16_t>(), n, dy->as<float>(), nullptr, c->stream);
   F3R_HIP(hipGetLastError());
   F3R_HIP(hipMemcpyAsync(y, dy->p, 4 * n, hipMemcpyDeviceToHost, c->stream));
   sync(c);
@@ -851,11 +959,10 @@ int f3r_lsys_scales(f3r_lsys L, f3r_mlp m, int32_t normalize, float *s) {
   LSys *S = L->L.get();
   Context *c = S->ctx.get();
   const int64_t n = S->n;
-  const dim3 g((unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, (int64_t)c->num_cu * 16)), b(kBlock);
-  mlp_forward_dev(m->m.get(), S->feat->as<uint16_t>(), n, S->y->as<float>(), c->stream);
-  hipLaunchKernelGGL(k_scale_from_y, g, b, 0, c->stream, n, (const float *)S->y->as<float>(), S->s->as<float>());
+  float *y = static_cast<float *>(c->workspace(8 * n));
+  mlp_forward_dev(m->m.get(), S->feat->as<uint16_t>(), n, y, y + n, c->stream);
   F3R_HIP(hipGetLastError());
-  F3R_HIP(hipMemcpyAsync(s, S->s->p, 4 * n, hipMemcpyDeviceToHost, c->stream));
+  F3R_HIP(hipMemcpyAsync(s, y + n, 4 * n, hipMemcpyDeviceToHost, c->stream));
   sync(c);
   if (normalize) {  // divide by the geometric mean: the loss of kind 1 cannot see a global scale
     double lm = 0;
