@@ -164,100 +164,138 @@ __global__ __launch_bounds__(1024) void k_bj_trsv_u(const int32_t *__restrict__ 
   }
 }
 
-// The same two solves fused in one launch with the block's vector in LDS:
-// xs = in (the block's rows), the L levels in place, then the U levels in
-// place, then out = xs.  Each row's entries are stored level by level as
-// structure-of-arrays records (local column, value, in the order the solves
-// above visit them; the U record also carries 1/u_ii), so the next level's
-// records are loaded before the barrier that ends the current one and only
-// LDS reads remain on the path from level to level.  Same arithmetic as
-// k_trsv_l / k_trsv_u.
-template <class S> struct BjRec {
-  const int32_t *start, *lptr;  // per block: first level pointer; level -> slot range
-  const int32_t *row, *cnt, *col;  // per slot: local row, entries, columns (R x slots)
-  const S *val, *dinv;             // values (R x slots), 1/u_ii (U only)
-  int32_t slots;
-};
-template <class S, int R> struct BjSlot {
-  int32_t row, cnt;
-  int32_t col[R];
+// The same two solves fused in one launch, the block's vector xs and the
+// records of its rows in LDS: xs = in (the block's rows), the L levels in
+// place, then the U levels in place, then out = xs.  Same arithmetic and
+// order as k_trsv_l / k_trsv_u.
+//
+// What bounds it is the chain from level to level (about 100 levels a side for
+// a 7-point 64^3 matrix in 112 blocks), so the chain is kept inside one
+// wavefront: a level's rows are solved in batches of up to 64, one row per
+// lane, and LDS operations of one wave complete in order, so a level needs no
+// barrier.  The rows' records (local row and columns as 16-bit numbers, the
+// values in visiting order, 1/u_ii) form one stream per block in solving
+// order.  It passes through LDS in segments of SR records: two are resident,
+// the third is on its way in registers, so the memory latency overlaps two
+// segments of work however narrow the levels are.  Wide levels (NW = 4) use
+// four waves and a barrier per batch.  Records read level by level from
+// global memory, four levels ahead, took 87 us at 64^3 / 112 blocks: 0.43 us
+// a level, the memory latency over four.
+constexpr uint16_t kBjNone = 0xffff;  // column of an unused entry
+template <class S, int R> struct alignas(8) BjRecord {
+  uint16_t row, col[R];
   S val[R];
-  S dinv;
+  S dinv;  // U only
 };
-// Loads the record of this thread's slot in level q (row -1: no slot, or q
-// past the block's last level).  Every call issues the same loads (indices
-// clamped into range; entries past the row's count are zero padding), so the
-// compiler can count them and wait for exactly the oldest ones.
-typedef const __attribute__((address_space(4))) int32_t *bj_const_i32;  // uniform read-only: scalar loads
-
-template <class S, int R>
-__device__ __forceinline__ void bj_load(const BjRec<S> &r, int32_t q, int32_t q1, bool upper, BjSlot<S, R> &sl) {
-  const bool lvl = q + 1 < q1;
-  const int32_t qq = __builtin_amdgcn_readfirstlane(lvl ? q : q1 - 2);
-  // the level pointers by scalar loads: the vector-load counter then holds
-  // only the records, and waiting for the oldest does not wait for the rest
-  const bj_const_i32 lp = (bj_const_i32)r.lptr;
-  const int32_t t0 = lp[qq] + (int32_t)threadIdx.x, te = lp[qq + 1];
-  const bool on = lvl && t0 < te;
-  const int32_t t = on ? t0 : te - 1;
-  sl.row = on ? r.row[t] : -1;
-  sl.cnt = r.cnt[t];
-#pragma unroll
-  for (int k = 0; k < R; ++k) {
-    sl.col[k] = r.col[(int64_t)k * r.slots + t];
-    sl.val[k] = r.val[(int64_t)k * r.slots + t];
-  }
-  sl.dinv = upper ? r.dinv[t] : S(0);
+// records per segment: a power of two of batches, about 16 KB
+template <class S, int R, int NW> constexpr int bj_segment() {
+  int m = 64 * NW;
+  while (2 * m * (int)sizeof(BjRecord<S, R>) <= 16384) m *= 2;
+  return m;
 }
+struct BjSide {
+  const void *rec;        // segments of all blocks
+  const int32_t *seg;     // block b: segments seg[b] .. seg[b + 1] - 1
+  const int32_t *bat;     // block b: batch sizes cnt[bat[b]] .. cnt[bat[b + 1] - 1]
+  const uint16_t *cnt;    // (64 entries of zero padding at the end)
+};
 // Barrier for LDS traffic only: this wave's LDS operations complete, then
 // s_barrier.  __syncthreads() would also wait for every outstanding global
-// load (its release fence), i.e. for the prefetched records below.  The
-// memory clobber keeps the compiler from moving LDS accesses across it.
+// load (its release fence), i.e. for the segment on its way.  The memory
+// clobber keeps the compiler from moving LDS accesses across it.
 __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The records of the next D levels stay in flight: level q + D is requested
-// as level q finishes, so its latency overlaps D levels of work.  The loop
-// is unrolled by D so the ring is indexed statically (registers).
-template <class S, int R>
-__device__ __forceinline__ void bj_levels(const BjRec<S> &r, bool upper, S *xs) {
+template <class S, int R, int NW>
+__device__ __forceinline__ void bj_side(const BjSide &sd, bool upper, S *xs, unsigned char *ring) {
   using A = typename Acc<S>::type;
-  constexpr int D = R <= 4 ? 4 : R <= 8 ? 3 : 2;
-  const bj_const_i32 st = (bj_const_i32)r.start;
-  const int32_t q0 = st[blockIdx.x], q1 = st[blockIdx.x + 1];
-  BjSlot<S, R> ring[D];
+  using Rec = BjRecord<S, R>;
+  using Unit = typename std::conditional<sizeof(Rec) % 16 == 0, u32x4, u32x2>::type;
+  constexpr int SR = bj_segment<S, R, NW>(), T = 64 * NW;
+  constexpr int kUnits = SR * (int)sizeof(Rec) / (int)sizeof(Unit) / T;  // of one thread
+  static_assert(SR * sizeof(Rec) == (size_t)kUnits * T * sizeof(Unit), "a segment is whole units per thread");
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int32_t s0 = sd.seg[blockIdx.x], nseg = sd.seg[blockIdx.x + 1] - s0;
+  const int32_t b0 = sd.bat[blockIdx.x], nb = sd.bat[blockIdx.x + 1] - b0;
+  const Unit *src = reinterpret_cast<const Unit *>(static_cast<const Rec *>(sd.rec) + (int64_t)s0 * SR);
+  Unit *const lring = reinterpret_cast<Unit *>(ring);
+  const Rec *const recs = reinterpret_cast<const Rec *>(ring);
+  Unit stage[kUnits];
+  auto issue = [&](int k) {
+    if (k < nseg) {
 #pragma unroll
-  for (int d = 0; d < D; ++d) bj_load<S, R>(r, q0 + d, q1, upper, ring[d]);
-  // straight-line steps; the at most D - 1 steps past the last level have
-  // no slots and only meet the barrier (the same count for every thread)
-  for (int32_t q = q0; q + 1 < q1; q += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      BjSlot<S, R> &cur = ring[d];
-      const int32_t row = cur.row;
-      A s = to_acc(xs[row >= 0 ? row : 0]);
-#pragma unroll
-      for (int k = 0; k < R; ++k)
-        if (k < cur.cnt) s = fma_<A>(-to_acc(cur.val[k]), to_acc(xs[cur.col[k]]), s);
-      const S res = upper ? cvt<S>(s * to_acc(cur.dinv)) : cvt<S>(s);
-      bj_load<S, R>(r, q + d + D, q1, upper, cur);
-      if (row >= 0) xs[row] = res;
-      lds_barrier();
+      for (int p = 0; p < kUnits; ++p) stage[p] = src[((int64_t)k * kUnits + p) * T + tid];
     }
+  };
+  auto commit = [&](int k) {
+    if (k < nseg) {
+#pragma unroll
+      for (int p = 0; p < kUnits; ++p) lring[((k & 1) * kUnits + p) * T + tid] = stage[p];
+    }
+  };
+  issue(0);
+  commit(0);
+  issue(1);
+  commit(1);
+  issue(2);
+  if constexpr (NW > 1) lds_barrier();
+  int32_t cnts = sd.cnt[b0 + lane], cntn = sd.cnt[b0 + kWave + lane];  // the next 64 batch sizes ahead
+  int k = 0, t0 = 0;
+  Rec rec = recs[tid];
+  for (int b = 0; b < nb; ++b) {
+    const int c = __builtin_amdgcn_readlane(cnts, b & (kWave - 1));
+    const Rec cur = rec;
+    // xs of this batch: every read is issued before the first is used
+    const int32_t row = tid < c ? cur.row : 0;
+    A s = to_acc(xs[row]);
+    S xv[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) xv[q] = xs[tid < c && cur.col[q] != kBjNone ? cur.col[q] : 0];
+    // the next batch's records, past the segment boundary if it is crossed
+    t0 += c;
+    if (t0 >= (k + 1) * SR) {
+      if constexpr (NW > 1) lds_barrier();  // segment k is read by every wave
+      commit(k + 2);
+      issue(k + 3);
+      ++k;
+      if constexpr (NW > 1) lds_barrier();
+    }
+    rec = recs[(t0 + tid) & (2 * SR - 1)];
+    if (((b + 1) & (kWave - 1)) == 0) {
+      cnts = cntn;
+      cntn = b + 1 + kWave < nb ? sd.cnt[b0 + b + 1 + kWave + lane] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+      if (cur.col[q] != kBjNone) s = fma_<A>(-to_acc(cur.val[q]), to_acc(xv[q]), s);
+    if (tid < c) xs[row] = upper ? cvt<S>(s * to_acc(cur.dinv)) : cvt<S>(s);
+    if constexpr (NW > 1) lds_barrier();
   }
 }
 
-template <class S, int R>
-__global__ __launch_bounds__(1024) void k_bj_lds(const int32_t *__restrict__ b0, const int32_t *__restrict__ bn,
-                                                 BjRec<S> L, BjRec<S> U, const S *__restrict__ in,
-                                                 S *__restrict__ out) {
-  extern __shared__ unsigned char bj_smem[];
-  S *xs = reinterpret_cast<S *>(bj_smem);
-  const int32_t r0 = b0[blockIdx.x], nr = bn[blockIdx.x];
-  for (int32_t i = threadIdx.x; i < nr; i += blockDim.x) xs[i] = in[r0 + i];
+template <class S, int R, int NW>
+__global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, BjSide L, BjSide U, const S *__restrict__ in,
+                                                   S *__restrict__ out) {
+  extern __shared__ __align__(16) unsigned char bj_smem[];
+  constexpr int kRing = 2 * bj_segment<S, R, NW>() * (int)sizeof(BjRecord<S, R>);
+  S *xs = reinterpret_cast<S *>(bj_smem + kRing);
+  const int32_t r0 = blockIdx.x * bsz, nr = n - r0 < bsz ? n - r0 : bsz;
+  // all waves move the vector, 8 rows in flight each
+  for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kBlock) {
+    S v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = i0 + q * kBlock < nr ? in[r0 + i0 + q * kBlock] : S(0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (i0 + q * kBlock < nr) xs[i0 + q * kBlock] = v[q];
+  }
   __syncthreads();
-  bj_levels<S, R>(L, false, xs);
-  bj_levels<S, R>(U, true, xs);
-  for (int32_t i = threadIdx.x; i < nr; i += blockDim.x) out[r0 + i] = xs[i];
+  if (threadIdx.x < 64 * NW) {
+    bj_side<S, R, NW>(L, false, xs, bj_smem);
+    if constexpr (NW > 1) lds_barrier();
+    bj_side<S, R, NW>(U, true, xs, bj_smem);
+  }
+  __syncthreads();
+  for (int32_t i = threadIdx.x; i < nr; i += kBlock) out[r0 + i] = xs[i];
 }
 
 static int grid_for(int64_t n, int cu) {
@@ -757,36 +795,83 @@ static void group_by_block(const std::vector<int32_t> &rows, const std::vector<i
   bstart[nb] = (int32_t)blptr.size();
 }
 
-// SoA records of a triangular factor in the grouped order `brows` (see
-// k_bj_lds): entries in the visiting order of the solve, columns local to
-// the row's block.  False when a row has more than `rmax` entries.
-static bool bj_records(const HostCSR &M, bool upper, const std::vector<int32_t> &brows, int32_t bsz, int rmax,
-                       std::vector<int32_t> &row, std::vector<int32_t> &cnt, std::vector<int32_t> &col,
-                       std::vector<double> &val) {
-  const int64_t ns = (int64_t)brows.size();
-  row.assign(ns, 0);
-  cnt.assign(ns, 0);
-  col.assign(ns * rmax, 0);
-  val.assign(ns * rmax, 0.0);
-  for (int64_t t = 0; t < ns; ++t) {
-    const int32_t i = brows[t], base = i / bsz * bsz;
-    row[t] = i - base;
-    int c = 0;
-    auto put = [&](int32_t k) {
-      if (c < rmax) {
-        col[c * ns + t] = M.idx[k] - base;
-        val[c * ns + t] = M.val[k];
-      }
-      ++c;
-    };
-    if (upper)
-      for (int32_t k = M.rptr[i + 1] - 1; k > M.rptr[i]; --k) put(k);
-    else
-      for (int32_t k = M.rptr[i]; k < M.rptr[i + 1] - 1; ++k) put(k);
-    if (c > rmax) return false;
-    cnt[t] = c;
+// Record stream of a triangular factor for k_bj_lds: the rows of each block
+// in the grouped order (`brows`, block by block and level by level), padded to
+// whole segments, and the sizes of the batches (at most 64 NW rows of one
+// level) they are solved in.
+struct BjStream {
+  std::vector<unsigned char> rec;
+  std::vector<int32_t> seg, bat;
+  std::vector<uint16_t> cnt;
+};
+template <class S, int R, int NW>
+static void bj_stream(const HostCSR &M, bool upper, const std::vector<int32_t> &brows,
+                      const std::vector<int32_t> &blptr, const std::vector<int32_t> &bstart, int32_t bsz,
+                      BjStream &out) {
+  using Rec = BjRecord<S, R>;
+  constexpr int SR = bj_segment<S, R, NW>();
+  const int32_t nb = (int32_t)bstart.size() - 1;
+  auto bits = [](double v) {
+    S s;
+    if constexpr (std::is_same<S, half_t>::value) {
+      const uint16_t h = d2h_bits(v);
+      std::memcpy(&s, &h, 2);
+    } else {
+      s = (S)v;
+    }
+    return s;
+  };
+  out.seg.assign(1, 0);
+  out.bat.assign(1, 0);
+  for (int32_t b = 0; b < nb; ++b) {
+    const int32_t rows = blptr[bstart[b + 1] - 1] - blptr[bstart[b]];
+    out.seg.push_back(out.seg.back() + (rows + SR - 1) / SR);
   }
-  return true;
+  Rec none{};
+  for (int q = 0; q < R; ++q) none.col[q] = kBjNone;
+  std::vector<Rec> rec((size_t)out.seg.back() * SR, none);
+  for (int32_t b = 0; b < nb; ++b) {
+    Rec *r = rec.data() + (size_t)out.seg[b] * SR;
+    const int32_t base = b * bsz;
+    for (int32_t t = blptr[bstart[b]]; t < blptr[bstart[b + 1] - 1]; ++t, ++r) {
+      const int32_t i = brows[t];
+      r->row = (uint16_t)(i - base);
+      int c = 0;
+      auto put = [&](int32_t k) {
+        r->col[c] = (uint16_t)(M.idx[k] - base);
+        r->val[c++] = bits(M.val[k]);
+      };
+      if (upper) {
+        for (int32_t k = M.rptr[i + 1] - 1; k > M.rptr[i]; --k) put(k);
+        r->dinv = bits(1. / M.val[M.rptr[i]]);
+      } else {
+        for (int32_t k = M.rptr[i]; k < M.rptr[i + 1] - 1; ++k) put(k);
+      }
+    }
+    for (int32_t q = bstart[b]; q + 1 < bstart[b + 1]; ++q)
+      for (int32_t w = blptr[q + 1] - blptr[q]; w > 0; w -= 64 * NW) out.cnt.push_back((uint16_t)std::min(w, 64 * NW));
+    out.bat.push_back((int32_t)out.cnt.size());
+  }
+  // the kernel reads batch sizes 64 at a time, two groups ahead
+  out.cnt.insert(out.cnt.end(), 2 * kWave, 0);
+  out.rec.resize(rec.size() * sizeof(Rec));
+  std::memcpy(out.rec.data(), rec.data(), out.rec.size());
+}
+
+// f(S tag, R, NW) for the preconditioner's record shape
+template <class F> static void bj_dispatch(int dtype, int R, int NW, F f) {
+  auto by_nw = [&](auto s, auto r) {
+    if (NW == 1) f(s, r, std::integral_constant<int, 1>());
+    else f(s, r, std::integral_constant<int, 4>());
+  };
+  auto by_r = [&](auto s) {
+    if (R == 3) by_nw(s, std::integral_constant<int, 3>());
+    else if (R == 7) by_nw(s, std::integral_constant<int, 7>());
+    else by_nw(s, std::integral_constant<int, 16>());
+  };
+  if (dtype == F3R_F16) by_r(half_t());
+  else if (dtype == F3R_F32) by_r(float());
+  else by_r(double());
 }
 
 static std::vector<int32_t> levels_upper(const HostCSR &U, std::vector<int32_t> &lptr) {
@@ -911,49 +996,47 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
       P->ub_ptr = upload_i32(c, bl);
       P->ub_start = upload_i32(c, bs);
       P->bj_groups = (int32_t)bs.size() - 1;
-      // the fused LDS kernel: the block's vector in LDS, at most 1024 rows
-      // per level of a block and 16 entries per row
-      int32_t maxrows = 0, maxw = 0, maxe = 0;
+      // the fused LDS kernel: the block's vector in LDS (local rows and
+      // columns then fit 16 bits) and at most 16 entries per row
+      int32_t maxrows = 0, maxe = 0;
       for (int32_t b = 0; b < P->bj_groups; ++b) maxrows = std::max(maxrows, std::min(n, (b + 1) * bsz) - b * bsz);
       std::vector<int32_t> lbr, lbl, lbs, ubr, ubl, ubs;
       group_by_block(lrows, P->l_lptr, n, bsz, lbr, lbl, lbs);
       group_by_block(urows, P->u_lptr, n, bsz, ubr, ubl, ubs);
-      for (const std::vector<int32_t> *v : {&lbl, &ubl})
-        for (size_t q = 0; q + 1 < v->size(); ++q) maxw = std::max(maxw, (*v)[q + 1] - (*v)[q]);
       for (int32_t i = 0; i < n; ++i) {
         maxe = std::max(maxe, L.rptr[i + 1] - L.rptr[i] - 1);
         maxe = std::max(maxe, U.rptr[i + 1] - U.rptr[i] - 1);
       }
       const size_t lds = (size_t)maxrows * dtype_size(P->dtype);
-      if (maxw <= 1024 && maxe <= 16 && lds <= kBjLdsBytes) {
-        const int R = maxe <= 4 ? 4 : maxe <= 8 ? 8 : 16;
-        std::vector<int32_t> row, cnt, col;
-        std::vector<double> val;
-        bj_records(L, false, lbr, bsz, R, row, cnt, col, val);
-        P->lr_row = upload_i32(c, row);
-        P->lr_cnt = upload_i32(c, cnt);
-        P->lr_col = upload_i32(c, col);
-        P->lr_val = upload_values(c, val, P->dtype);
-        bj_records(U, true, ubr, bsz, R, row, cnt, col, val);
-        P->ur_row = upload_i32(c, row);
-        P->ur_cnt = upload_i32(c, cnt);
-        P->ur_col = upload_i32(c, col);
-        P->ur_val = upload_values(c, val, P->dtype);
-        std::vector<double> dv(n);
-        for (int32_t t = 0; t < n; ++t) dv[t] = 1. / U.val[U.rptr[ubr[t]]];
-        P->ur_dinv = upload_values(c, dv, P->dtype);
-        std::vector<int32_t> b0(P->bj_groups), bn(P->bj_groups);
-        for (int32_t b = 0; b < P->bj_groups; ++b) {
-          b0[b] = b * bsz;
-          bn[b] = std::min(n, (b + 1) * bsz) - b * bsz;
-        }
-        P->bj_b0 = upload_i32(c, b0);
-        P->bj_bn = upload_i32(c, bn);
-        P->bj_R = R;
-        P->bj_lds = lds;
-        // one thread per row of the widest level: idle waves would still
-        // load records and meet every barrier
-        P->bj_threads = std::max(64, (maxw + 63) / 64 * 64);
+      if (maxe <= 16 && lds <= kBjLdsBytes) {
+        P->bj_R = maxe <= 3 ? 3 : maxe <= 7 ? 7 : 16;
+        // one wave up to 128 rows per level on average (two batches); wider
+        // levels on four waves with a barrier per batch
+        const double levels = (double)(lbl.size() + ubl.size()) - 2.0 * P->bj_groups;
+        P->bj_waves = 2.0 * n <= 128.0 * levels ? 1 : 4;
+        bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
+          using S = decltype(s);
+          constexpr int R = decltype(r)::value, NW = decltype(w)::value;
+          for (int side = 0; side < 2; ++side) {
+            BjStream bt;
+            if (side == 0) bj_stream<S, R, NW>(L, false, lbr, lbl, lbs, bsz, bt);
+            else bj_stream<S, R, NW>(U, true, ubr, ubl, ubs, bsz, bt);
+            Prec::BjData &d = P->bj[side];
+            auto up = [&](DevPtr &p, const void *h, size_t bytes) {
+              p = dev_alloc(std::max<size_t>(bytes, 16));
+              if (bytes) F3R_HIP(hipMemcpyAsync(p->p, h, bytes, hipMemcpyHostToDevice, c->stream));
+            };
+            up(d.rec, bt.rec.data(), bt.rec.size());
+            up(d.cnt, bt.cnt.data(), 2 * bt.cnt.size());
+            up(d.seg, bt.seg.data(), 4 * bt.seg.size());
+            up(d.bat, bt.bat.data(), 4 * bt.bat.size());
+            F3R_HIP(hipStreamSynchronize(c->stream));
+          }
+          P->bj_lds = lds + 2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>);
+          // up to 154 KB of the CU's 160 KB
+          F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, R, NW>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->bj_lds));
+        });
       }
     }
     P->l_rptr = upload_i32(c, L.rptr);
@@ -971,18 +1054,15 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
 template <class S> static void ilu_apply_t(Prec *P, const S *in, S *out, hipStream_t st) {
   S *tmp = P->tmp->as<S>();
   if (P->bj_R) {
-    const int32_t ns = P->n;
-    BjRec<S> L{P->lb_start->as<int32_t>(), P->lb_ptr->as<int32_t>(), P->lr_row->as<int32_t>(),
-               P->lr_cnt->as<int32_t>(), P->lr_col->as<int32_t>(), P->lr_val->as<S>(), nullptr, ns};
-    BjRec<S> U{P->ub_start->as<int32_t>(), P->ub_ptr->as<int32_t>(), P->ur_row->as<int32_t>(),
-               P->ur_cnt->as<int32_t>(), P->ur_col->as<int32_t>(), P->ur_val->as<S>(), P->ur_dinv->as<S>(), ns};
-    const int32_t *b0 = P->bj_b0->as<int32_t>(), *bn = P->bj_bn->as<int32_t>();
-    const unsigned lds = (unsigned)P->bj_lds;
-    switch (P->bj_R) {
-      case 4: hipLaunchKernelGGL((k_bj_lds<S, 4>), dim3(P->bj_groups), dim3(P->bj_threads), lds, st, b0, bn, L, U, in, out); break;
-      case 8: hipLaunchKernelGGL((k_bj_lds<S, 8>), dim3(P->bj_groups), dim3(P->bj_threads), lds, st, b0, bn, L, U, in, out); break;
-      default: hipLaunchKernelGGL((k_bj_lds<S, 16>), dim3(P->bj_groups), dim3(P->bj_threads), lds, st, b0, bn, L, U, in, out); break;
-    }
+    auto side = [&](const Prec::BjData &d) {
+      return BjSide{d.rec->p, d.seg->as<int32_t>(), d.bat->as<int32_t>(), d.cnt->as<uint16_t>()};
+    };
+    const int32_t blocks = P->bj_blocks, bsz = (P->n + blocks - 1) / blocks;
+    bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
+      if constexpr (std::is_same<decltype(s), S>::value)
+        hipLaunchKernelGGL((k_bj_lds<S, decltype(r)::value, decltype(w)::value>), dim3(P->bj_groups), dim3(kBlock),
+                           P->bj_lds, st, P->n, bsz, side(P->bj[0]), side(P->bj[1]), in, out);
+    });
     return;
   }
   if (P->bj_blocks) {

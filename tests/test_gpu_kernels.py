@@ -243,6 +243,58 @@ def test_bjilu0_block_per_workgroup_matches_oracle(ctx, blocks, dtype):
     assert np.array_equal(got, out)
 
 
+def _coupled(n, dists, seed):
+    """diagonally dominant rows coupled to the rows at the given distances"""
+    import scipy.sparse as sp
+    import f3r_amd as F
+    rng = np.random.default_rng(seed)
+    dists = sorted({s * d for d in dists for s in (-1, 1)} | {0})
+    M = sp.diags([np.full(n, 2.0) if d == 0 else rng.uniform(-1, 1, n - abs(d)) / len(dists) for d in dists], dists,
+                 format="csr")
+    M.sort_indices()
+    return F.CSR(n, M.indptr, M.indices, M.data)
+
+
+@pytest.mark.parametrize("n,blocks,dists", [
+    (40007, 32, [1]),                          # one row per level: 1251 levels, many segments
+    (40007, 50, [1, 60]),                      # a 2-D wavefront
+    (33 * 97, 33, [1, 2, 5, 30, 31]),          # 7 entries a row at most
+    (20000, 40, list(range(1, 14))),           # 13 entries: the widest records
+    (20011, 40, list(range(1, 17))),           # 16
+    (40007, 32, [600]),                        # 600 rows per level: four waves
+    (40007, 32, [300, 301, 302, 303, 304]),
+    (40009, 37, [290 + k for k in range(16)]),
+    (4096, 64, []),                            # diagonal blocks: one level
+    (127, 64, [1])])                           # 2 rows a block, 1 in the last
+@pytest.mark.parametrize("dtype", ["f64", "f32", "f16"])
+def test_bjilu0_record_streams(ctx, n, blocks, dists, dtype):
+    """the record streams of the fused block-Jacobi solve: entry classes, level
+    widths (one and four waves), segment ends and ragged last blocks"""
+    import f3r_amd as F
+    A = _coupled(n, dists, 11)
+    print(f"bjilu0 streams n={n} blocks={blocks} entries={len(dists)} {dtype}", flush=True)
+    P = F.ILU0(A, blocks=blocks, acc=1.0, dtype=dtype, ctx=ctx)
+    x = np.random.default_rng(8).uniform(-1, 1, n)
+    xs = x.astype({"f64": np.float64, "f32": np.float32, "f16": np.float16}[dtype])
+    yv = F.vector(ctx, dtype, n)
+    P.operate(F.vector.from_numpy(ctx, xs), yv)
+    h = O.lib().orc_ilu0(A.n, O.P(A.rptr), O.P(A.idx), O.P(A.val), blocks, 1.0)
+    if dtype == "f16":
+        out, tmp = np.zeros(n, np.uint16), np.zeros(n, np.uint16)
+        O.lib().orc_bj_solve16(h, O.P(xs.view(np.uint16)), O.P(out), O.P(tmp), 0)
+        assert np.array_equal(yv.download().view(np.uint16), out)
+    else:
+        out, tmp = np.zeros(n), np.zeros(n)
+        xd = xs.astype(np.float64)
+        O.lib().orc_bj_solve(h, O.P(xd), O.P(out), O.P(tmp))
+        got = yv.download()
+        if dtype == "f64":
+            assert np.array_equal(got, out)
+        else:  # contraction by rows (dominance 2 : 1), 2 x 17 roundings of 2^-24 a row and level
+            assert np.abs(got - out).max() <= 1e-5 * np.abs(out).max()
+    O.lib().orc_factor_free(h)
+
+
 def _device_fits(A, C, sigma, offsets):
     # the device build's on-chip sorts: sigma windows of at most 4096 rows and,
     # in the offset format, chunks of at most 4096 entries (else the host builds)
