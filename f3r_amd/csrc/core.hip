@@ -272,21 +272,39 @@ __device__ __forceinline__ void bj_side(const BjSide &sd, bool upper, S *xs, uns
   }
 }
 
-template <class S, int R, int NW>
-__global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, BjSide L, BjSide U, const S *__restrict__ in,
-                                                   S *__restrict__ out) {
+template <class S, class F, int R, int NW>
+__global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, BjSide L, BjSide U, MIo<S, F> io) {
   extern __shared__ __align__(16) unsigned char bj_smem[];
   constexpr int kRing = 2 * bj_segment<S, R, NW>() * (int)sizeof(BjRecord<S, R>);
   S *xs = reinterpret_cast<S *>(bj_smem + kRing);
   const int32_t r0 = blockIdx.x * bsz, nr = n - r0 < bsz ? n - r0 : bsz;
   // all waves move the vector, 8 rows in flight each
-  for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kBlock) {
-    S v[8];
+  if (io.raw) {
+    const MEntry<S, F> en(io);
+    for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kBlock) {
+      F v[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = i0 + q * kBlock < nr ? in[r0 + i0 + q * kBlock] : S(0);
+      for (int q = 0; q < 8; ++q) v[q] = i0 + q * kBlock < nr ? io.raw[r0 + i0 + q * kBlock] : F(0);
 #pragma unroll
-    for (int q = 0; q < 8; ++q)
-      if (i0 + q * kBlock < nr) xs[i0 + q * kBlock] = v[q];
+      for (int q = 0; q < 8; ++q)
+        if (i0 + q * kBlock < nr) {
+          const int32_t i = i0 + q * kBlock;
+          const F vn = en.norm(v[q]);
+          const S h = en.store(vn);
+          if (io.vout) io.vout[r0 + i] = vn;
+          if (io.hin) io.hin[r0 + i] = h;
+          xs[i] = h;
+        }
+    }
+  } else {
+    for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kBlock) {
+      S v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = i0 + q * kBlock < nr ? io.in[r0 + i0 + q * kBlock] : S(0);
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (i0 + q * kBlock < nr) xs[i0 + q * kBlock] = v[q];
+    }
   }
   __syncthreads();
   if (threadIdx.x < 64 * NW) {
@@ -295,7 +313,99 @@ __global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, BjSid
     bj_side<S, R, NW>(U, true, xs, bj_smem);
   }
   __syncthreads();
-  for (int32_t i = threadIdx.x; i < nr; i += kBlock) out[r0 + i] = xs[i];
+  const MExit<S, F> mo(io);
+  for (int32_t i = threadIdx.x; i < nr; i += kBlock) mo.put(r0 + i, xs[i], mo.pre(r0 + i));
+}
+
+// ------------------------------------------ M with its entry and update ---
+// Diagonal SDAINV: entry, z (w h) and the weight in one pass.  Streams its
+// vectors (4 rows per lane with VEC: every array 4-element aligned).
+template <class S, class F, bool VEC>
+__global__ __launch_bounds__(kBlock) void k_m_diag(int64_t n, DiagWZ<S> d, MIo<S, F> io) {
+  const MEntry<S, F> en(io);
+  const MExit<S, F> mo(io);
+  const int64_t gid = blockIdx.x * (int64_t)kBlock + threadIdx.x, gstride = (int64_t)gridDim.x * kBlock;
+  int64_t i0 = 0;
+  if constexpr (VEC) {
+    const int64_t n4 = n / 4;
+    for (int64_t q = gid; q < n4; q += gstride) {
+      V4<F> v = ld4(io.raw + 4 * q);
+      V4<S> h, o, w4, z4;
+      if constexpr (std::is_same<S, half_t>::value) {
+        const V4<uint32_t> wz = ld4(d.wz + 4 * q);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const typename DiagWZ<S>::V e = DiagWZ<S>::unpack(wz.v[c]);
+          w4.v[c] = e.w;
+          z4.v[c] = e.z;
+        }
+      } else {
+        w4 = ld4(d.w + 4 * q);
+        z4 = ld4(d.z + 4 * q);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        v.v[c] = en.norm(v.v[c]);
+        h.v[c] = en.store(v.v[c]);
+        o.v[c] = mo.value(diag_apply<S>({w4.v[c], z4.v[c]}, h.v[c]), S(0));
+      }
+      if (io.vout) st4(io.vout + 4 * q, v);
+      if (io.hin) st4(io.hin + 4 * q, h);
+      st4(io.out + 4 * q, o);
+    }
+    i0 = 4 * n4;
+  }
+  for (int64_t i = i0 + gid; i < n; i += gstride) {
+    const F v = en.norm(io.raw[i]);
+    const S h = en.store(v);
+    if (io.vout) io.vout[i] = v;
+    if (io.hin) io.hin[i] = h;
+    io.out[i] = mo.value(diag_apply<S>(d.at(i), h), S(0));
+  }
+}
+
+// General SDAINV, first half: t = W^T h with h entered from the basis vector
+// as it is gathered (the few entries of a row convert a neighbour's element
+// again; storing h first would be another launch), and the row's own element
+// normalised and stored.
+template <class S, class F, int K>
+__global__ __launch_bounds__(kBlock) void k_m_entry_w(SellArgs a, const S *__restrict__ val, MIo<S, F> io,
+                                                      S *__restrict__ t) {
+  using ACC = typename Acc<S>::type;
+  const MEntry<S, F> en(io);
+  for (int r = xcd_block() * kBlock + threadIdx.x; r < a.n; r += gridDim.x * kBlock) {
+    const F v = en.norm(io.raw[r]);
+    t[r] = cvt<S>(sell_row<S, F, ACC, K>(a, val, io.raw, r, en));
+    if (io.vout) io.vout[r] = v;
+    if (io.hin) io.hin[r] = en.store(v);
+  }
+}
+// second half: Z t with the weight and the update
+template <class S, class F> struct EpiMExit {
+  using State = NoState;
+  struct Pre {
+    S add;
+  };
+  MIo<S, F> io;
+  __device__ Pre pre(int r) const { return {io.add ? io.add[r] : S(0)}; }
+  __device__ void row(int r, typename Acc<S>::type acc, const Pre &p, State &) const {
+    MExit<S, F>(io).put(r, cvt<S>(acc), p.add);
+  }
+  __device__ void finish(State &) const {}
+};
+// element-wise entry and output for kinds of M without fused kernels
+template <class S, class F> __global__ void k_m_entry(int64_t n, MIo<S, F> io, S *__restrict__ h) {
+  const MEntry<S, F> en(io);
+  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+    const F v = en.norm(io.raw[i]);
+    if (io.vout) io.vout[i] = v;
+    if (h) h[i] = en.store(v);
+  }
+}
+template <class S, class F> __global__ void k_m_out(int64_t n, const S *__restrict__ x, MIo<S, F> io) {
+  const MExit<S, F> mo(io);
+  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
+    mo.put(i, x[i], mo.pre(i));
 }
 
 static int grid_for(int64_t n, int cu) {
@@ -1034,8 +1144,11 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
           }
           P->bj_lds = lds + 2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>);
           // up to 154 KB of the CU's 160 KB
-          F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, R, NW>),
+          F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, S, R, NW>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->bj_lds));
+          if constexpr (std::is_same<S, half_t>::value)
+            F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, float, R, NW>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->bj_lds));
         });
       }
     }
@@ -1051,18 +1164,26 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
   }
 }
 
+// the fused block-Jacobi solve
+template <class S, class F> static void bj_apply(Prec *P, const MIo<S, F> &io, hipStream_t st) {
+  auto side = [&](const Prec::BjData &d) {
+    return BjSide{d.rec->p, d.seg->as<int32_t>(), d.bat->as<int32_t>(), d.cnt->as<uint16_t>()};
+  };
+  const int32_t blocks = P->bj_blocks, bsz = (P->n + blocks - 1) / blocks;
+  bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
+    if constexpr (std::is_same<decltype(s), S>::value)
+      hipLaunchKernelGGL((k_bj_lds<S, F, decltype(r)::value, decltype(w)::value>), dim3(P->bj_groups), dim3(kBlock),
+                         P->bj_lds, st, P->n, bsz, side(P->bj[0]), side(P->bj[1]), io);
+  });
+}
+
 template <class S> static void ilu_apply_t(Prec *P, const S *in, S *out, hipStream_t st) {
   S *tmp = P->tmp->as<S>();
   if (P->bj_R) {
-    auto side = [&](const Prec::BjData &d) {
-      return BjSide{d.rec->p, d.seg->as<int32_t>(), d.bat->as<int32_t>(), d.cnt->as<uint16_t>()};
-    };
-    const int32_t blocks = P->bj_blocks, bsz = (P->n + blocks - 1) / blocks;
-    bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
-      if constexpr (std::is_same<decltype(s), S>::value)
-        hipLaunchKernelGGL((k_bj_lds<S, decltype(r)::value, decltype(w)::value>), dim3(P->bj_groups), dim3(kBlock),
-                           P->bj_lds, st, P->n, bsz, side(P->bj[0]), side(P->bj[1]), in, out);
-    });
+    MIo<S, S> io;
+    io.in = in;
+    io.out = out;
+    bj_apply<S, S>(P, io, st);
     return;
   }
   if (P->bj_blocks) {
@@ -1116,6 +1237,53 @@ void prec_apply_raw(Prec *P, const void *in, void *out, hipStream_t st) {
   }
   F3R_HIP(hipGetLastError());
 }
+
+// true when p (or a null pointer) is aligned to 4 elements
+template <class T> static bool align4(const T *p) { return ((uintptr_t)p % (4 * sizeof(T))) == 0; }
+
+template <class S, class F> void prec_apply_io(Prec *P, const MIo<S, F> &io, hipStream_t st) {
+  using ACC = typename Acc<S>::type;
+  const int64_t n = P->n;
+  const dim3 g(grid_for(n, P->ctx->num_cu)), b(kBlock);
+  if (P->kind == 0 && P->diag && io.raw && !io.add && !io.outf) {
+    const DiagWZ<S> d = diag_wz<S>(*P);
+    bool vec = align4(io.raw) && align4(io.vout) && align4(io.hin) && align4(io.out);
+    if constexpr (std::is_same<S, half_t>::value) vec = vec && align4(d.wz);
+    else vec = vec && align4(d.w) && align4(d.z);
+    auto kern = vec ? k_m_diag<S, F, true> : k_m_diag<S, F, false>;
+    hipLaunchKernelGGL(kern, dim3(vec ? grid_for((n + 3) / 4, P->ctx->num_cu) : g.x), b, 0, st, n, d, io);
+  } else if (P->kind == 0) {
+    S *tmp = P->tmp->as<S>();
+    SellArgs aw = sell_args(*P->W->sh, false), az = sell_args(*P->Z->sh, false);
+    const S *wv = P->W->s_val->as<S>(), *zv = P->Z->s_val->as<S>();
+    if (io.raw) {
+      const int K = P->W->sh->K;
+      auto kern = K == 1 ? k_m_entry_w<S, F, 1> : K == 2 ? k_m_entry_w<S, F, 2> : K == 4 ? k_m_entry_w<S, F, 4>
+                                                                                        : k_m_entry_w<S, F, 8>;
+      hipLaunchKernelGGL(kern, dim3(sell_blocks(aw, 0)), b, 0, st, aw, wv, io, tmp);
+    } else {
+      launch_sell<S, S, ACC>(P->W->sh->K, aw, wv, io.in, EpiStore<S, ACC>{tmp, nullptr}, st);
+    }
+    launch_sell<S, S, ACC>(P->Z->sh->K, az, zv, (const S *)tmp, EpiMExit<S, F>{io}, st);
+  } else if (P->bj_R) {
+    bj_apply<S, F>(P, io, st);
+  } else {
+    const S *in = io.in;
+    if (io.raw) {
+      if (io.hin || io.vout) hipLaunchKernelGGL((k_m_entry<S, F>), g, b, 0, st, n, io, io.hin);
+      if (io.hin) in = io.hin;
+      else if constexpr (std::is_same<S, F>::value) in = io.vout ? io.vout : io.raw;
+    }
+    const bool plain = !io.w && !io.outf;
+    S *x = plain || !io.add ? io.out : io.scratch;
+    prec_apply_raw(P, in, x, st);
+    if (!plain) hipLaunchKernelGGL((k_m_out<S, F>), g, b, 0, st, n, (const S *)x, io);
+  }
+  F3R_HIP(hipGetLastError());
+}
+template void prec_apply_io<half_t, float>(Prec *, const MIo<half_t, float> &, hipStream_t);
+template void prec_apply_io<float, float>(Prec *, const MIo<float, float> &, hipStream_t);
+template void prec_apply_io<double, double>(Prec *, const MIo<double, double> &, hipStream_t);
 
 HostCSR host_csr_from(int32_t nrows, int32_t ncols, int64_t nnz, const int32_t *rptr,
                       const int32_t *col, const double *val) {

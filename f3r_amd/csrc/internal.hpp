@@ -1,6 +1,8 @@
 // Declarations shared between the translation units of libf3r_amd.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "sell_kernel.hpp"
 
@@ -43,6 +45,94 @@ constexpr size_t kBjLdsBytes = 64 * 1024;
 // fewer diagonal blocks than this: one launch per level instead (a block
 // per workgroup would leave most of the GPU idle)
 constexpr int32_t kBjBlockKernel = 32;
+
+// One application of M inside the innermost level, with the element-wise work
+// around it: the entry from the basis vector above (normalised in passing and
+// converted to the storage type S) and the weighted update of the Richardson
+// iterate.  Every kind of M does these in its own kernels, so a call costs no
+// launch (2.4 to 4.9 us each at 64^3 to 96^3) beyond M's own.
+// S: storage and type of M; F: type of the basis vector (F = S outside the
+// HALF build, where nothing is scaled or converted).
+template <class S, class F> struct MIo {
+  // input: `in`, or the entry from `raw`
+  const S *in = nullptr;
+  const F *raw = nullptr;
+  const F *inv = nullptr;  // 1/||raw||; null: raw is normalised
+  F *vout = nullptr;       // the normalised vector (with inv; not raw: rows gather raw meanwhile)
+  F s = 1;                 // hin = S(raw * inv * s)
+  S *hin = nullptr;        // null with S = F: the normalised vector is M's input
+  // output: x = M in; out = x, S(x * w) with `w`, or S(fma(w, x, add)) with
+  // `add` too; outf (instead of out): the last, in F and unscaled
+  S *out = nullptr;
+  const double *w = nullptr;
+  const S *add = nullptr;
+  F *outf = nullptr;
+  F inv_s = 1;
+  S *scratch = nullptr;  // a vector of S for kinds of M without fused kernels (with add)
+};
+template <class S, class F> void prec_apply_io(Prec *P, const MIo<S, F> &io, hipStream_t st);
+
+// the entry of one element
+template <class S, class F> struct MEntry {
+  F iv, s;
+  bool has_inv;
+  __device__ explicit MEntry(const MIo<S, F> &io) : iv(io.inv ? *io.inv : (F)1), s(io.s), has_inv(io.inv != nullptr) {}
+  __device__ __forceinline__ F norm(F v) const { return has_inv ? v * iv : v; }
+  __device__ __forceinline__ S store(F v) const {  // v normalised
+    if constexpr (std::is_same<S, F>::value) return v; else return cvt<S>(v * s);
+  }
+  __device__ __forceinline__ auto operator()(F v) const { return to_acc(store(norm(v))); }
+};
+// the output of one element
+template <class S, class F> struct MExit {
+  using A = typename Acc<S>::type;
+  S *out;
+  const S *add;
+  F *outf;
+  A w;
+  F inv_s;
+  bool weighted;
+  __device__ explicit MExit(const MIo<S, F> &io)
+      : out(io.out), add(io.add), outf(io.outf), w(io.w ? (A)*io.w : (A)1), inv_s(io.inv_s), weighted(io.w != nullptr) {}
+  __device__ __forceinline__ S pre(int64_t r) const { return add ? add[r] : S(0); }
+  __device__ __forceinline__ S value(S x, S ad) const {
+    if (!weighted) return x;
+    return add ? cvt<S>(fma_<A>(w, to_acc(x), to_acc(ad))) : cvt<S>(to_acc(x) * w);
+  }
+  __device__ __forceinline__ void put(int64_t r, S x, S ad) const {
+    const S h = value(x, ad);
+    if (outf) outf[r] = (F)to_acc(h) * inv_s;
+    else out[r] = h;
+  }
+};
+// a row's diagonal factors (w, z): one 32-bit word in fp16
+template <class S> struct DiagWZ {
+  const S *w = nullptr, *z = nullptr;
+  struct V {
+    S w, z;
+  };
+  __device__ __forceinline__ V at(int64_t r) const { return {w[r], z[r]}; }
+};
+template <> struct DiagWZ<half_t> {
+  const uint32_t *wz = nullptr;
+  struct V {
+    half_t w, z;
+  };
+  static __device__ __forceinline__ V unpack(uint32_t v) {
+    return {__builtin_bit_cast(half_t, (uint16_t)(v & 0xffffu)), __builtin_bit_cast(half_t, (uint16_t)(v >> 16))};
+  }
+  __device__ __forceinline__ V at(int64_t r) const { return unpack(wz[r]); }
+};
+template <class S> inline DiagWZ<S> diag_wz(const Prec &P) {
+  if constexpr (std::is_same<S, half_t>::value) return {P.dwz->template as<uint32_t>()};
+  else return {P.dw->template as<S>(), P.dz->template as<S>()};
+}
+// z (w x) of a row, each product rounded to S
+template <class S> __device__ __forceinline__ S diag_apply(const typename DiagWZ<S>::V &d, S x) {
+  using A = typename Acc<S>::type;
+  const S t = cvt<S>(fma_<A>(to_acc(d.w), to_acc(x), (A)0));
+  return cvt<S>(fma_<A>(to_acc(d.z), to_acc(t), (A)0));
+}
 
 std::shared_ptr<Context> ctx_create(int device);
 double read_scalar(Context *c, const double *dev);

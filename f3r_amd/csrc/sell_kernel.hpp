@@ -61,16 +61,22 @@ __device__ __forceinline__ X buffer_gather(__amdgpu_buffer_rsrc_t rs, int voff, 
   }
 }
 
+// what a gathered element of x stands for in the sum: itself, or a value
+// computed from it (the preconditioner's entry, internal.hpp)
+struct XValue {
+  template <class X> __device__ __forceinline__ auto operator()(X v) const { return to_acc(v); }
+};
+
 #ifndef F3R_FIXED_ROWS
 #define F3R_FIXED_ROWS 1
 #endif
 // Row of an offset chunk of G full groups and, if HALF, a half group, with
 // every value load and x gather issued before the first multiply-add (a
 // runtime loop keeps one or two groups in flight).  Same sum, same order.
-template <int G, bool HALF, class V, class X, class ACC, int K>
+template <int G, bool HALF, class V, class X, class ACC, int K, class XF>
 __device__ __forceinline__ ACC sell_row_fixed(const V *__restrict__ val, int64_t pos, int64_t step, int64_t hpos,
                                               __amdgpu_buffer_rsrc_t rs, int vo, int bias,
-                                              const __attribute__((address_space(4))) int32_t *off) {
+                                              const __attribute__((address_space(4))) int32_t *off, const XF &xf) {
   constexpr int H = K / 2;
   Pack<V, K> pv[G];
   X xv[G][K];
@@ -91,18 +97,18 @@ __device__ __forceinline__ ACC sell_row_fixed(const V *__restrict__ val, int64_t
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv[g].v[k]), (ACC)to_acc(xv[g][k]), acc);
+    for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv[g].v[k]), (ACC)xf(xv[g][k]), acc);
   if constexpr (HALF) {
 #pragma unroll
-    for (int k = 0; k < H; ++k) acc = fma_<ACC>((ACC)to_acc(ph.v[k]), (ACC)to_acc(xh[k]), acc);
+    for (int k = 0; k < H; ++k) acc = fma_<ACC>((ACC)to_acc(ph.v[k]), (ACC)xf(xh[k]), acc);
   }
   return acc;
 }
 
 // Sum of row r (in sorted order) of A*x with accumulator ACC.
-template <class V, class X, class ACC, int K>
+template <class V, class X, class ACC, int K, class XF = XValue>
 __device__ __forceinline__ ACC sell_row(const SellArgs &a, const V *__restrict__ val,
-                                        const X *__restrict__ x, int r) {
+                                        const X *__restrict__ x, int r, const XF &xf = XF()) {
   const int s = r >> a.log2C;
   const int j = r - (s << a.log2C);
   const int C = 1 << a.log2C;
@@ -138,16 +144,17 @@ __device__ __forceinline__ ACC sell_row(const SellArgs &a, const V *__restrict__
         const int cwu = __builtin_amdgcn_readfirstlane(cw);
         const int64_t hpos = (int64_t)a.cptr[s] + (int64_t)groups * step + (int64_t)j * (K / 2);
         if constexpr (K == 8) {
-          if (cwu == (3 | kHalfTail)) return sell_row_fixed<3, true, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
-          if (cwu == 4) return sell_row_fixed<4, false, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
-          if (cwu == 1) return sell_row_fixed<1, false, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
+          if (cwu == (3 | kHalfTail)) return sell_row_fixed<3, true, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
+          if (cwu == 4) return sell_row_fixed<4, false, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
+          if (cwu == 1) return sell_row_fixed<1, false, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
         } else if constexpr (K == 4) {
-          if (cwu == 7) return sell_row_fixed<7, false, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
-          if (cwu == 2) return sell_row_fixed<2, false, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
+          if (cwu == 7) return sell_row_fixed<7, false, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
+          if (cwu == 2) return sell_row_fixed<2, false, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
+          if (cwu == 1) return sell_row_fixed<1, false, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
         } else if constexpr (K == 2) {
-          if (cwu == (13 | kHalfTail)) return sell_row_fixed<13, true, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
-          if (cwu == 14) return sell_row_fixed<14, false, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
-          if (cwu == (3 | kHalfTail)) return sell_row_fixed<3, true, V, X, ACC, K>(val, pos, step, hpos, rs, vo, bias, off);
+          if (cwu == (13 | kHalfTail)) return sell_row_fixed<13, true, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
+          if (cwu == 14) return sell_row_fixed<14, false, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
+          if (cwu == (3 | kHalfTail)) return sell_row_fixed<3, true, V, X, ACC, K, XF>(val, pos, step, hpos, rs, vo, bias, off, xf);
         }
       }
 #endif
@@ -158,7 +165,7 @@ __device__ __forceinline__ ACC sell_row(const SellArgs &a, const V *__restrict__
 #pragma unroll
         for (int k = 0; k < K; ++k) xv[k] = buffer_gather<X>(rs, vo, (off[g * K + k] + bias) * (int)sizeof(X));
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xv[k]), acc);
+        for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)xf(xv[k]), acc);
       }
       if constexpr (K >= 2) {
         if (cw & kHalfTail) {  // the half group: K / 2 slots per row, rows consecutive
@@ -168,7 +175,7 @@ __device__ __forceinline__ ACC sell_row(const SellArgs &a, const V *__restrict__
 #pragma unroll
           for (int k = 0; k < H; ++k) xv[k] = buffer_gather<X>(rs, vo, (off[groups * K + k] + bias) * (int)sizeof(X));
 #pragma unroll
-          for (int k = 0; k < H; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xv[k]), acc);
+          for (int k = 0; k < H; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)xf(xv[k]), acc);
         }
       }
 #else
@@ -180,7 +187,7 @@ __device__ __forceinline__ ACC sell_row(const SellArgs &a, const V *__restrict__
 #pragma unroll
         for (int k = 0; k < K; ++k) xv[k] = xr[off[g * K + k]];
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xv[k]), acc);
+        for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)xf(xv[k]), acc);
       }
       if constexpr (K >= 2) {
         if (cw & kHalfTail) {
@@ -188,7 +195,7 @@ __device__ __forceinline__ ACC sell_row(const SellArgs &a, const V *__restrict__
           const Pack<V, H> pv = load_pack<V, H>(val + ((int64_t)a.cptr[s] + (int64_t)groups * step + (int64_t)j * H));
 #pragma unroll
           for (int k = 0; k < H; ++k)
-            acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xr[off[groups * K + k]]), acc);
+            acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)xf(xr[off[groups * K + k]]), acc);
         }
       }
 #endif
@@ -200,7 +207,7 @@ __device__ __forceinline__ ACC sell_row(const SellArgs &a, const V *__restrict__
     const Pack<V, K> pv = load_pack<V, K>(val + pos);
     const Pack<int32_t, K> pi = load_pack<int32_t, K>(ip);
 #pragma unroll
-    for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(x[pi.v[k]]), acc);
+    for (int k = 0; k < K; ++k) acc = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)xf(x[pi.v[k]]), acc);
   }
   return acc;
 }

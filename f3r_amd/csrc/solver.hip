@@ -421,115 +421,61 @@ __global__ void k_scatter(int64_t n, const double *__restrict__ s, const int32_t
     d[perm[i]] = s[i];
 }
 
-// ---------------------------------------------- Richardson (fp16 level) ---
-// the interleaved diagonal factors of a row: (w, z) in one 32-bit word
-__device__ __forceinline__ half_t dwz_w(uint32_t v) { return __builtin_bit_cast(half_t, (uint16_t)(v & 0xffffu)); }
-__device__ __forceinline__ half_t dwz_z(uint32_t v) { return __builtin_bit_cast(half_t, (uint16_t)(v >> 16)); }
-// Entry of one call (work/src/f3r-gpu.cpp:231-243 in this build's
-// arithmetic): hin = fp16(in * s); with diagonal SDAINV factors also
-// hout = fp16(z * fp16(w * hin)) and, outside probe calls, hout *= ome_0.
-// `inv` (optional): `in` is a basis vector not yet normalised; it is scaled
-// by *inv in place first (the normalisation of the Arnoldi step that made it).
-// VEC: 4 consecutive rows per lane (every array 4-element aligned).
-__device__ __forceinline__ void l4_entry_row(float &v, const float iv, bool has_inv, float s, half_t &h, half_t &o,
-                                             half_t dwi, half_t dzi, bool diag, bool scale_ome, float om) {
-  if (has_inv) v *= iv;
-  h = cvt<half_t>(v * s);
-  if (diag) {
-    const half_t t = cvt<half_t>(__builtin_fmaf((float)dwi, (float)h, 0.f));
-    o = cvt<half_t>(__builtin_fmaf((float)dzi, (float)t, 0.f));
-    if (scale_ome) o = cvt<half_t>((float)o * om);
-  }
-}
-template <bool VEC>
-__global__ void k_l4_entry(int64_t n, float *__restrict__ in, const float *__restrict__ inv, float s,
-                           half_t *__restrict__ hin, half_t *__restrict__ hout, const uint32_t *__restrict__ dwz,
-                           const RichDev *st, int scale_ome) {
-  const float om = scale_ome ? (float)st->ome[0] : 1.f;
-  const float iv = inv ? *inv : 1.f;
-  const bool diag = dwz != nullptr;
-  const int64_t gid = blockIdx.x * (int64_t)kBlock + threadIdx.x, gstride = (int64_t)gridDim.x * kBlock;
-  int64_t i0 = 0;
-  if constexpr (VEC) {
-    const int64_t n4 = n / 4;
-    for (int64_t q = gid; q < n4; q += gstride) {
-      V4<float> v = ld4(in + 4 * q);
-      V4<uint32_t> wz{};
-      V4<half_t> h, o{};
-      if (diag) wz = ld4(dwz + 4 * q);
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        l4_entry_row(v.v[c], iv, inv != nullptr, s, h.v[c], o.v[c], dwz_w(wz.v[c]), dwz_z(wz.v[c]), diag,
-                     scale_ome != 0, om);
-      if (inv) st4(in + 4 * q, v);
-      st4(hin + 4 * q, h);
-      if (diag) st4(hout + 4 * q, o);
-    }
-    i0 = 4 * n4;
-  }
-  for (int64_t i = i0 + gid; i < n; i += gstride) {
-    float v = in[i];
-    half_t h, o = (half_t)0;
-    const uint32_t wz = diag ? dwz[i] : 0u;
-    l4_entry_row(v, iv, inv != nullptr, s, h, o, dwz_w(wz), dwz_z(wz), diag, scale_ome != 0, om);
-    if (inv) in[i] = v;
-    hin[i] = h;
-    if (diag) hout[i] = o;
-  }
-}
-
-// hout *= ome_0 (or alpha_0 in probe calls)
-__global__ void k_l4_scale(int64_t n, half_t *__restrict__ hout, const double *w) {
-  const float a = (float)*w;
+// ------------------------------------------------- Richardson level ---
+// hout *= alpha_0 in probe calls
+template <class S> __global__ void k_l4_scale(int64_t n, S *__restrict__ hout, const double *w) {
+  using A = typename Acc<S>::type;
+  const A a = (A)*w;
   for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-    hout[i] = cvt<half_t>((float)hout[i] * a);
+    hout[i] = cvt<S>(to_acc(hout[i]) * a);
 }
 
-// hout' = fp16(fma(w_k, tmp2, hout)); last step: out = fp32(hout') / s
-__global__ void k_l4_update(int64_t n, const half_t *__restrict__ tmp2, const half_t *__restrict__ hout,
-                            const double *w, half_t *__restrict__ hnext, float *__restrict__ out,
-                            float inv_s) {
-  const float a = (float)*w;
+// hout' = S(fma(w_k, tmp2, hout)); with `out` (last step): out = F(hout') / s
+template <class S, class F>
+__global__ void k_l4_update(int64_t n, const S *__restrict__ tmp2, const S *__restrict__ hout, const double *w,
+                            S *__restrict__ hnext, F *__restrict__ out, F inv_s) {
+  using A = typename Acc<S>::type;
+  const A a = (A)*w;
   for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const half_t h = cvt<half_t>(__builtin_fmaf(a, (float)tmp2[i], (float)hout[i]));
+    const S h = cvt<S>(fma_<A>(a, to_acc(tmp2[i]), to_acc(hout[i])));
     if (out)
-      out[i] = (float)h * inv_s;
+      out[i] = (F)to_acc(h) * inv_s;
     else
       hnext[i] = h;
   }
 }
 
-// Richardson step k fused into the fp16 residual SpMV, diagonal factors:
-// hr = fp16(hin - A16 hout), tmp2 = fp16(z * fp16(w * hr)), and outside
-// probe calls hout' = fp16(fma(ome_k, tmp2, hout)) (last step: out = hout'/s).
-struct EpiL4Diag {
+// Richardson step k fused into the residual SpMV, diagonal factors:
+// hr = S(hin - A hout), tmp2 = S(z * S(w * hr)), and outside probe calls
+// hout' = S(fma(ome_k, tmp2, hout)) (last step with `out`: out = hout'/s).
+template <class S, class F, class ACC> struct EpiL4Diag {
   using State = NoState;
+  using A = typename Acc<S>::type;
   struct Pre {
-    half_t hin, hout;
-    uint32_t wz;
+    S hin, hout;
+    typename DiagWZ<S>::V wz;
   };
-  const half_t *__restrict__ hin;
-  const half_t *__restrict__ hout;
-  const uint32_t *__restrict__ dwz;  // (w, z) diagonals interleaved
+  const S *__restrict__ hin;
+  const S *__restrict__ hout;
+  DiagWZ<S> d;
   const double *w;  // ome_k
-  half_t *__restrict__ hr_out;    // probe calls: keep hr and tmp2
-  half_t *__restrict__ tmp2_out;
-  half_t *__restrict__ hnext;
-  float *__restrict__ out;
-  float inv_s;
-  __device__ Pre pre(int r) const { return {hin[r], hr_out ? (half_t)0 : hout[r], dwz[r]}; }
-  __device__ void row(int r, float acc, const Pre &p, State &) const {
-    const half_t hr = cvt<half_t>((float)p.hin - acc);
-    const half_t t = cvt<half_t>(__builtin_fmaf((float)dwz_w(p.wz), (float)hr, 0.f));
-    const half_t t2 = cvt<half_t>(__builtin_fmaf((float)dwz_z(p.wz), (float)t, 0.f));
+  S *__restrict__ hr_out;    // probe calls: keep hr and tmp2
+  S *__restrict__ tmp2_out;
+  S *__restrict__ hnext;
+  F *__restrict__ out;
+  F inv_s;
+  __device__ Pre pre(int r) const { return {hin[r], hr_out ? S(0) : hout[r], d.at(r)}; }
+  __device__ void row(int r, ACC acc, const Pre &p, State &) const {
+    const S hr = cvt<S>((ACC)to_acc(p.hin) - acc);
+    const S t2 = diag_apply<S>(p.wz, hr);
     if (hr_out) {
       hr_out[r] = hr;
       tmp2_out[r] = t2;
       return;
     }
-    const half_t h = cvt<half_t>(__builtin_fmaf((float)*w, (float)t2, (float)p.hout));
+    const S h = cvt<S>(fma_<A>((A)*w, to_acc(t2), to_acc(p.hout)));
     if (out)
-      out[r] = (float)h * inv_s;
+      out[r] = (F)to_acc(h) * inv_s;
     else
       hnext[r] = h;
   }
@@ -538,21 +484,23 @@ struct EpiL4Diag {
 
 // probe: alpha_k = <t, r> / <t, t> (fp32 sums of fp16 data); the last block
 // updates sum_k, ome_k (work/src/f3r-gpu.cpp:234-240, 248-254)
-__global__ __launch_bounds__(kBlock) void k_probe(int64_t n, const half_t *__restrict__ t,
-                                                  const half_t *__restrict__ r, RichDev *st, int k,
-                                                  float *partial, unsigned *counter) {
-  __shared__ float lds[2 * kWavesPerBlock];
-  float v[2] = {0.f, 0.f};
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_probe(int64_t n, const S *__restrict__ t, const S *__restrict__ r,
+                                                  RichDev *st, int k, typename Acc<S>::type *partial,
+                                                  unsigned *counter) {
+  using A = typename Acc<S>::type;
+  __shared__ A lds[2 * kWavesPerBlock];
+  A v[2] = {0, 0};
   for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const float ti = (float)t[i];
-    v[0] = __builtin_fmaf(ti, ti, v[0]);
-    v[1] = __builtin_fmaf(ti, (float)r[i], v[1]);
+    const A ti = to_acc(t[i]);
+    v[0] = fma_<A>(ti, ti, v[0]);
+    v[1] = fma_<A>(ti, to_acc(r[i]), v[1]);
   }
-  if (grid_sum<float, 2>(v, partial, counter, lds) && threadIdx.x == 0) {
-    const float al = v[1] / v[0];
+  if (grid_sum<A, 2>(v, partial, counter, lds) && threadIdx.x == 0) {
+    const A al = v[1] / v[0];
     if (k == 0) st->nprobe += 1;
-    const float den = (float)(st->nprobe + 1);
-    const float s = (float)st->sum[k] + al;
+    const A den = (A)(st->nprobe + 1);
+    const A s = (A)st->sum[k] + al;
     st->sum[k] = s;
     st->ome[k] = s / den;
     st->alpha[k] = al;
@@ -568,41 +516,6 @@ __global__ void k_rich_reset(RichDev *st, double w) {
       st->alpha[k] = 0.0;
     }
     st->nprobe = 0;
-  }
-}
-
-// ---------------------------- Richardson of the FLOAT / DOUBLE builds ---
-template <class T>
-__global__ void k_scale_t(int64_t n, T *__restrict__ out, const double *w) {
-  const T a = (T)*w;
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-    out[i] *= a;
-}
-template <class T>
-__global__ void k_update_t(int64_t n, const T *__restrict__ t2, T *__restrict__ out, const double *w) {
-  const T a = (T)*w;
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-    out[i] = fma_<T>(a, t2[i], out[i]);
-}
-// alpha_k = <t, r> / <t, t> summed in T; the last block updates sum_k, ome_k
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_probe_t(int64_t n, const T *__restrict__ t, const T *__restrict__ r,
-                                                    RichDev *st, int k, T *partial, unsigned *counter) {
-  __shared__ T lds[2 * kWavesPerBlock];
-  T v[2] = {0, 0};
-  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    const T ti = t[i];
-    v[0] = fma_<T>(ti, ti, v[0]);
-    v[1] = fma_<T>(ti, r[i], v[1]);
-  }
-  if (grid_sum<T, 2>(v, partial, counter, lds) && threadIdx.x == 0) {
-    const T al = v[1] / v[0];
-    if (k == 0) st->nprobe += 1;
-    const T den = (T)(st->nprobe + 1);
-    const T s = (T)st->sum[k] + al;
-    st->sum[k] = s;
-    st->ome[k] = s / den;
-    st->alpha[k] = al;
   }
 }
 
@@ -704,6 +617,10 @@ template <class T> struct InnerLevel {
   int m = 0;
   DevPtr Vbuf, Zbuf, H, cs, sn, e, inv;
   std::vector<T *> V, Z;  // column pointers; V[0] aliases the level's input
+  // w = A z_j of the running step: V[j + 1] before its normalisation, which
+  // the next innermost entry writes as it reads w (rows gather w meanwhile)
+  DevPtr wbuf;
+  T *w() const { return wbuf->as<T>(); }
   // level 3 of the HALF variant: Z_j as the fp16 Richardson output h
   // (Z_j = h / s exactly, s the power-of-two range scale), half the bytes
   DevPtr Zhbuf;
@@ -757,9 +674,12 @@ struct Solver {
   std::vector<double> hist;
   std::map<uint64_t, hipGraphExec_t> graphs;
   std::vector<hipGraph_t> graph_src;
-  // 1/||w|| of a basis vector left unnormalised by the last Arnoldi step;
-  // the next innermost entry kernel (its first reader) applies it
-  const float *pending_inv = nullptr;
+  // the last Arnoldi step's w and 1/||w||, still to be written to its basis
+  // column: the next innermost entry (the column's first reader) does it
+  struct Pending {
+    const void *w = nullptr, *inv = nullptr;
+    void *col = nullptr;
+  } pending;
   bool layouts_on_device = false;  // the matrix layouts were built on the device
   int red_grid = 1;   // capped grid of the outer level's strided reductions
   int dots_grid = 1;  // blocks of the streaming kernels with a grid reduction
@@ -802,7 +722,7 @@ struct Solver {
   void spmv_dots(InnerLevel<T> &L, const V *val, int j) {
     Cols<T, NV> c{};
     for (int k = 0; k <= j; ++k) c.p[k] = L.V[k];
-    EpiDots<T, NV> epi{L.V[j + 1], c, j + 1, L.Hp() + (int64_t)j * L.ldh(), partial<T>(), counter(0)};
+    EpiDots<T, NV> epi{L.w(), c, j + 1, L.Hp() + (int64_t)j * L.ldh(), partial<T>(), counter(0)};
     if (!L.Zh.empty()) {
       epi.xs = (T)(1.0 / range_s);
       launch_sell<V, half_t, T>(shv<V>().K, argsv<V>(), val, L.Zh[j], epi, st(), spmv_grid);
@@ -816,11 +736,11 @@ struct Solver {
   template <class T, int NV> void cgs_update(InnerLevel<T> &L, int j) {
     Cols<T, NV> c{};
     for (int k = 0; k <= j; ++k) c.p[k] = L.V[k];
-    bool vec = aligned4(L.V[j + 1]);
+    bool vec = true;
     for (int k = 0; k <= j; ++k) vec = vec && aligned4(L.V[k]);
     auto kern = vec ? k_cgs_update<T, NV, true> : k_cgs_update<T, NV, false>;
     hipLaunchKernelGGL(kern, dim3(dots_grid), dim3(kBlock), 0, st(), (int64_t)n,
-                       L.V[j + 1], c, j + 1, L.Hp() + (int64_t)j * L.ldh(), L.cs->template as<T>(),
+                       L.w(), c, j + 1, L.Hp() + (int64_t)j * L.ldh(), L.cs->template as<T>(),
                        L.sn->template as<T>(), L.e->template as<T>(), j, 1, L.inv->template as<T>(),
                        (double *)nullptr, partial<T>(), counter(1), j + 1 < L.m ? 1 : 0);
   }
@@ -836,20 +756,10 @@ struct Solver {
       cgs_update<T, 16>(L, j);
     }
     // the last basis vector of an inner level is never read (the level's
-    // output is Z y), so it is left unnormalised.  In the HALF variant the
-    // first reader of V[j+1] is the next innermost entry kernel (level 3's
-    // next step, or level 3's start when this is level 2), which normalises
-    // it in passing.
-    if (j + 1 < L.m) {
-      if constexpr (std::is_same<T, float>::value) {
-        if (p.variant == 0) {
-          pending_inv = L.inv->template as<float>();
-          return;
-        }
-      }
-      hipLaunchKernelGGL(k_vscale<T>, dim3(grid()), dim3(kBlock), 0, st(), (int64_t)n, L.V[j + 1],
-                         (const T *)L.inv->template as<T>());
-    }
+    // output is Z y).  The first reader of the others is the next innermost
+    // entry (level 3's next step, or level 3's start when this is level 2),
+    // which normalises w into its column in passing.
+    if (j + 1 < L.m) pending = {L.w(), L.inv->p, L.V[j + 1]};
   }
   template <class T, class TO> void solution(InnerLevel<T> &L, TO *out) {
     const int j = L.m;
@@ -878,132 +788,110 @@ struct Solver {
     else go(std::integral_constant<int, 16>());
   }
 
-  // ------------------------------------------------- level 4 (fp16) ---
-  // out: fp32 result h / s; or, with hz, the fp16 result h itself
-  void level4_half(const float *in, float *out, half_t *hz = nullptr) {
+  // --------------------------------------------------------- level 4 ---
+  // The adaptive Richardson on storage S (fp16 in HALF, else the basis type
+  // F): vectors and weights in S, M in S, products with the values MV summed
+  // in ACC (FLOAT / DOUBLE: the fp64 A summed in fp64, work/src/f3r-gpu.cpp:
+  // 123-152, 174-203).  The result goes to `hz` (S), or h / s to `out` (F).
+  template <class S, class F, class MV, class ACC>
+  void richardson(const F *in, F *out, S *hz, const MV *aval, const SellShared &lay) {
     ++cnt;
     ++calls;
     const bool probe = p.static_weight <= 0 && (cnt % p.c) == 0;
     const int64_t nn = n;
     const dim3 g(grid()), b(kBlock);
     RichDev *rs = rich->as<RichDev>();
-    half_t *hi = hin->as<half_t>(), *ho = hout->as<half_t>(), *ho2 = hout2->as<half_t>();
-    const float inv_s = 1.f / range_s;
+    const F inv_s = (F)(1.f / range_s);
     const bool diag = P->kind == 0 && P->diag;
-    const uint32_t *dwz = diag ? P->dwz->as<uint32_t>() : nullptr;
-    const half_t *a16 = A16->as<half_t>();
-    SellArgs a = argsv<half_t>();
-    const int K16 = sh16->K;
-    // entry (normalising `in` first when the Arnoldi step that made it did not)
-    const float *pinv = pending_inv;
-    pending_inv = nullptr;
-    const bool vec = aligned4(in) && aligned4(hi) && aligned4(ho) && (!diag || aligned4(dwz));
-    if (vec)
-      hipLaunchKernelGGL(k_l4_entry<true>, g, b, 0, st(), nn, const_cast<float *>(in), pinv, range_s, hi, ho, dwz,
-                         (const RichDev *)rs, (diag && !probe) ? 1 : 0);
-    else
-      hipLaunchKernelGGL(k_l4_entry<false>, g, b, 0, st(), nn, const_cast<float *>(in), pinv, range_s, hi, ho, dwz,
-                         (const RichDev *)rs, (diag && !probe) ? 1 : 0);
-    if (!diag) {
-      prec_apply_raw(P.get(), hi, ho, st());
-      if (!probe) hipLaunchKernelGGL(k_l4_scale, g, b, 0, st(), nn, ho, (const double *)&rs->ome[0]);
+    const SellArgs a = sell_args(lay, false);
+    constexpr bool kSame = std::is_same<S, F>::value;
+    S *hi = hin->as<S>(), *ho = hout->as<S>(), *ho2 = hout2->as<S>();
+    S *hr_ = hr->as<S>(), *t2 = tmp2->as<S>(), *t = tt->as<S>();
+    if constexpr (kSame) hz = out;
+    if (p.m4 == 1 && hz) ho = hz;  // no Richardson step
+    // entry (normalising `in` first when the Arnoldi step that made it did
+    // not), M, and outside probe calls the first weight
+    MIo<S, F> io;
+    io.raw = in;
+    if (pending.col == in) {
+      io.raw = static_cast<const F *>(pending.w);
+      io.inv = static_cast<const F *>(pending.inv);
+      io.vout = const_cast<F *>(in);
     }
+    pending = Pending();
+    io.s = (F)range_s;
+    if constexpr (kSame) hi = const_cast<F *>(in);
+    else io.hin = hi;
+    io.out = ho;
+    io.w = probe ? nullptr : &rs->ome[0];
+    prec_apply_io<S, F>(P.get(), io, st());
+    auto product = [&](const S *x, S *y) {
+      launch_sell<MV, S, ACC>(lay.K, a, aval, x, EpiStore<S, ACC>{y, nullptr}, st());
+    };
+    auto probe_dots = [&](const S *ts, const S *r, int k) {
+      hipLaunchKernelGGL(k_probe<S>, dim3(dots_grid), b, 0, st(), nn, ts, r, rs, k,
+                         partial<typename Acc<S>::type>(), counter(2));
+    };
     if (probe) {
-      half_t *t = tt->as<half_t>();
-      launch_sell<half_t, half_t, float>(K16, a, a16, ho, EpiStore<half_t, float>{t, nullptr}, st());
-      hipLaunchKernelGGL(k_probe, dim3(dots_grid), b, 0, st(), nn, (const half_t *)t, (const half_t *)hi, rs,
-                         0, partial<float>(), counter(2));
-      hipLaunchKernelGGL(k_l4_scale, g, b, 0, st(), nn, ho, (const double *)&rs->alpha[0]);
+      product(ho, t);
+      probe_dots(t, hi, 0);
+      hipLaunchKernelGGL(k_l4_scale<S>, g, b, 0, st(), nn, ho, (const double *)&rs->alpha[0]);
     }
     for (int k = 1; k < p.m4; ++k) {
       const bool last = k == p.m4 - 1;
-      half_t *hr_ = hr->as<half_t>(), *t2 = tmp2->as<half_t>();
-      half_t *hn = last && hz ? hz : ho2;     // the step's fp16 result
-      float *of = last && !hz ? out : nullptr;  // or, last step, its fp32 h / s
+      S *hn = last && hz ? hz : ho2;            // the step's result in S
+      F *of = last && !hz ? out : nullptr;      // or, last step, h / s
       if (diag) {
-        EpiL4Diag epi{hi, ho, dwz, &rs->ome[k], probe ? hr_ : nullptr, probe ? t2 : nullptr,
-                      hn, of, inv_s};
-        launch_sell<half_t, half_t, float>(K16, a, a16, ho, epi, st());
+        EpiL4Diag<S, F, ACC> epi{hi, ho, diag_wz<S>(*P), &rs->ome[k], probe ? hr_ : nullptr, probe ? t2 : nullptr,
+                                 hn, of, inv_s};
+        launch_sell<MV, S, ACC>(lay.K, a, aval, ho, epi, st());
       } else {
-        launch_sell<half_t, half_t, float>(K16, a, a16, ho, EpiResid<half_t, half_t, float>{hr_, hi, nullptr},
-                                           st());
-        prec_apply_raw(P.get(), hr_, t2, st());
+        launch_sell<MV, S, ACC>(lay.K, a, aval, ho, EpiResid<S, S, ACC>{hr_, hi, nullptr}, st());
+        MIo<S, F> up;
+        up.in = hr_;
+        up.out = t2;
+        if (!probe) {
+          up.out = hn;
+          up.outf = of;
+          up.w = &rs->ome[k];
+          up.add = ho;
+          up.inv_s = inv_s;
+          up.scratch = t2;
+        }
+        prec_apply_io<S, F>(P.get(), up, st());
       }
       if (probe) {
-        half_t *t = tt->as<half_t>();
-        launch_sell<half_t, half_t, float>(K16, a, a16, t2, EpiStore<half_t, float>{t, nullptr}, st());
-        hipLaunchKernelGGL(k_probe, dim3(dots_grid), b, 0, st(), nn, (const half_t *)t, (const half_t *)hr_, rs,
-                           k, partial<float>(), counter(2));
-        hipLaunchKernelGGL(k_l4_update, g, b, 0, st(), nn, (const half_t *)t2, (const half_t *)ho,
+        product(t2, t);
+        probe_dots(t, hr_, k);
+        hipLaunchKernelGGL((k_l4_update<S, F>), g, b, 0, st(), nn, (const S *)t2, (const S *)ho,
                            (const double *)&rs->alpha[k], hn, of, inv_s);
-      } else if (!diag) {
-        hipLaunchKernelGGL(k_l4_update, g, b, 0, st(), nn, (const half_t *)t2, (const half_t *)ho,
-                           (const double *)&rs->ome[k], hn, of, inv_s);
       }
       if (!last) std::swap(ho, ho2);
     }
-    if (p.m4 == 1) {  // no Richardson step: out = fp32(hout) / s, or hz = hout
-      if (hz)
-        hipLaunchKernelGGL((k_cast2<half_t, half_t>), g, b, 0, st(), nn, (const half_t *)ho, hz);
-      else
-        hipLaunchKernelGGL((k_g_entry<half_t, float>), g, b, 0, st(), nn, (const half_t *)ho, out, (double)inv_s);
-    }
-  }
-
-  // ------------------------------------ level 4 of the FLOAT / DOUBLE builds ---
-  // Vectors and weights in T, preconditioner in T, SpMVs with the fp64 A
-  // summed in fp64 (work/src/f3r-gpu.cpp:123-152, 174-203); `out` is updated
-  // in place.
-  template <class T> void level4_t(const T *in, T *out) {
-    ++cnt;
-    ++calls;
-    const bool probe = p.static_weight <= 0 && (cnt % p.c) == 0;
-    const int64_t nn = n;
-    const dim3 g(grid()), b(kBlock);
-    RichDev *rs = rich->as<RichDev>();
-    const double *a64 = A64->as<double>();
-    SellArgs a = args();
-    T *t = tt->as<T>(), *hr_ = hr->as<T>(), *t2 = tmp2->as<T>();
-    prec_apply_raw(P.get(), in, out, st());
-    if (probe) {
-      launch_sell<double, T, double>(sh->K, a, a64, out, EpiStore<T, double>{t, nullptr}, st());
-      hipLaunchKernelGGL(k_probe_t<T>, dim3(dots_grid), b, 0, st(), nn, (const T *)t, in, rs, 0, partial<T>(),
-                         counter(2));
-      hipLaunchKernelGGL(k_scale_t<T>, g, b, 0, st(), nn, out, (const double *)&rs->alpha[0]);
-    } else {
-      hipLaunchKernelGGL(k_scale_t<T>, g, b, 0, st(), nn, out, (const double *)&rs->ome[0]);
-    }
-    for (int k = 1; k < p.m4; ++k) {
-      launch_sell<double, T, double>(sh->K, a, a64, out, EpiResid<T, T, double>{hr_, in, nullptr}, st());
-      prec_apply_raw(P.get(), hr_, t2, st());
-      if (probe) {
-        launch_sell<double, T, double>(sh->K, a, a64, t2, EpiStore<T, double>{t, nullptr}, st());
-        hipLaunchKernelGGL(k_probe_t<T>, dim3(dots_grid), b, 0, st(), nn, (const T *)t, (const T *)hr_, rs, k,
-                           partial<T>(), counter(2));
-        hipLaunchKernelGGL(k_update_t<T>, g, b, 0, st(), nn, (const T *)t2, out, (const double *)&rs->alpha[k]);
-      } else {
-        hipLaunchKernelGGL(k_update_t<T>, g, b, 0, st(), nn, (const T *)t2, out, (const double *)&rs->ome[k]);
-      }
-    }
+    if (p.m4 == 1 && !hz)  // out = F(hout) / s
+      hipLaunchKernelGGL((k_g_entry<S, F>), g, b, 0, st(), nn, (const S *)ho, out, (double)inv_s);
   }
 
   // hz (HALF variant, level 3): the fp16 result instead of `out`
   template <class T> void level4(const T *in, T *out, half_t *hz = nullptr) {
     if (capturing() && calls % cap_every == 0) {
       float *dst = cap->as<float>() + (int64_t)cap_n * n;
+      // a basis vector still to be normalised is recorded as it is
+      const T *src = pending.col == in ? static_cast<const T *>(pending.w) : in;
       if constexpr (std::is_same<T, float>::value)
-        F3R_HIP(hipMemcpyAsync(dst, in, sizeof(float) * n, hipMemcpyDeviceToDevice, st()));
+        F3R_HIP(hipMemcpyAsync(dst, src, sizeof(float) * n, hipMemcpyDeviceToDevice, st()));
       else
-        hipLaunchKernelGGL((k_cast2<T, float>), dim3(grid()), dim3(kBlock), 0, st(), (int64_t)n, in, dst);
+        hipLaunchKernelGGL((k_cast2<T, float>), dim3(grid()), dim3(kBlock), 0, st(), (int64_t)n, src, dst);
       ++cap_n;
     }
     if constexpr (std::is_same<T, float>::value) {
-      if (p.variant == 0) {
-        level4_half(in, out, hz);
-        return;
-      }
+      if (p.variant == 0)
+        richardson<half_t, float, half_t, float>(in, out, hz, A16->as<half_t>(), *sh16);
+      else
+        richardson<float, float, double, double>(in, out, nullptr, A64->as<double>(), *sh);
+    } else {
+      richardson<double, double, double, double>(in, out, nullptr, A64->as<double>(), *sh);
     }
-    level4_t<T>(in, out);
   }
 
   // ----------------------------------------------- level 3 and level 2 ---
@@ -1409,6 +1297,7 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
     const int64_t ld = (n + 63) / 64 * 64;
     L.Vbuf = dev_alloc(sizeof(E) * ld * (m + 1));
     L.Zbuf = dev_alloc(sizeof(E) * ld * m);
+    L.wbuf = dev_alloc(sizeof(E) * ld);
     L.H = dev_alloc(sizeof(E) * (m + 1) * m);
     L.cs = dev_alloc(sizeof(E) * m);
     L.sn = dev_alloc(sizeof(E) * m);
@@ -1844,7 +1733,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
         for (int j = 0; j < m; ++j) {
           Cols<float, 4> c{};
           for (int k = 0; k <= j; ++k) c.p[k] = s->L3f.V[k];
-          EpiDots<float, 4> epi{s->L3f.V[j + 1], c, j + 1, s->L3f.Hp() + (int64_t)j * s->L3f.ldh(),
+          EpiDots<float, 4> epi{s->L3f.w(), c, j + 1, s->L3f.Hp() + (int64_t)j * s->L3f.ldh(),
                                 s->template partial<float>(), s->counter(0)};
           if (!s->L3f.Zh.empty()) {
             epi.xs = 1.f / s->range_s;
@@ -1873,8 +1762,9 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
       }
       case 8: {  // the fused Richardson step (residual SpMV + diagonal SDAINV + weighted update), fp16 out
         RichDev *rs = s->rich->as<RichDev>();
-        EpiL4Diag epi{s->hin->as<half_t>(), s->hout->as<half_t>(), s->P->dwz->as<uint32_t>(), &rs->ome[1],
-                      nullptr, nullptr, s->hout2->as<half_t>(), nullptr, 1.f / s->range_s};
+        EpiL4Diag<half_t, float, float> epi{s->hin->as<half_t>(), s->hout->as<half_t>(), diag_wz<half_t>(*s->P),
+                                            &rs->ome[1], nullptr, nullptr, s->hout2->as<half_t>(), nullptr,
+                                            1.f / s->range_s};
         launch_sell<half_t, half_t, float>(s->sh16->K, a16, s->A16->as<half_t>(), s->hout->as<half_t>(), epi,
                                            s->st());
         // values, h gathered, hin / h / (w, z) read per row, h' written
@@ -1882,13 +1772,16 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
         break;
       }
       case 9: {  // the innermost entry: normalise the basis vector, fp16 input, first weighted M application
-        const int64_t nn = s->n;
-        float *in = s->L3f.V[s->L3f.m];
-        hipLaunchKernelGGL(k_l4_entry<true>, dim3(s->grid()), dim3(kBlock), 0, s->st(), nn, in,
-                           (const float *)one->as<float>(), s->range_s, s->hin->as<half_t>(),
-                           s->hout2->as<half_t>(), (const uint32_t *)s->P->dwz->as<uint32_t>(),
-                           (const RichDev *)s->rich->as<RichDev>(), 1);
-        by = (double)s->n * (4 + 4 + 4 + 2 + 2);  // in read and written, (w, z) read, hin and hout written
+        MIo<half_t, float> io;
+        io.raw = s->L3f.w();
+        io.inv = one->as<float>();
+        io.vout = s->L3f.V[s->L3f.m];
+        io.s = s->range_s;
+        io.hin = s->hin->as<half_t>();
+        io.out = s->hout2->as<half_t>();
+        io.w = &s->rich->as<RichDev>()->ome[0];
+        prec_apply_io<half_t, float>(s->P.get(), io, s->st());
+        by = (double)s->n * (4 + 4 + 4 + 2 + 2);  // w read, the column written, (w, z) read, hin and hout written
         break;
       }
     }
