@@ -1144,11 +1144,8 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
           }
           P->bj_lds = lds + 2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>);
           // up to 154 KB of the CU's 160 KB
-          F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, S, R, NW>),
+          F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, typename Acc<S>::type, R, NW>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->bj_lds));
-          if constexpr (std::is_same<S, half_t>::value)
-            F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, float, R, NW>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->bj_lds));
         });
       }
     }
@@ -1180,10 +1177,11 @@ template <class S, class F> static void bj_apply(Prec *P, const MIo<S, F> &io, h
 template <class S> static void ilu_apply_t(Prec *P, const S *in, S *out, hipStream_t st) {
   S *tmp = P->tmp->as<S>();
   if (P->bj_R) {
-    MIo<S, S> io;
+    using F = typename Acc<S>::type;
+    MIo<S, F> io;
     io.in = in;
     io.out = out;
-    bj_apply<S, S>(P, io, st);
+    bj_apply<S, F>(P, io, st);
     return;
   }
   if (P->bj_blocks) {

@@ -57,8 +57,13 @@ template <class S, class F> struct MIo {
   // input: `in`, or the entry from `raw`
   const S *in = nullptr;
   const F *raw = nullptr;
-  const F *inv = nullptr;  // 1/||raw||; null: raw is normalised
-  F *vout = nullptr;       // the normalised vector (with inv; not raw: rows gather raw meanwhile)
+  // block sums of ||raw||^2 left by the Arnoldi step that made it (null: raw
+  // is normalised); every block adds them up itself, the first one also
+  // writes the norm to its place in the Hessenberg column
+  const F *npart = nullptr;
+  int nparts = 0;
+  F *hnorm = nullptr;
+  F *vout = nullptr;       // the normalised vector (with npart; not raw: rows gather raw meanwhile)
   F s = 1;                 // hin = S(raw * inv * s)
   S *hin = nullptr;        // null with S = F: the normalised vector is M's input
   // output: x = M in; out = x, S(x * w) with `w`, or S(fma(w, x, add)) with
@@ -72,11 +77,17 @@ template <class S, class F> struct MIo {
 };
 template <class S, class F> void prec_apply_io(Prec *P, const MIo<S, F> &io, hipStream_t st);
 
-// the entry of one element
+// the entry of one element (constructed by every thread of a block: the
+// block adds up the norm's partial sums)
 template <class S, class F> struct MEntry {
   F iv, s;
   bool has_inv;
-  __device__ explicit MEntry(const MIo<S, F> &io) : iv(io.inv ? *io.inv : (F)1), s(io.s), has_inv(io.inv != nullptr) {}
+  __device__ explicit MEntry(const MIo<S, F> &io) : iv(1), s(io.s), has_inv(io.npart != nullptr) {
+    if (!has_inv) return;
+    const F nv = sqrt(parts_sum<F>(io.npart, io.nparts));
+    if (blockIdx.x == 0 && threadIdx.x == 0) *io.hnorm = nv;
+    iv = (F)1 / nv;
+  }
   __device__ __forceinline__ F norm(F v) const { return has_inv ? v * iv : v; }
   __device__ __forceinline__ S store(F v) const {  // v normalised
     if constexpr (std::is_same<S, F>::value) return v; else return cvt<S>(v * s);

@@ -28,6 +28,18 @@
 
 namespace f3r {
 
+// Up to this many block sums per dot, the CGS update's blocks add the dots up
+// themselves (at 262 K rows 1024 sums of 4 dots, 16 KB per block from L2,
+// against a finishing launch of 4.2 us); beyond, k_dots_finish does it (8192
+// sums at 2 M rows would be 128 KB for each of 2048 blocks).
+constexpr int kDirectDots = 1024;
+// where the CGS update leaves its block sums in the reduction scratch, clear
+// of the dots' sums that its blocks read meanwhile (at most 16 per block of
+// the largest reduction grid)
+constexpr int64_t kNormParts = (int64_t)1 << 19;
+static_assert(16 * (int64_t)kMaxReduceGrid <= kNormParts && kNormParts + kMaxReduceGrid <= Reducer::kPartialDoubles,
+              "the two kinds of block sums fit the scratch side by side");
+
 // true when p is aligned to 4 elements (the vectorised kernels need it)
 template <class T> inline bool aligned4(const T *p) { return ((uintptr_t)p % (4 * sizeof(T))) == 0; }
 
@@ -183,21 +195,57 @@ template <class T> struct EpiResidNorm {
   }
 };
 
-// V_{j+1} -= V H(j)[0..j] (MULMV order: V_0 h_0, then fused adds), ||V_{j+1}||,
-// then the last block: H(j, j+1), 1/h, Givens, |e_{j+1}| for the host.
+// w -= V H(j)[0..j] (MULMV order: V_0 h_0, then fused adds) and the block
+// sums of ||w||^2 into npart[block].  Nothing waits for the grid here: the
+// entry that reads w next adds the block sums up itself, and the level's
+// solution does the Givens rotations of all its columns.  (Finished in this
+// kernel by the last block to arrive, the norm and the rotation took 4 us of
+// its 6.6 at 14 K rows, and of its 11 at 2 M.)
+// dG > 0: H(j)[0..j] from the dG block sums of each dot, dpart[k * dG + b],
+// which every block adds up itself, the first one also writing Hcol; dG = 0:
+// Hcol holds them.
 // VEC: every pointer is 4-element aligned; each lane then takes 4
 // consecutive rows per step with 16-byte (fp32) loads and stores.
 // store = 0: the updated vector is not written back (the last basis vector
 // of an inner level, which nothing reads), only its norm is taken
 template <class T, int NV, bool VEC = false>
 __global__ __launch_bounds__(kBlock) void k_cgs_update(int64_t n, T *__restrict__ w, Cols<T, NV> cols,
-                                                       int ncols, T *Hcol, T *cs, T *sn, T *e, int j,
-                                                       int e0_one, T *inv, double *status, T *partial,
-                                                       unsigned *counter, int store) {
-  __shared__ T lds[kWavesPerBlock];
+                                                       int ncols, T *Hcol, const T *__restrict__ dpart, int dG,
+                                                       T *__restrict__ npart, int store) {
+  __shared__ T lds[NV * kWavesPerBlock];
   T h[NV];
+  if (dG > 0) {
+    constexpr int kPer = kDirectDots / kBlock;  // every load in flight at once
+    T t[NV][kPer];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) h[k] = k < ncols ? Hcol[k] : (T)0;
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) {
+        const int b = threadIdx.x + q * kBlock;
+        t[k][q] = k < ncols && b < dG ? dpart[(int64_t)k * dG + b] : (T)0;
+      }
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      T v = t[k][0];
+#pragma unroll
+      for (int q = 1; q < kPer; ++q) v += t[k][q];
+      v = wave_sum(v);
+      if (lane == 0) lds[k * kWavesPerBlock + wid] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      h[k] = lds[k * kWavesPerBlock];
+#pragma unroll
+      for (int q = 1; q < kWavesPerBlock; ++q) h[k] += lds[k * kWavesPerBlock + q];
+      if (blockIdx.x == 0 && threadIdx.x == 0 && k < ncols) Hcol[k] = h[k];
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) h[k] = k < ncols ? Hcol[k] : (T)0;
+  }
   T v[1] = {0};
   const int64_t gid = blockIdx.x * (int64_t)kBlock + threadIdx.x, gstride = (int64_t)gridDim.x * kBlock;
   int64_t i0 = 0;
@@ -232,15 +280,53 @@ __global__ __launch_bounds__(kBlock) void k_cgs_update(int64_t n, T *__restrict_
     if (store) w[i] = wn;
     v[0] = fma_<T>(wn, wn, v[0]);
   }
-  // the grid's sum of ||w||^2 in the last block (one wave of blocks: the
-  // arrivals cost less than a one-block finishing launch, 0.12 ms per solve
-  // at 128^3)
-  if (grid_sum<T, 1>(v, partial, counter, lds) && threadIdx.x == 0) {
-    T nv = (T)sqrt(v[0]);
-    Hcol[j + 1] = nv;
-    *inv = (T)1 / nv;
-    givens_step<T>(Hcol, cs, sn, e, j, e0_one != 0);
-    if (status) *status = fabs((double)e[j + 1]);
+  block_sum<T, 1>(v, lds);
+  if (threadIdx.x == 0) npart[blockIdx.x] = v[0];
+}
+
+// The small least-squares problem of an inner level by one thread: Givens
+// rotations of the m columns of H (H(j) at H + j * (m + 1), e_0 = 1;
+// Blas1::full_grot / final_grot, gmres.hpp:14-38) and the back substitution
+// (Blas1::trsv, gmres.hpp:41-53).  Up to 8 columns in registers.
+template <class T, int NV> __device__ void level_solve(T *H, int m, T *y) {
+  if constexpr (NV <= 8) {
+    T R[NV][NV], cs[NV], sn[NV], e[NV], yr[NV];
+    T en = 1;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+      if (j < m) {
+        T c[NV + 1];
+#pragma unroll
+        for (int i = 0; i <= j + 1; ++i) c[i] = H[j * (m + 1) + i];
+#pragma unroll
+        for (int i = 0; i < j; ++i) {
+          const T t = c[i], h1 = c[i + 1];
+          c[i] = fma_<T>(cs[i], t, sn[i] * h1);
+          c[i + 1] = fma_<T>(-sn[i], t, cs[i] * h1);
+        }
+        const T t = (T)sqrt(fma_<T>(c[j], c[j], c[j + 1] * c[j + 1]));
+        cs[j] = c[j] / t;
+        sn[j] = c[j + 1] / t;
+        c[j] = t;
+#pragma unroll
+        for (int i = 0; i <= j; ++i) R[j][i] = c[i];
+        e[j] = cs[j] * en;
+        en = -sn[j] * en;
+      }
+#pragma unroll
+    for (int i = NV - 1; i >= 0; --i)
+      if (i < m) {
+        T t = e[i];
+#pragma unroll
+        for (int q = NV - 1; q > i; --q)
+          if (q < m) t = fma_<T>(-R[q][i], yr[q], t);
+        yr[i] = t / R[i][i];
+        y[i] = yr[i];
+      }
+  } else {
+    __shared__ T cs[NV], sn[NV], e[NV + 1];
+    for (int j = 0; j < m; ++j) givens_step<T>(H + j * (m + 1), cs, sn, e, j, true);
+    hess_solve<T>(H, m + 1, e, y, m);
   }
 }
 
@@ -345,14 +431,22 @@ __global__ void k_vscale(int64_t n, T *__restrict__ v, const T *__restrict__ inv
     v[i] *= a;
 }
 
-// out = Z y (with_init) of an inner level; every block solves the small
-// triangular system itself (j <= NV).  Columns of type ZT hold z * s (fp16
-// storage, s a power of two): z = column * zs is exact.
+// out = Z y (with_init) of an inner level of j <= NV steps; every block
+// solves the small least-squares problem itself (the last column's norm from
+// its block sums).  Columns of type ZT hold z * s (fp16 storage, s a power of
+// two): z = column * zs is exact.
 template <class T, class TO, int NV, bool VEC = false, class ZT = T>
-__global__ __launch_bounds__(kBlock) void k_solution(int64_t n, Cols<ZT, NV> Z, int j, const T *H, int ldh,
-                                                     const T *e, TO *__restrict__ out, T zs) {
-  __shared__ T y[NV];
-  if (threadIdx.x == 0) hess_solve<T>(H, ldh, e, y, j);
+__global__ __launch_bounds__(kBlock) void k_solution(int64_t n, Cols<ZT, NV> Z, int j, const T *__restrict__ H,
+                                                     const T *__restrict__ npart, int nparts, TO *__restrict__ out,
+                                                     T zs) {
+  __shared__ T y[NV], Hs[NV * (NV + 1)];
+  const T last = parts_sum<T>(npart, nparts);
+  for (int i = threadIdx.x; i < j * (j + 1); i += kBlock) Hs[i] = H[i];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    Hs[j * (j + 1) - 1] = (T)sqrt(last);
+    level_solve<T, NV>(Hs, j, y);
+  }
   __syncthreads();
   const int64_t gid = blockIdx.x * (int64_t)kBlock + threadIdx.x, gstride = (int64_t)gridDim.x * kBlock;
   int64_t i0 = 0;
@@ -615,7 +709,7 @@ __global__ __launch_bounds__(kBlock) void k_g_combine(int64_t n, const S *__rest
 // ------------------------------------------------------------ the solver ---
 template <class T> struct InnerLevel {
   int m = 0;
-  DevPtr Vbuf, Zbuf, H, cs, sn, e, inv;
+  DevPtr Vbuf, Zbuf, H;  // H(j) at H + j * ldh(): dots and norms, before any rotation
   std::vector<T *> V, Z;  // column pointers; V[0] aliases the level's input
   // w = A z_j of the running step: V[j + 1] before its normalisation, which
   // the next innermost entry writes as it reads w (rows gather w meanwhile)
@@ -674,15 +768,18 @@ struct Solver {
   std::vector<double> hist;
   std::map<uint64_t, hipGraphExec_t> graphs;
   std::vector<hipGraph_t> graph_src;
-  // the last Arnoldi step's w and 1/||w||, still to be written to its basis
-  // column: the next innermost entry (the column's first reader) does it
+  // the last Arnoldi step's w and the place of its norm, still to be written
+  // to its basis column: the next innermost entry (the column's first reader)
+  // does it
   struct Pending {
-    const void *w = nullptr, *inv = nullptr;
-    void *col = nullptr;
+    const void *w = nullptr;
+    void *hnorm = nullptr, *col = nullptr;
   } pending;
   bool layouts_on_device = false;  // the matrix layouts were built on the device
   int red_grid = 1;   // capped grid of the outer level's strided reductions
   int dots_grid = 1;  // blocks of the streaming kernels with a grid reduction
+  int dots_parts = 0;    // block sums per dot of the last inner SpMV + dots (0: added up in H)
+  int update_parts = 0;  // block sums of the norm of the last inner CGS update
   int spmv_grid = 0;  // blocks of the SpMV kernels with a fused grid reduction (0 = one row per thread)
   // capture of level-4 inputs (fp32, internal row order): every cap_every-th
   // call until cap_max vectors are held; level 2 runs eagerly meanwhile
@@ -699,6 +796,12 @@ struct Solver {
   int grid() const {
     int64_t g = (n + kBlock - 1) / kBlock;
     return (int)std::min<int64_t>(g, (int64_t)ctx->num_cu * 16);
+  }
+  // blocks of a streaming kernel: one row, or with 4-element accesses four,
+  // per lane, capped
+  int vgrid(bool vec) const {
+    const int64_t per = vec ? 4 * kBlock : kBlock;
+    return (int)std::min<int64_t>((n + per - 1) / per, (int64_t)ctx->num_cu * 16);
   }
   SellArgs args() const { return sell_args(*sh, false); }
   // the layout of the matrix with value type V (the fp16 copy may differ in K)
@@ -729,20 +832,26 @@ struct Solver {
     } else {
       launch_sell<V, T, T>(shv<V>().K, argsv<V>(), val, L.Z[j], epi, st(), spmv_grid);
     }
-    // block partials the SpMV + dots kernel wrote per dot: its grid
-    hipLaunchKernelGGL(k_dots_finish<T>, dim3(j + 1), dim3(1024), 0, st(), (const T *)partial<T>(),
-                       sell_blocks(argsv<V>(), spmv_grid), L.Hp() + (int64_t)j * L.ldh());
+    // block sums the SpMV + dots kernel wrote per dot: its grid
+    const int G = sell_blocks(argsv<V>(), spmv_grid);
+    if (G > kDirectDots)
+      hipLaunchKernelGGL(k_dots_finish<T>, dim3(j + 1), dim3(1024), 0, st(), (const T *)partial<T>(), G,
+                         L.Hp() + (int64_t)j * L.ldh());
+    dots_parts = G > kDirectDots ? 0 : G;
   }
+  template <class T> T *norm_parts() const { return partial<T>() + kNormParts; }
   template <class T, int NV> void cgs_update(InnerLevel<T> &L, int j) {
     Cols<T, NV> c{};
     for (int k = 0; k <= j; ++k) c.p[k] = L.V[k];
     bool vec = true;
     for (int k = 0; k <= j; ++k) vec = vec && aligned4(L.V[k]);
     auto kern = vec ? k_cgs_update<T, NV, true> : k_cgs_update<T, NV, false>;
-    hipLaunchKernelGGL(kern, dim3(dots_grid), dim3(kBlock), 0, st(), (int64_t)n,
-                       L.w(), c, j + 1, L.Hp() + (int64_t)j * L.ldh(), L.cs->template as<T>(),
-                       L.sn->template as<T>(), L.e->template as<T>(), j, 1, L.inv->template as<T>(),
-                       (double *)nullptr, partial<T>(), counter(1), j + 1 < L.m ? 1 : 0);
+    // no block without rows (4 per lane and step with aligned columns)
+    const int64_t per = vec ? 4 * kBlock : kBlock;
+    update_parts = (int)std::min<int64_t>((n + per - 1) / per, dots_grid);
+    hipLaunchKernelGGL(kern, dim3(update_parts), dim3(kBlock), 0, st(), (int64_t)n, L.w(), c, j + 1,
+                       L.Hp() + (int64_t)j * L.ldh(), (const T *)partial<T>(), dots_parts, norm_parts<T>(),
+                       j + 1 < L.m ? 1 : 0);
   }
   template <class T, class V> void arnoldi(InnerLevel<T> &L, const V *val, int j) {
     if (j + 1 <= 4) {
@@ -759,7 +868,7 @@ struct Solver {
     // output is Z y).  The first reader of the others is the next innermost
     // entry (level 3's next step, or level 3's start when this is level 2),
     // which normalises w into its column in passing.
-    if (j + 1 < L.m) pending = {L.w(), L.inv->p, L.V[j + 1]};
+    if (j + 1 < L.m) pending = {L.w(), L.Hp() + (int64_t)j * L.ldh() + j + 1, L.V[j + 1]};
   }
   template <class T, class TO> void solution(InnerLevel<T> &L, TO *out) {
     const int j = L.m;
@@ -771,8 +880,8 @@ struct Solver {
         bool vec = aligned4(out);
         for (int k = 0; k < j; ++k) vec = vec && aligned4(L.Zh[k]);
         auto kern = vec ? k_solution<T, TO, NV, true, half_t> : k_solution<T, TO, NV, false, half_t>;
-        hipLaunchKernelGGL(kern, dim3(grid()), dim3(kBlock), 0, st(), (int64_t)n, c, j, (const T *)L.Hp(),
-                           L.ldh(), (const T *)L.e->template as<T>(), out, (T)(1.0 / range_s));
+        hipLaunchKernelGGL(kern, dim3(vgrid(vec)), dim3(kBlock), 0, st(), (int64_t)n, c, j, (const T *)L.Hp(),
+                           (const T *)norm_parts<T>(), update_parts, out, (T)(1.0 / range_s));
         return;
       }
       Cols<T, NV> c{};
@@ -780,8 +889,8 @@ struct Solver {
       bool vec = aligned4(out);
       for (int k = 0; k < j; ++k) vec = vec && aligned4(L.Z[k]);
       auto kern = vec ? k_solution<T, TO, NV, true> : k_solution<T, TO, NV, false>;
-      hipLaunchKernelGGL(kern, dim3(grid()), dim3(kBlock), 0, st(), (int64_t)n, c, j,
-                         (const T *)L.Hp(), L.ldh(), (const T *)L.e->template as<T>(), out, (T)1);
+      hipLaunchKernelGGL(kern, dim3(vgrid(vec)), dim3(kBlock), 0, st(), (int64_t)n, c, j, (const T *)L.Hp(),
+                         (const T *)norm_parts<T>(), update_parts, out, (T)1);
     };
     if (j <= 4) go(std::integral_constant<int, 4>());
     else if (j <= 8) go(std::integral_constant<int, 8>());
@@ -815,7 +924,9 @@ struct Solver {
     io.raw = in;
     if (pending.col == in) {
       io.raw = static_cast<const F *>(pending.w);
-      io.inv = static_cast<const F *>(pending.inv);
+      io.npart = norm_parts<F>();
+      io.nparts = update_parts;
+      io.hnorm = static_cast<F *>(pending.hnorm);
       io.vout = const_cast<F *>(in);
     }
     pending = Pending();
@@ -1299,10 +1410,6 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
     L.Zbuf = dev_alloc(sizeof(E) * ld * m);
     L.wbuf = dev_alloc(sizeof(E) * ld);
     L.H = dev_alloc(sizeof(E) * (m + 1) * m);
-    L.cs = dev_alloc(sizeof(E) * m);
-    L.sn = dev_alloc(sizeof(E) * m);
-    L.e = dev_alloc(sizeof(E) * (m + 1));
-    L.inv = dev_alloc(sizeof(E) * 4);
     L.V.resize(m + 1);
     L.Z.resize(m);
     for (int k = 0; k <= m; ++k) L.V[k] = L.Vbuf->template as<E>() + (int64_t)k * ld;
@@ -1691,12 +1798,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
   const int per = (which == 6 || which == 7) ? s->L3f.m : 1;
   const bool diag = s->P->kind == 0 && s->P->diag;
   F3R_CHECK(which < 8 || diag, F3R_ERR_UNSUPPORTED, "time_kernel: the fused Richardson kernels need diagonal SDAINV");
-  DevPtr one;  // 1/||w|| = 1 for the entry kernel's in-place normalisation
-  if (which == 9) {
-    one = dev_alloc(sizeof(float));
-    const float f1 = 1.f;
-    F3R_HIP(hipMemcpyAsync(one->p, &f1, sizeof(float), hipMemcpyHostToDevice, s->st()));
-  }
+  if (which == 9) s->cgs_update<float, 4>(s->L3f, s->L3f.m - 1);  // the block sums of the norm that the entry reads
   auto launch = [&]() {
     switch (which) {
       case 0:  // fp16 values, fp16 x and y (the metric's fp16 SpMV)
@@ -1723,7 +1825,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
         s->template spmv_dots<float, half_t, 4>(s->L3f, s->A16->as<half_t>(), s->L3f.m - 1);
         by = s->sh16->algo_bytes(2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * s->L3f.m;
         break;
-      case 5:  // level-3 CGS update + norm + Givens of that step (the last: w is not stored)
+      case 5:  // level-3 CGS update + norm of that step (the last: w is not stored)
         s->template cgs_update<float, 4>(s->L3f, s->L3f.m - 1);
         by = 4.0 * s->n * (s->L3f.m + 1);
         break;
@@ -1749,7 +1851,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
         by /= m;
         break;
       }
-      case 7: {  // the solve's mix of CGS update + norm + Givens launches, steps j = 0 .. m3 - 1
+      case 7: {  // the solve's mix of CGS update + norm launches, steps j = 0 .. m3 - 1
         const int m = s->L3f.m;
         by = 0;
         for (int j = 0; j < m; ++j) {
@@ -1774,7 +1876,9 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
       case 9: {  // the innermost entry: normalise the basis vector, fp16 input, first weighted M application
         MIo<half_t, float> io;
         io.raw = s->L3f.w();
-        io.inv = one->as<float>();
+        io.npart = s->norm_parts<float>();
+        io.nparts = s->update_parts;
+        io.hnorm = s->L3f.Hp() + (int64_t)s->L3f.m * s->L3f.ldh() - 1;
         io.vout = s->L3f.V[s->L3f.m];
         io.s = s->range_s;
         io.hin = s->hin->as<half_t>();
