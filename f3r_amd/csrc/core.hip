@@ -351,7 +351,13 @@ __global__ __launch_bounds__(kBlock) void k_m_diag(int64_t n, DiagWZ<S> d, MIo<S
       }
       if (io.vout) st4(io.vout + 4 * q, v);
       if (io.hin) st4(io.hin + 4 * q, h);
-      st4(io.out + 4 * q, o);
+      if (io.outf) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v.v[c] = (F)to_acc(o.v[c]) * io.inv_s;
+        st4(io.outf + 4 * q, v);
+      } else {
+        st4(io.out + 4 * q, o);
+      }
     }
     i0 = 4 * n4;
   }
@@ -360,7 +366,7 @@ __global__ __launch_bounds__(kBlock) void k_m_diag(int64_t n, DiagWZ<S> d, MIo<S
     const S h = en.store(v);
     if (io.vout) io.vout[i] = v;
     if (io.hin) io.hin[i] = h;
-    io.out[i] = mo.value(diag_apply<S>(d.at(i), h), S(0));
+    mo.put(i, diag_apply<S>(d.at(i), h), S(0));
   }
 }
 
@@ -1239,13 +1245,21 @@ void prec_apply_raw(Prec *P, const void *in, void *out, hipStream_t st) {
 // true when p (or a null pointer) is aligned to 4 elements
 template <class T> static bool align4(const T *p) { return ((uintptr_t)p % (4 * sizeof(T))) == 0; }
 
+template <class S, class F>
+void prec_entry(const MIo<S, F> &io, int64_t n, S *h, int num_cu, hipStream_t st) {
+  hipLaunchKernelGGL((k_m_entry<S, F>), dim3(grid_for(n, num_cu)), dim3(kBlock), 0, st, n, io, h);
+  F3R_HIP(hipGetLastError());
+}
+template void prec_entry<half_t, float>(const MIo<half_t, float> &, int64_t, half_t *, int, hipStream_t);
+template void prec_entry<float, float>(const MIo<float, float> &, int64_t, float *, int, hipStream_t);
+
 template <class S, class F> void prec_apply_io(Prec *P, const MIo<S, F> &io, hipStream_t st) {
   using ACC = typename Acc<S>::type;
   const int64_t n = P->n;
   const dim3 g(grid_for(n, P->ctx->num_cu)), b(kBlock);
-  if (P->kind == 0 && P->diag && io.raw && !io.add && !io.outf) {
+  if (P->kind == 0 && P->diag && io.raw && !io.add) {
     const DiagWZ<S> d = diag_wz<S>(*P);
-    bool vec = align4(io.raw) && align4(io.vout) && align4(io.hin) && align4(io.out);
+    bool vec = align4(io.raw) && align4(io.vout) && align4(io.hin) && align4(io.out) && align4(io.outf);
     if constexpr (std::is_same<S, half_t>::value) vec = vec && align4(d.wz);
     else vec = vec && align4(d.w) && align4(d.z);
     auto kern = vec ? k_m_diag<S, F, true> : k_m_diag<S, F, false>;

@@ -39,6 +39,8 @@ struct Prec {
   struct BjData {
     DevPtr rec, seg, bat, cnt;
   } bj[2];
+  // its kernels take the entry themselves (no vector for its result needed)
+  bool has_fused_entry() const { return kind == 0 || bj_R != 0; }
 };
 // LDS the fused block-Jacobi kernel may take for a block's vector
 constexpr size_t kBjLdsBytes = 64 * 1024;
@@ -76,6 +78,9 @@ template <class S, class F> struct MIo {
   S *scratch = nullptr;  // a vector of S for kinds of M without fused kernels (with add)
 };
 template <class S, class F> void prec_apply_io(Prec *P, const MIo<S, F> &io, hipStream_t st);
+// the entry alone: h = S(raw * inv * s) where h is not null, and vout
+template <class S, class F>
+void prec_entry(const MIo<S, F> &io, int64_t n, S *h, int num_cu, hipStream_t st);
 
 // the entry of one element (constructed by every thread of a block: the
 // block adds up the norm's partial sums)

@@ -434,11 +434,11 @@ __global__ void k_vscale(int64_t n, T *__restrict__ v, const T *__restrict__ inv
 // out = Z y (with_init) of an inner level of j <= NV steps; every block
 // solves the small least-squares problem itself (the last column's norm from
 // its block sums).  Columns of type ZT hold z * s (fp16 storage, s a power of
-// two): z = column * zs is exact.
+// two): z = column * zs is exact.  os: factor of the output.
 template <class T, class TO, int NV, bool VEC = false, class ZT = T>
 __global__ __launch_bounds__(kBlock) void k_solution(int64_t n, Cols<ZT, NV> Z, int j, const T *__restrict__ H,
                                                      const T *__restrict__ npart, int nparts, TO *__restrict__ out,
-                                                     T zs) {
+                                                     T zs, T os) {
   __shared__ T y[NV], Hs[NV * (NV + 1)];
   const T last = parts_sum<T>(npart, nparts);
   for (int i = threadIdx.x; i < j * (j + 1); i += kBlock) Hs[i] = H[i];
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(kBlock) void k_solution(int64_t n, Cols<ZT, NV> Z, 
 #pragma unroll
         for (int k = 1; k < NV; ++k)
           if (k < j) r = fma_<T>((T)to_acc(zk[k].v[c]) * zs, y[k], r);
-        o.v[c] = cvt<TO>(r);
+        o.v[c] = cvt<TO>(r * os);
       }
       st4(out + 4 * q, o);
     }
@@ -475,7 +475,7 @@ __global__ __launch_bounds__(kBlock) void k_solution(int64_t n, Cols<ZT, NV> Z, 
 #pragma unroll
     for (int k = 1; k < NV; ++k)
       if (k < j) r = fma_<T>((T)to_acc(Z.p[k][i]) * zs, y[k], r);
-    out[i] = cvt<TO>(r);
+    out[i] = cvt<TO>(r * os);
   }
 }
 
@@ -746,7 +746,7 @@ struct Solver {
     int mat = F3R_F32;    // the level's matrix values: F3R_F32 or F3R_F16
     float s = 1.f;        // storage scale (stored = s * value), fp16 levels
     int64_t ld = 0;
-    DevPtr V, Z, H, cs, sn, e, inv;
+    DevPtr V, Z, H, cs, sn, e, inv, w;  // w: A z_j before its normalisation (fp32 levels)
     template <class S> S *Vc(int k) const { return V->as<S>() + (int64_t)k * ld; }
     template <class S> S *Zc(int k) const { return Z->as<S>() + (int64_t)k * ld; }
   };
@@ -833,25 +833,28 @@ struct Solver {
       launch_sell<V, T, T>(shv<V>().K, argsv<V>(), val, L.Z[j], epi, st(), spmv_grid);
     }
     // block sums the SpMV + dots kernel wrote per dot: its grid
-    const int G = sell_blocks(argsv<V>(), spmv_grid);
+    finish_dots<T>(sell_blocks(argsv<V>(), spmv_grid), j, L.Hp() + (int64_t)j * L.ldh());
+  }
+  template <class T> void finish_dots(int G, int j, T *Hcol) {
     if (G > kDirectDots)
-      hipLaunchKernelGGL(k_dots_finish<T>, dim3(j + 1), dim3(1024), 0, st(), (const T *)partial<T>(), G,
-                         L.Hp() + (int64_t)j * L.ldh());
+      hipLaunchKernelGGL(k_dots_finish<T>, dim3(j + 1), dim3(1024), 0, st(), (const T *)partial<T>(), G, Hcol);
     dots_parts = G > kDirectDots ? 0 : G;
   }
   template <class T> T *norm_parts() const { return partial<T>() + kNormParts; }
   template <class T, int NV> void cgs_update(InnerLevel<T> &L, int j) {
     Cols<T, NV> c{};
     for (int k = 0; k <= j; ++k) c.p[k] = L.V[k];
-    bool vec = true;
-    for (int k = 0; k <= j; ++k) vec = vec && aligned4(L.V[k]);
+    update_launch<T, NV>(L.w(), c, j, L.Hp() + (int64_t)j * L.ldh(), j + 1 < L.m);
+  }
+  template <class T, int NV> void update_launch(T *w, const Cols<T, NV> &c, int j, T *Hcol, bool store) {
+    bool vec = aligned4(w);
+    for (int k = 0; k <= j; ++k) vec = vec && aligned4(c.p[k]);
     auto kern = vec ? k_cgs_update<T, NV, true> : k_cgs_update<T, NV, false>;
     // no block without rows (4 per lane and step with aligned columns)
     const int64_t per = vec ? 4 * kBlock : kBlock;
     update_parts = (int)std::min<int64_t>((n + per - 1) / per, dots_grid);
-    hipLaunchKernelGGL(kern, dim3(update_parts), dim3(kBlock), 0, st(), (int64_t)n, L.w(), c, j + 1,
-                       L.Hp() + (int64_t)j * L.ldh(), (const T *)partial<T>(), dots_parts, norm_parts<T>(),
-                       j + 1 < L.m ? 1 : 0);
+    hipLaunchKernelGGL(kern, dim3(update_parts), dim3(kBlock), 0, st(), (int64_t)n, w, c, j + 1, Hcol,
+                       (const T *)partial<T>(), dots_parts, norm_parts<T>(), store ? 1 : 0);
   }
   template <class T, class V> void arnoldi(InnerLevel<T> &L, const V *val, int j) {
     if (j + 1 <= 4) {
@@ -881,7 +884,7 @@ struct Solver {
         for (int k = 0; k < j; ++k) vec = vec && aligned4(L.Zh[k]);
         auto kern = vec ? k_solution<T, TO, NV, true, half_t> : k_solution<T, TO, NV, false, half_t>;
         hipLaunchKernelGGL(kern, dim3(vgrid(vec)), dim3(kBlock), 0, st(), (int64_t)n, c, j, (const T *)L.Hp(),
-                           (const T *)norm_parts<T>(), update_parts, out, (T)(1.0 / range_s));
+                           (const T *)norm_parts<T>(), update_parts, out, (T)(1.0 / range_s), (T)1);
         return;
       }
       Cols<T, NV> c{};
@@ -890,11 +893,27 @@ struct Solver {
       for (int k = 0; k < j; ++k) vec = vec && aligned4(L.Z[k]);
       auto kern = vec ? k_solution<T, TO, NV, true> : k_solution<T, TO, NV, false>;
       hipLaunchKernelGGL(kern, dim3(vgrid(vec)), dim3(kBlock), 0, st(), (int64_t)n, c, j, (const T *)L.Hp(),
-                         (const T *)norm_parts<T>(), update_parts, out, (T)1);
+                         (const T *)norm_parts<T>(), update_parts, out, (T)1, (T)1);
     };
     if (j <= 4) go(std::integral_constant<int, 4>());
     else if (j <= 8) go(std::integral_constant<int, 8>());
     else go(std::integral_constant<int, 16>());
+  }
+
+  // the input half of an entry from the basis column `in`: the column, or the
+  // pending w that becomes it
+  template <class S, class F> MIo<S, F> entry_io(const F *in) {
+    MIo<S, F> io;
+    io.raw = in;
+    if (pending.col == in) {
+      io.raw = static_cast<const F *>(pending.w);
+      io.npart = norm_parts<F>();
+      io.nparts = update_parts;
+      io.hnorm = static_cast<F *>(pending.hnorm);
+      io.vout = const_cast<F *>(in);
+      pending = Pending();
+    }
+    return io;
   }
 
   // --------------------------------------------------------- level 4 ---
@@ -920,16 +939,7 @@ struct Solver {
     if (p.m4 == 1 && hz) ho = hz;  // no Richardson step
     // entry (normalising `in` first when the Arnoldi step that made it did
     // not), M, and outside probe calls the first weight
-    MIo<S, F> io;
-    io.raw = in;
-    if (pending.col == in) {
-      io.raw = static_cast<const F *>(pending.w);
-      io.npart = norm_parts<F>();
-      io.nparts = update_parts;
-      io.hnorm = static_cast<F *>(pending.hnorm);
-      io.vout = const_cast<F *>(in);
-    }
-    pending = Pending();
+    MIo<S, F> io = entry_io<S, F>(in);
     io.s = (F)range_s;
     if constexpr (kSame) hi = const_cast<F *>(in);
     else io.hin = hi;
@@ -1079,12 +1089,27 @@ struct Solver {
   }
 
   // ------------------------------------ generic levels (depth ablations) ---
+  // w and its norm written to the basis column they belong to, where the
+  // column's first reader does not do it itself
+  void normalise_pending() {
+    if (!pending.col) return;
+    MIo<float, float> io = entry_io<float, float>(static_cast<const float *>(pending.col));
+    prec_entry<float, float>(io, n, nullptr, ctx->num_cu, st());
+  }
   // M applied directly to a vector of the caller's storage SI, scaled by s_in
   template <class SI> void mdirect(const SI *in, SI *out, float s_in) {
     ++cnt;
     ++calls;
     if constexpr (std::is_same<SI, half_t>::value) {
       prec_apply_raw(P.get(), in, out, st());  // M is linear: the scale carries through
+    } else if constexpr (std::is_same<SI, float>::value) {
+      MIo<half_t, float> io = entry_io<half_t, float>(in);
+      io.s = (float)((double)range_s / s_in);
+      io.outf = out;
+      io.inv_s = (float)((double)s_in / range_s);
+      if (!P->has_fused_entry()) io.hin = hin->as<half_t>();
+      io.out = hout->as<half_t>();  // M's own result, where it needs one
+      prec_apply_io<half_t, float>(P.get(), io, st());
     } else {
       half_t *hi = hin->as<half_t>(), *ho = hout->as<half_t>();
       hipLaunchKernelGGL((k_g_entry<SI, half_t>), dim3(grid()), dim3(kBlock), 0, st(), (int64_t)n, in, hi,
@@ -1103,6 +1128,7 @@ struct Solver {
     const int64_t nn = n;
     const dim3 g(grid()), b(kBlock);
     const double s_op = op_dtype == F3R_F16 ? (double)range_s : 1.0;
+    if constexpr (std::is_same<SI, float>::value) normalise_pending();
     auto to_op = [&](auto tag) {
       using T = decltype(tag);
       hipLaunchKernelGGL((k_g_entry<SI, T>), g, b, 0, st(), nn, in, op_in->as<T>(), s_op / s_in);
@@ -1143,7 +1169,11 @@ struct Solver {
       glevel_t<SI, float>(l, in, out, s_in);
   }
   // FGMRES(m) with normalize = false (solver/gmres2.hpp:84-145): V_0 = in,
-  // e_0 = 1; CGS with the dots, the update and the norm as separate passes
+  // e_0 = 1; classical Gram-Schmidt.  fp32 levels of up to 16 steps run as the
+  // F3R levels do: the dots in the SpMV, block sums of dots and norms added up
+  // by their readers, w normalised by its first reader and the rotations in
+  // the combination, 4 launches a step under M in place of 11 (each 2 to 6 us
+  // at 118 K rows).  fp16 levels, and more than 16 columns, keep their passes.
   template <class SI, class S> void glevel_t(int l, const SI *in, SI *out, float s_in) {
     GLevel &L = glev[l];
     const int64_t nn = n;
@@ -1151,17 +1181,35 @@ struct Solver {
     const float sc = 1.f / (L.s * L.s);
     const int G = dots_grid;
     float *part = partial<float>();
-    hipLaunchKernelGGL((k_g_entry<SI, S>), g, b, 0, st(), nn, in, L.Vc<S>(0), (double)L.s / s_in);
+    constexpr bool kF32 = std::is_same<S, float>::value;
+    const bool fused = kF32 && L.m <= 16;
+    if constexpr (std::is_same<SI, float>::value) {
+      if (pending.col == in) {
+        MIo<S, float> io = entry_io<S, float>(in);
+        io.s = L.s / s_in;
+        prec_entry<S, float>(io, nn, L.Vc<S>(0), ctx->num_cu, st());
+      } else {
+        hipLaunchKernelGGL((k_g_entry<SI, S>), g, b, 0, st(), nn, in, L.Vc<S>(0), (double)L.s / s_in);
+      }
+    } else {
+      hipLaunchKernelGGL((k_g_entry<SI, S>), g, b, 0, st(), nn, in, L.Vc<S>(0), (double)L.s / s_in);
+    }
     for (int j = 0; j < L.m; ++j) {
       glevel<S>(l + 1, L.Vc<S>(j), L.Zc<S>(j), L.s);
+      const int ncols = j + 1;
+      float *Hcol = L.H->as<float>() + (int64_t)j * (L.m + 1);
+      if constexpr (kF32) {
+        if (fused) {
+          gstep(L, j, Hcol);
+          continue;
+        }
+      }
       if (L.mat == F3R_F16)
         launch_sell<half_t, S, float>(sh16->K, argsv<half_t>(), A16->as<half_t>(), L.Zc<S>(j),
                                       EpiStore<S, float>{L.Vc<S>(j + 1), nullptr}, st());
       else
         launch_sell<float, S, float>(sh->K, args(), A32->as<float>(), L.Zc<S>(j),
                                      EpiStore<S, float>{L.Vc<S>(j + 1), nullptr}, st());
-      const int ncols = j + 1;
-      float *Hcol = L.H->as<float>() + (int64_t)j * (L.m + 1);
       hipLaunchKernelGGL(k_g_mdot<S>, dim3(G, (ncols + 15) / 16), b, 0, st(), nn, (const S *)L.Vc<S>(j + 1),
                          (const S *)L.Vc<S>(0), L.ld, ncols, part);
       hipLaunchKernelGGL(k_g_dots_finish, dim3(ncols), b, 0, st(), (const float *)part, G, Hcol, sc);
@@ -1172,9 +1220,51 @@ struct Solver {
                          (double *)nullptr);
       hipLaunchKernelGGL(k_g_vscale<S>, g, b, 0, st(), nn, L.Vc<S>(j + 1), (const float *)L.inv->as<float>());
     }
+    if constexpr (kF32) {
+      if (fused) {
+        gsolution<SI>(L, out, s_in);
+        return;
+      }
+    }
     hipLaunchKernelGGL((k_g_combine<S, SI>), g, b, 0, st(), nn, (const S *)L.Zc<S>(0), L.ld, L.m,
                        (const float *)L.H->as<float>(), L.m + 1, (const float *)L.e->as<float>(), out,
                        s_in / L.s);
+  }
+  // f(number of columns rounded up to 4, 8 or 16)
+  template <class Fn> static void by_columns(int k, Fn f) {
+    if (k <= 4) f(std::integral_constant<int, 4>());
+    else if (k <= 8) f(std::integral_constant<int, 8>());
+    else f(std::integral_constant<int, 16>());
+  }
+  // Arnoldi step j of an fp32 generic level: SpMV + dots and the update
+  void gstep(GLevel &L, int j, float *Hcol) {
+    float *w = L.w->as<float>();
+    by_columns(j + 1, [&](auto nv) {
+      constexpr int NV = decltype(nv)::value;
+      Cols<float, NV> c{};
+      for (int k = 0; k <= j; ++k) c.p[k] = L.Vc<float>(k);
+      EpiDots<float, NV> epi{w, c, j + 1, Hcol, partial<float>(), counter(0)};
+      const SellArgs a = L.mat == F3R_F16 ? argsv<half_t>() : args();
+      if (L.mat == F3R_F16)
+        launch_sell<half_t, float, float>(sh16->K, a, A16->as<half_t>(), L.Zc<float>(j), epi, st(), spmv_grid);
+      else
+        launch_sell<float, float, float>(sh->K, a, A32->as<float>(), L.Zc<float>(j), epi, st(), spmv_grid);
+      finish_dots<float>(sell_blocks(a, spmv_grid), j, Hcol);
+      update_launch<float, NV>(w, c, j, Hcol, j + 1 < L.m);
+    });
+    if (j + 1 < L.m) pending = {w, Hcol + j + 1, L.Vc<float>(j + 1)};
+  }
+  template <class SI> void gsolution(GLevel &L, SI *out, float s_in) {
+    by_columns(L.m, [&](auto nv) {
+      constexpr int NV = decltype(nv)::value;
+      Cols<float, NV> c{};
+      for (int k = 0; k < L.m; ++k) c.p[k] = L.Zc<float>(k);
+      const bool vec = aligned4(out);  // the columns are
+      auto kern = vec ? k_solution<float, SI, NV, true> : k_solution<float, SI, NV, false>;
+      hipLaunchKernelGGL(kern, dim3(vgrid(vec)), dim3(kBlock), 0, st(), (int64_t)n, c, L.m,
+                         (const float *)L.H->as<float>(), (const float *)norm_parts<float>(), update_parts, out, 1.f,
+                         s_in / L.s);
+    });
   }
 
   void level2_any(const double *in, double *out) {
@@ -1455,6 +1545,7 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
       L.sn = dev_alloc(sizeof(float) * q.m);
       L.e = dev_alloc(sizeof(float) * (q.m + 1));
       L.inv = dev_alloc(sizeof(float) * 4);
+      if (q.store == F3R_F32) L.w = dev_alloc(sizeof(float) * ld);
       S->glev.push_back(L);
     }
   } else if (p.variant == 2) {

@@ -274,3 +274,33 @@ def test_training_lowers_loss_and_learned_solve_converges(ctx):
     print(f"held-in system: {r}")
     for k in ("plain", "learned"):
         assert r[k]["solved"] and r[k]["true_rel_res"] <= 1e-8
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("count", [1, 8, 11])
+def test_probe_groups(ctx, kind, count):
+    """the loss over any number of probes (groups of 8 share their launches) is
+    the mean over the probes taken one at a time, and so is its gradient"""
+    import f3r_amd as F
+    from f3r_amd import learn
+    A = F.CSR.convdiff7(13, 12, 11, sigma=1.0, corr=3.0, peclet=0.0, seed=2)
+    d = A.diagonal()
+    F.algorithm.scaling(A)
+    P = F.SDAINV(A, 0.1, 1.0, "f16", ctx=ctx)
+    L = learn.LearnSystem(ctx, A, P, learn.features(A, P, d))
+    Z = learn.random_probes(A.n, count, 3)
+    mlp = learn.MLP(ctx, 1)
+    p = learn.unpack(mlp.get())
+    p["w3"] = np.random.default_rng(1).normal(0, 0.1, p["w3"].shape).astype(np.float32)
+    mlp.set(learn.pack(p))
+
+    def run(z):
+        L.set_probes(z)
+        mlp.grad_zero()
+        return L.loss(mlp, grad=True, kind=kind), mlp.grad().astype(np.float64)
+    loss, grad = run(Z)
+    each = [run(Z[k:k + 1]) for k in range(count)]
+    assert abs(loss - np.mean([e[0] for e in each])) <= 1e-6 * abs(loss)
+    ref = np.mean([e[1] for e in each], 0)
+    # the row gradients are rounded to bf16 in the backward products (2^-9 each, of either sign)
+    assert np.linalg.norm(grad - ref) <= 2.0 ** -8 * np.mean([np.linalg.norm(e[1]) for e in each])
