@@ -71,26 +71,63 @@ __global__ __launch_bounds__(kBlock) void k_dot(int64_t n, const T1 *__restrict_
 // CSR SpMV (CSR<T>::operate / compute_residual, csr.hpp:32-50): y = A x, or
 // y = b - A x with b.  TPR consecutive lanes take a row: lane q sums entries
 // q, q + TPR, ... in order, and the TPR sums are added by a butterfly over
-// the lanes, so every lane's loads of val and idx are coalesced with its
-// neighbours'.  TPR = 1 sums each row in CSR order (bit-identical to the SELL
+// the lanes.  TPR = 1 sums each row in CSR order (bit-identical to the SELL
 // kernels and the oracle); TPR > 1 reassociates the sum.  Sums in fp64 for
 // fp64 values, else fp32.
+// A block's kBlock / TPR rows are one run of entries: when it fits kCsrCap,
+// all threads load it coalesced, every load and gather of a thread in flight
+// at once, and leave values and gathered x in LDS for the row sums.  Read row
+// by row instead, each lane waited for its index and then its x once per TPR
+// entries: 36 us against 20 for 300 K uneven rows of 14 entries in fp64.  A
+// longer run (rows far above the mean, or TPR set below it) is read row by row.
+constexpr int kCsrCap = 2048;
 template <class V, class X, class Y, class ACC, int TPR>
 __global__ __launch_bounds__(kBlock) void k_csr(int32_t n, const int32_t *__restrict__ rptr,
                                                 const int32_t *__restrict__ idx, const V *__restrict__ val,
                                                 const X *__restrict__ x, Y *__restrict__ y,
                                                 const Y *__restrict__ b) {
-  constexpr int kRowsPerBlock = kBlock / TPR;
+  constexpr int kRows = kBlock / TPR, kPer = kCsrCap / kBlock;
+  __shared__ V sv[kCsrCap];
+  __shared__ X sx[kCsrCap];
   const int q = threadIdx.x % TPR;
-  for (int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + threadIdx.x / TPR; row < n;
-       row += (int64_t)gridDim.x * kRowsPerBlock) {
+  for (int64_t row0 = (int64_t)xcd_block() * kRows; row0 < n; row0 += (int64_t)gridDim.x * kRows) {
+    const int32_t e0 = rptr[row0], e1 = rptr[row0 + kRows < n ? row0 + kRows : n];
+    const int64_t row = row0 + threadIdx.x / TPR;
+    int32_t k0 = 0, k1 = 0;
+    if (row < n) {
+      k0 = rptr[row];
+      k1 = rptr[row + 1];
+    }
     ACC acc = 0;
-    const int32_t k1 = rptr[row + 1];
-    for (int32_t k = rptr[row] + q; k < k1; k += TPR)
-      acc = fma_<ACC>((ACC)to_acc(val[k]), (ACC)to_acc(x[idx[k]]), acc);
+    if (e1 - e0 <= kCsrCap) {
+      int32_t c[kPer];
+      V v[kPer];
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int32_t k = e0 + (int32_t)threadIdx.x + i * kBlock;
+        c[i] = k < e1 ? idx[k] : 0;
+        v[i] = k < e1 ? val[k] : V(0);
+      }
+      X xv[kPer];
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        if (e0 + (int32_t)threadIdx.x + i * kBlock < e1) xv[i] = x[c[i]];
+#pragma unroll
+      for (int i = 0; i < kPer; ++i)
+        if (e0 + (int32_t)threadIdx.x + i * kBlock < e1) {
+          sv[threadIdx.x + i * kBlock] = v[i];
+          sx[threadIdx.x + i * kBlock] = xv[i];
+        }
+      __syncthreads();
+      for (int32_t k = k0 - e0 + q; k < k1 - e0; k += TPR)
+        acc = fma_<ACC>((ACC)to_acc(sv[k]), (ACC)to_acc(sx[k]), acc);
+      __syncthreads();  // the next run overwrites the staging
+    } else {
+      for (int32_t k = k0 + q; k < k1; k += TPR) acc = fma_<ACC>((ACC)to_acc(val[k]), (ACC)to_acc(x[idx[k]]), acc);
+    }
 #pragma unroll
     for (int off = TPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
-    if (q == 0) y[row] = b ? cvt<Y>((ACC)to_acc(b[row]) - acc) : cvt<Y>(acc);
+    if (q == 0 && row < n) y[row] = b ? cvt<Y>((ACC)to_acc(b[row]) - acc) : cvt<Y>(acc);
   }
 }
 

@@ -394,6 +394,40 @@ def test_csr_spmv_lanes_per_row(ctx, tpr, vd, xd, yd):
         assert np.all(np.abs(got - exact) <= tol), (name, float(np.max(np.abs(got - exact) - tol)))
 
 
+@pytest.mark.parametrize("lens", [[8] * 256,                      # one block's run fills the staging exactly
+                                  [8] * 255 + [9],                # one entry more: read row by row
+                                  [8] * 257, [0] * 300, [1, 0, 5] * 200,
+                                  [3] * 400 + [5000] + [0, 2] * 150])
+@pytest.mark.parametrize("tpr", [1, 4, 64])
+def test_csr_staged_runs(ctx, lens, tpr):
+    """the CSR product at the ends of its staged runs of entries: bit-exact
+    with one lane per row, within the sums' rounding with several"""
+    import f3r_amd as F
+    rng = np.random.default_rng(12)
+    n = max(len(lens), max(lens) + 1)
+    lens = np.array(list(lens) + [1] * (n - len(lens)))
+    rptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    idx = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in lens]).astype(np.int32)
+    A = F.CSR(n, rptr, idx, rng.uniform(-1, 1, idx.size))
+    x, b = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n)
+    print(f"csr staged runs n={n} nnz={A.nnz} tpr={tpr}", flush=True)
+    M = F.CSRDevice(ctx, A, "f64", tpr=tpr)
+    xv, bv, yv = F.vector.from_numpy(ctx, x), F.vector.from_numpy(ctx, b), F.vector(ctx, "f64", n)
+    for rhs in (None, b):
+        if rhs is None:
+            M.operate(xv, yv)
+        else:
+            M.compute_residual(bv, xv, yv)
+        got = yv.download()
+        ref = O.spmv(n, rptr, idx, A.val, x, 0, 0, 0, 0, **({} if rhs is None else {"b": b}))
+        if tpr == 1:
+            assert np.array_equal(got, ref)
+        else:
+            rows = np.repeat(np.arange(n), lens)
+            mag = np.bincount(rows, np.abs(A.val * x[idx]), minlength=n) + np.abs(b)
+            assert np.all(np.abs(got - ref) <= 2 * (int(lens.max()) + 1) * 2.0 ** -53 * mag)
+
+
 @pytest.mark.parametrize("C,sigma,K", [(64, 1, 2), (32, 256, 4), (128, 1, 8)])
 @pytest.mark.parametrize("vd,xd,yd", [("f64", "f64", "f64"), ("f32", "f32", "f32"), ("f16", "f16", "f16"),
                                       ("f16", "f32", "f32")])
