@@ -67,7 +67,6 @@ struct Reducer {
   DevPtr partial;
   static constexpr int kSlots = 24;                     // reduction slots of kCounterSlot counters
   DevPtr counters;
-  DevPtr scalars;   // 64 doubles of results
 };
 
 struct Context {
@@ -77,6 +76,7 @@ struct Context {
   int num_cu = 256;
   Reducer red;
   double *pinned = nullptr;  // host-pinned landing buffer for small reads
+  double *pinned_dev = nullptr;  // its device address
   // scratch of the calls that need some between launches on this stream (the
   // largest size asked for so far; a call uses it only until it returns, and
   // calls on one context run one after another)

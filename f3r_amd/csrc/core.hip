@@ -2,6 +2,7 @@
 // vectors, CSR / SELL-C-sigma matrices, the BLAS-1 kernels with single-pass
 // grid reductions, and the SDAINV / ILU(0) preconditioner objects.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -38,6 +39,10 @@ template <class T> __global__ void k_fill(T *__restrict__ p, int64_t n, T v) {
     p[i] = v;
 }
 
+template <class T> __global__ void k_copy(const T *s, T *d, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) d[i] = s[i];
+}
+
 template <class S, class D> __global__ void k_cast(const S *__restrict__ s, D *__restrict__ d, int64_t n) {
   for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
     d[i] = cvt<D>(to_acc(s[i]));
@@ -65,7 +70,9 @@ __global__ __launch_bounds__(kBlock) void k_dot(int64_t n, const T1 *__restrict_
   A v[1] = {0};
   for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
     v[0] = fma_<A>((A)to_acc(a[i]), (A)to_acc(b[i]), v[0]);
-  if (grid_sum<A, 1>(v, partial, counter, lds) && threadIdx.x == 0) *out = (double)v[0];
+  // system scope: `out` may be host memory that the caller polls
+  if (grid_sum<A, 1>(v, partial, counter, lds) && threadIdx.x == 0)
+    __hip_atomic_store(out, (double)v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // CSR SpMV (CSR<T>::operate / compute_residual, csr.hpp:32-50): y = A x, or
@@ -509,9 +516,9 @@ std::shared_ptr<Context> ctx_create(int device) {
   F3R_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   c->red.partial = dev_alloc(sizeof(double) * Reducer::kPartialDoubles);
   c->red.counters = dev_alloc(sizeof(unsigned) * Reducer::kSlots * kCounterSlot);
-  c->red.scalars = dev_alloc(sizeof(double) * 64);
   F3R_HIP(hipMemsetAsync(c->red.counters->p, 0, sizeof(unsigned) * Reducer::kSlots * kCounterSlot, c->stream));
   F3R_HIP(hipHostMalloc((void **)&c->pinned, 4096, hipHostMallocDefault));
+  F3R_HIP(hipHostGetDevicePointer((void **)&c->pinned_dev, c->pinned, 0));
   c->na_scratch = noalloc_scratch(device);
   F3R_HIP(hipStreamSynchronize(c->stream));
   return c;
@@ -534,10 +541,36 @@ void *Context::workspace(size_t bytes) {
   return work->p;
 }
 
-double read_scalar(Context *c, const double *dev) {
-  F3R_HIP(hipMemcpyAsync(c->pinned, dev, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  F3R_HIP(hipStreamSynchronize(c->stream));
-  return c->pinned[0];
+// A NaN that no arithmetic produces: the landing slot before its value comes.
+constexpr uint64_t kNoScalar = 0x7ff8f3f3f3f3f3f3ULL;
+
+double *arm_scalar(Context *c) {
+  *reinterpret_cast<volatile uint64_t *>(c->pinned) = kNoScalar;
+  return c->pinned_dev;
+}
+// A copy back to the host and a stream synchronisation cost 15 us a scalar;
+// the kernel's own store to pinned memory is seen 2 us after it is made.
+// Polls for at most 0.2 ms, then waits for the stream (a long queue, a failed
+// launch, or the armed value itself as the result).
+double wait_scalar(Context *c) {
+  const volatile uint64_t *slot = reinterpret_cast<const volatile uint64_t *>(c->pinned);
+  uint64_t u = *slot;
+  if (u == kNoScalar) {
+    const auto t0 = std::chrono::steady_clock::now();
+    do {
+      for (int i = 0; i < 64 && u == kNoScalar; ++i) {
+        __builtin_ia32_pause();
+        u = *slot;
+      }
+    } while (u == kNoScalar && std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200));
+    if (u == kNoScalar) {
+      F3R_HIP(hipStreamSynchronize(c->stream));
+      u = *slot;
+    }
+  }
+  double v;
+  std::memcpy(&v, &u, 8);
+  return v;
 }
 
 // ------------------------------------------------------------- vectors ---
@@ -572,6 +605,17 @@ void vec_copy(Vec *s, Vec *d) {
   F3R_CHECK(s->dtype != F3R_I32 && d->dtype != F3R_I32, F3R_ERR_UNSUPPORTED, "copy: int32 vectors");
   hipStream_t st = d->ctx->stream;
   if (s->dtype == d->dtype) {
+    // a copy kernel costs the host a third of a copy command; beyond 1 MB the
+    // copy itself is what counts
+    const size_t es = dtype_size(s->dtype);
+    if (s->n && s->n * es <= (1 << 20)) {
+      const dim3 g(grid_for(s->n, d->ctx->num_cu)), b(kBlock);
+      if (es == 8) hipLaunchKernelGGL(k_copy<uint64_t>, g, b, 0, st, (const uint64_t *)s->ptr(), (uint64_t *)d->ptr(), s->n);
+      else if (es == 4) hipLaunchKernelGGL(k_copy<uint32_t>, g, b, 0, st, (const uint32_t *)s->ptr(), (uint32_t *)d->ptr(), s->n);
+      else hipLaunchKernelGGL(k_copy<uint16_t>, g, b, 0, st, (const uint16_t *)s->ptr(), (uint16_t *)d->ptr(), s->n);
+      F3R_HIP(hipGetLastError());
+      return;
+    }
     F3R_HIP(hipMemcpyAsync(d->ptr(), s->ptr(), s->n * dtype_size(s->dtype), hipMemcpyDeviceToDevice, st));
     return;
   }
@@ -620,7 +664,7 @@ static void dot_launch(Context *c, int64_t n, const T1 *a, const T2 *b, double *
 }
 
 double dot_raw(Context *c, int da, const void *pa, int db, const void *pb, int64_t n) {
-  double *slot = c->red.scalars->as<double>();
+  double *slot = arm_scalar(c);
   F3R_CHECK(da != F3R_I32 && db != F3R_I32, F3R_ERR_UNSUPPORTED, "dot: int32");
   // accumulate in the wider type; fp16 data in fp32
 #define F3R_DOT(TA, TB)                                                         \
@@ -645,7 +689,7 @@ double dot_raw(Context *c, int da, const void *pa, int db, const void *pb, int64
   }
 #undef F3R_DOT
   F3R_HIP(hipGetLastError());
-  return read_scalar(c, slot);
+  return wait_scalar(c);
 }
 
 // dot of two device arrays into *out (device), with the scratch array as

@@ -296,6 +296,17 @@ __device__ __forceinline__ bool grid_sum(T (&v)[NV], T *__restrict__ partial,
   __syncthreads();
   if (wid != 0) return false;
   const int G = gridDim.x;
+  if (G == 1) {  // nothing to wait for
+    if (lane == 0)
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        T t = lds[i * kWavesPerBlock];
+#pragma unroll
+        for (int w = 1; w < kWavesPerBlock; ++w) t += lds[i * kWavesPerBlock + w];
+        v[i] = t;
+      }
+    return lane == 0;
+  }
   const int ng = (G + kGroup - 1) / kGroup;
   const int grp = blockIdx.x / kGroup;
   const int b0 = grp * kGroup;
@@ -320,6 +331,14 @@ __device__ __forceinline__ bool grid_sum(T (&v)[NV], T *__restrict__ partial,
   for (int i = 0; i < NV; ++i) {
     acc[i] = lane < gsize ? collect(&partial[(int64_t)i * G + b0 + lane]) : (T)0;
     acc[i] = wave_sum(acc[i]);
+  }
+  if (ng == 1) {  // one group: its sums are the totals (a second round trip saved)
+    if (lane == 0) {
+      __hip_atomic_store(&counters[(1 + grp) * kCounterStride], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) v[i] = acc[i];
+    }
+    return lane == 0;
   }
   T *gpart = partial + (int64_t)NV * G;
   last = 0;

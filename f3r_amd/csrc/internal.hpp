@@ -151,7 +151,11 @@ template <class S> __device__ __forceinline__ S diag_apply(const typename DiagWZ
 }
 
 std::shared_ptr<Context> ctx_create(int device);
-double read_scalar(Context *c, const double *dev);
+// The context's landing slot for one fp64 result of a kernel: arm_scalar
+// before the launch gives the address the kernel stores to (one 8-byte
+// system-scope store), wait_scalar returns the value.
+double *arm_scalar(Context *c);
+double wait_scalar(Context *c);
 SellArgs sell_args(const SellShared &sh, bool with_perm);
 DevPtr upload_values(Context *ctx, const std::vector<double> &v, int dtype);
 HostCSR permute_csr(const HostCSR &M, const std::vector<int32_t> &perm);
