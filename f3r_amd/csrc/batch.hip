@@ -211,6 +211,52 @@ __global__ __launch_bounds__(kBlock) void k_b_norm2(const A *__restrict__ v, A *
   if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
 }
 
+// Right-hand sides and initial guesses into the tiles of all segments (zero
+// in the padding), and the block sums of ||b||^2.  bp[seg], xp[seg]: the
+// callers' vectors; rows[seg] of them.  One launch; a copy per vector and a
+// dot per segment, each waited for, took 3 ms of 16 for 64 segments.
+__global__ __launch_bounds__(kBlock) void k_b_take(const double *const *bp, const double *const *xp,
+                                                   const int32_t *__restrict__ rows, const int32_t *__restrict__ bseg,
+                                                   const int32_t *__restrict__ sb0, double *__restrict__ b,
+                                                   double *__restrict__ x, double *__restrict__ partial) {
+  __shared__ double lds[kWavesPerBlock];
+  const int seg = bseg[blockIdx.x];
+  const int64_t r0 = (int64_t)sb0[seg] * kTile;
+  const int32_t n = rows[seg];
+  const double *bs = bp[seg], *xs = xp[seg];
+  double s[1] = {0.0};
+  double bv[kRows], xv[kRows];
+#pragma unroll
+  for (int q = 0; q < kRows; ++q) {
+    const int64_t k = tile_row(q) - r0;
+    bv[q] = k < n ? bs[k] : 0.0;
+    xv[q] = k < n ? xs[k] : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < kRows; ++q) {
+    const int64_t i = tile_row(q);
+    b[i] = bv[q];
+    x[i] = xv[q];
+    s[0] = fma_<double>(bv[q], bv[q], s[0]);
+  }
+  block_sum<double, 1>(s, lds);
+  if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
+}
+// the solutions back into the callers' vectors
+__global__ __launch_bounds__(kBlock) void k_b_give(const double *__restrict__ x, double *const *xp,
+                                                   const int32_t *__restrict__ rows, const int32_t *__restrict__ bseg,
+                                                   const int32_t *__restrict__ sb0) {
+  const int seg = bseg[blockIdx.x];
+  const int64_t r0 = (int64_t)sb0[seg] * kTile;
+  const int32_t n = rows[seg];
+  double *xs = xp[seg];
+#pragma unroll
+  for (int q = 0; q < kRows; ++q) {
+    const int64_t i = tile_row(q), k = i - r0;
+    if (k < n) xs[k] = x[i];
+  }
+}
+
 // One block per segment: ||w|| from its blocks' partials, then H(j+1, j),
 // 1/||w|| (0 for a zero vector), the guarded Givens step and |e_{j+1}|.
 // H, e, cs, sn point at segment 0's column j / arrays; strides per segment.
@@ -771,8 +817,16 @@ struct BatchSolver {
   bool zh = false;
   DevPtr Zh3;
   half_t *zh3(int k) const { return Zh3->as<half_t>() + (int64_t)k * N; }
-  DevPtr partial, status, jseg, rich;
-  DevPtr b_int, x_int, r_int;
+  DevPtr partial, rich, rows;  // rows: per segment, without the padding
+  DevPtr b_int, x_int;
+  // per-segment host values that the kernels read and write in pinned host
+  // memory (no copy commands): status, the residual norms; jseg, the steps of
+  // a cycle; bp / xp, the callers' vectors of a solve
+  void *pin = nullptr;
+  double *status = nullptr;
+  int32_t *jseg = nullptr;
+  const double **bp = nullptr;
+  double **xp = nullptr;
   // outer level (fp64)
   BLevel<double> L1;
   BLevel<float> L2, L3;
@@ -791,6 +845,19 @@ struct BatchSolver {
     for (auto &g : graphs) (void)hipGraphExecDestroy(g.second);
     for (auto &g : step_graphs) (void)hipGraphExecDestroy(g.second);
     for (auto &g : graph_src) (void)hipGraphDestroy(g);
+    if (pin) (void)hipHostFree(pin);
+  }
+  // the pinned values (device addresses equal to the host's)
+  void alloc_pinned() {
+    const size_t n = (size_t)nseg;
+    F3R_HIP(hipHostMalloc(&pin, n * (8 + 8 + 8 + 4), hipHostMallocDefault));
+    void *dev = nullptr;
+    F3R_HIP(hipHostGetDevicePointer(&dev, pin, 0));
+    F3R_CHECK(dev == pin, F3R_ERR_HIP, "batch: pinned memory without a unified address");
+    status = static_cast<double *>(pin);
+    xp = reinterpret_cast<double **>(status + n);
+    bp = const_cast<const double **>(xp + n);
+    jseg = reinterpret_cast<int32_t *>(xp + 2 * n);
   }
 
   hipStream_t st() const { return ctx->stream; }
@@ -1076,7 +1143,7 @@ struct BatchSolver {
       level2(V + (int64_t)j * N, L.Zc(N, j), body_graph);
       spmv<double, double, double, double>(A64->as<double>(), false, (const double *)L.Zc(N, j),
                                            V + (int64_t)(j + 1) * N, nullptr);
-      arnoldi(L, j, 0, status->as<double>(), (const double *)L.Vc(N, 0), false);
+      arnoldi(L, j, 0, status, (const double *)L.Vc(N, 0), false);
     };
     const uint64_t pat = p.use_graph ? next_pattern() : UINT64_MAX;
     const auto key = std::make_pair(pat, j);
@@ -1111,10 +1178,8 @@ struct BatchSolver {
   }
 
   std::vector<double> read_status() {
-    std::vector<double> h(nseg);
-    F3R_HIP(hipMemcpyAsync(h.data(), status->p, sizeof(double) * nseg, hipMemcpyDeviceToHost, st()));
     F3R_HIP(hipStreamSynchronize(st()));
-    return h;
+    return std::vector<double>(status, status + nseg);
   }
 
   // Restarted<double>(FGMRES<double>(A, L2, {m1, true}), {restart}) per segment
@@ -1143,7 +1208,7 @@ struct BatchSolver {
                          (const double *)partial->as<double>(), (const int32_t *)sb0->as<int32_t>(),
                          (const int32_t *)snb->as<int32_t>(), L.e->as<double>(), (int64_t)(m1 + 1),
                          (double *)nullptr, (double *)nullptr, (int64_t)0, (double *)nullptr, (int64_t)0, -1, 0,
-                         L.inv->as<double>(), status->as<double>());
+                         L.inv->as<double>(), status);
       hipLaunchKernelGGL((k_b_vscale<double, double>), dim3(G), dim3(kBlock), 0, st(), V,
                          (const double *)L.inv->as<double>(), (const int32_t *)bs());
       std::vector<double> e = read_status();
@@ -1181,12 +1246,12 @@ struct BatchSolver {
         if (!left) break;
       }
       // x += Z y(j_s) for every segment that stepped in this cycle
-      F3R_HIP(hipMemcpyAsync(jseg->p, jdone.data(), sizeof(int32_t) * nseg, hipMemcpyHostToDevice, st()));
+      std::copy(jdone.begin(), jdone.end(), jseg);
       hipLaunchKernelGGL((k_b_combine<double, double, double>), dim3(G), dim3(kBlock), 0, st(),
                          (const double *)L.Zc(N, 0), N, (const double *)Hd, L.hs(), m1 + 1,
-                         (const double *)L.e->as<double>(), (int64_t)(m1 + 1), (const int32_t *)jseg->as<int32_t>(),
+                         (const double *)L.e->as<double>(), (int64_t)(m1 + 1), (const int32_t *)jseg,
                          0, (const int32_t *)bs(), x_int->as<double>(), 1, (const float *)nullptr);
-      F3R_HIP(hipStreamSynchronize(st()));  // jdone is host memory of this scope
+      F3R_HIP(hipStreamSynchronize(st()));  // jseg is written again by the next cycle
     }
     F3R_HIP(hipGetLastError());
     res.resize(nseg);
@@ -1426,8 +1491,8 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
   B->b_int = dev_alloc(sizeof(double) * N);
   B->x_int = dev_alloc(sizeof(double) * N);
   B->partial = dev_alloc(sizeof(double) * (int64_t)B->G * (p.m1 + 1 + 16));
-  B->status = dev_alloc(sizeof(double) * nseg);
-  B->jseg = dev_alloc(sizeof(int32_t) * nseg);
+  B->rows = up32(B->nrow);
+  B->alloc_pinned();
   B->rich = dev_alloc(sizeof(RichSeg) * nseg);
   F3R_HIP(hipStreamSynchronize(c->stream));
   return B.release();
@@ -1469,28 +1534,35 @@ int f3r_batch_solve(f3r_batch B, const f3r_vec *b, f3r_vec *x, f3r_result *res) 
   hipStream_t st = S->ctx->stream;
   const int nseg = S->nseg;
   std::vector<double> nrm_b(nseg);
-  F3R_HIP(hipMemsetAsync(S->b_int->p, 0, sizeof(double) * S->N, st));
-  F3R_HIP(hipMemsetAsync(S->x_int->p, 0, sizeof(double) * S->N, st));
   for (int s = 0; s < nseg; ++s) {
     Vec *bv = vec_of(b[s]), *xv = vec_of(x[s]);
     F3R_CHECK(bv && xv && bv->dtype == F3R_F64 && xv->dtype == F3R_F64 && bv->n == S->nrow[s] && xv->n == S->nrow[s],
               F3R_ERR_ARG, "batch_solve: b and x of each segment: fp64 vectors of its matrix size");
-    F3R_HIP(hipMemcpyAsync(S->b_int->as<double>() + S->off[s], bv->ptr(), sizeof(double) * S->nrow[s],
-                           hipMemcpyDeviceToDevice, st));
-    F3R_HIP(hipMemcpyAsync(S->x_int->as<double>() + S->off[s], xv->ptr(), sizeof(double) * S->nrow[s],
-                           hipMemcpyDeviceToDevice, st));
-    nrm_b[s] = std::sqrt(dot_raw(S->ctx.get(), F3R_F64, bv->ptr(), F3R_F64, bv->ptr(), S->nrow[s]));
   }
-  F3R_HIP(hipStreamSynchronize(st));
+  F3R_HIP(hipStreamSynchronize(st));  // the last solve's reads of the pinned pointers
+  for (int s = 0; s < nseg; ++s) {
+    S->bp[s] = static_cast<const double *>(vec_of(b[s])->ptr());
+    S->xp[s] = static_cast<double *>(vec_of(x[s])->ptr());
+  }
+  const int32_t *rows = S->rows->as<int32_t>(), *bseg = S->bs(), *sb0 = S->sb0->as<int32_t>();
+  hipLaunchKernelGGL(k_b_take, dim3(S->G), dim3(kBlock), 0, st, S->bp, (const double *const *)S->xp, rows, bseg, sb0,
+                     S->b_int->as<double>(), S->x_int->as<double>(), S->partial->as<double>());
+  // no rotation (j = -1), no Hessenberg column: the norm itself
+  hipLaunchKernelGGL(k_b_norm_finish<double>, dim3(nseg), dim3(kBlock), 0, st, (const double *)S->partial->as<double>(),
+                     sb0, (const int32_t *)S->snb->as<int32_t>(), S->L1.e->as<double>(), (int64_t)(S->L1.m + 1),
+                     (double *)nullptr, (double *)nullptr, (int64_t)0, (double *)nullptr, (int64_t)0, -1, 0,
+                     S->L1.inv->as<double>(), S->status);
+  F3R_HIP(hipGetLastError());
+  nrm_b = S->read_status();
   const auto t0 = std::chrono::steady_clock::now();
   std::vector<f3r_result> r;
   S->solve(nrm_b, r);
   F3R_HIP(hipStreamSynchronize(st));
   const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+  hipLaunchKernelGGL(k_b_give, dim3(S->G), dim3(kBlock), 0, st, (const double *)S->x_int->as<double>(), S->xp, rows,
+                     bseg, sb0);
+  F3R_HIP(hipGetLastError());
   for (int s = 0; s < nseg; ++s) {
-    Vec *xv = vec_of(x[s]);
-    F3R_HIP(hipMemcpyAsync(xv->ptr(), S->x_int->as<double>() + S->off[s], sizeof(double) * S->nrow[s],
-                           hipMemcpyDeviceToDevice, st));
     r[s].solve_s = secs;
     res[s] = r[s];
   }
