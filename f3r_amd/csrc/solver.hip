@@ -1475,10 +1475,13 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
   S->dots_grid = (int)std::min<int64_t>((n + kBlock - 1) / kBlock, std::min(kMaxReduceGrid, 8 * ctx->num_cu));
   if (p.grid > 0) S->dots_grid = (int)std::min<int64_t>((n + kBlock - 1) / kBlock, std::min((int)p.grid, kMaxReduceGrid));
   // the SpMV kernels with a fused reduction: one row per thread (the gathers
-  // need the waves; the arrivals of 8x more blocks cost less than that), up
-  // to the reduction's block limit; flags bit 1 caps them like the others
-  S->spmv_grid = (p.flags & 2) ? S->dots_grid
-                               : (int)std::min<int64_t>((n + kBlock - 1) / kBlock, kMaxReduceGrid);
+  // need the waves), or two where that brings their blocks within what
+  // the CGS update adds up itself: 27-point 352 K rows 4.75 -> 4.55 ms a solve
+  // without the finishing launches.  With four rows (7-point, 885 K rows) the
+  // longer SpMV takes the gain back.
+  // flags bit 1 caps them like the others.
+  const int64_t full = (n + kBlock - 1) / kBlock, per = (full + kDirectDots - 1) / kDirectDots;
+  S->spmv_grid = (p.flags & 2) ? S->dots_grid : (int)std::min<int64_t>(per <= 2 ? (full + per - 1) / per : full, kMaxReduceGrid);
   auto dd = [](int64_t cnt) { return dev_alloc(sizeof(double) * std::max<int64_t>(cnt, 1)); };
   S->V1 = dd(n * (p.m1 + 1));
   S->Z1 = dd(n * p.m1);
