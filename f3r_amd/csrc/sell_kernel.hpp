@@ -394,6 +394,16 @@ template <class Y, class ACC> struct EpiStore {
     const int row = perm ? perm[r] : r;
     y[row] = cvt<Y>(acc);
   }
+  // four consecutive rows of a lane (quad.hpp)
+  struct Pre4 {};
+  bool vec4() const { return !perm && ((uintptr_t)y % (4 * sizeof(Y))) == 0; }
+  __device__ Pre4 pre4(int) const { return {}; }
+  __device__ void row4(int r, ACC (&acc)[4], const Pre4 &, State &) const {
+    V4<Y> o;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o.v[c] = cvt<Y>(acc[c]);
+    st4(y + r, o);
+  }
   __device__ void finish(State &) const {}
 };
 
@@ -409,6 +419,19 @@ template <class Y, class B, class ACC> struct EpiResid {
   __device__ void row(int r, ACC acc, const Pre &p, State &) const {
     const int row = perm ? perm[r] : r;
     y[row] = cvt<Y>((ACC)to_acc(p.b) - acc);
+  }
+  struct Pre4 {
+    V4<B> b;
+  };
+  bool vec4() const {
+    return !perm && ((uintptr_t)y % (4 * sizeof(Y))) == 0 && ((uintptr_t)b % (4 * sizeof(B))) == 0;
+  }
+  __device__ Pre4 pre4(int r) const { return {ld4(b + r)}; }
+  __device__ void row4(int r, ACC (&acc)[4], const Pre4 &p, State &) const {
+    V4<Y> o;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o.v[c] = cvt<Y>((ACC)to_acc(p.b.v[c]) - acc[c]);
+    st4(y + r, o);
   }
   __device__ void finish(State &) const {}
 };

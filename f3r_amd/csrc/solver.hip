@@ -24,6 +24,7 @@
 
 #include "common.hpp"
 #include "internal.hpp"
+#include "quad.hpp"
 #include "sell_kernel.hpp"
 
 namespace f3r {
@@ -119,6 +120,32 @@ template <class T, int NV> struct EpiDots {
 #pragma unroll
     for (int k = 0; k < NV; ++k)
       if (k < ncols) s.v[k] = fma_<T>(acc, p.v[k], s.v[k]);
+  }
+  struct Pre4 {
+    V4<T> v[NV];
+  };
+  bool vec4() const {
+    bool ok = aligned4(w);
+    for (int k = 0; k < ncols; ++k) ok = ok && aligned4(cols.p[k]);
+    return ok;
+  }
+  __device__ Pre4 pre4(int r) const {
+    Pre4 p;
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (k < ncols) p.v[k] = ld4(cols.p[k] + r);
+    return p;
+  }
+  __device__ void row4(int r, T (&acc)[4], const Pre4 &p, State &s) const {
+    V4<T> o;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o.v[c] = acc[c] * xs;
+    st4(w + r, o);
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (k < ncols)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s.v[k] = fma_<T>(o.v[c], p.v[k].v[c], s.v[k]);
   }
   // Block sums only, into partial[k * gridDim.x + block]; k_dots_finish adds
   // them in the next launch.  A grid reduction finished in this kernel made
@@ -573,6 +600,45 @@ template <class S, class F, class ACC> struct EpiL4Diag {
     else
       hnext[r] = h;
   }
+  struct Pre4 {
+    V4<S> hin, hout, w, z;
+  };
+  bool vec4() const {
+    bool ok = aligned4(hin) && aligned4(hout) && aligned4(hnext) && aligned4(out);
+    if constexpr (std::is_same<S, half_t>::value) return ok && aligned4(d.wz) && !hr_out;
+    else return ok && aligned4(d.w) && aligned4(d.z) && !hr_out;
+  }
+  __device__ Pre4 pre4(int r) const {
+    Pre4 p;
+    p.hin = ld4(hin + r);
+    p.hout = ld4(hout + r);
+    if constexpr (std::is_same<S, half_t>::value) {
+      const V4<uint32_t> u = ld4(d.wz + r);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const typename DiagWZ<S>::V e = DiagWZ<S>::unpack(u.v[c]);
+        p.w.v[c] = e.w;
+        p.z.v[c] = e.z;
+      }
+    } else {
+      p.w = ld4(d.w + r);
+      p.z = ld4(d.z + r);
+    }
+    return p;
+  }
+  __device__ void row4(int r, ACC (&acc)[4], const Pre4 &p, State &) const {
+    V4<S> h;
+    V4<F> o;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const S hr = cvt<S>((ACC)to_acc(p.hin.v[c]) - acc[c]);
+      const S t2 = diag_apply<S>({p.w.v[c], p.z.v[c]}, hr);
+      h.v[c] = cvt<S>(fma_<A>((A)*w, to_acc(t2), to_acc(p.hout.v[c])));
+      o.v[c] = (F)to_acc(h.v[c]) * inv_s;
+    }
+    if (out) st4(out + r, o);
+    else st4(hnext + r, h);
+  }
   __device__ void finish(State &) const {}
 };
 
@@ -730,6 +796,7 @@ struct Solver {
   int64_t nnz = 0;
   std::shared_ptr<SellShared> sh;    // layout of A64 / A32
   std::shared_ptr<SellShared> sh16;  // layout of A16 (sh itself when K agrees)
+  std::shared_ptr<QuadSet> quad;     // value codes of A (null: too many distinct values)
   DevPtr A64, A32, A16;
   std::shared_ptr<Prec> P;
   float range_s = 1.f;
@@ -803,6 +870,27 @@ struct Solver {
     const int64_t per = vec ? 4 * kBlock : kBlock;
     return (int)std::min<int64_t>((n + per - 1) / per, (int64_t)ctx->num_cu * 16);
   }
+  // a product with A's values V: by their codes where the matrix has them
+  template <class V, class X, class ACC, class Epi>
+  void product(const V *val, const X *x, const Epi &epi, int grid = 0) const {
+    const SellShared &L = shv<V>();
+    const SellArgs a = argsv<V>();
+    if (quad) {
+      if constexpr (std::is_same<V, half_t>::value) {
+        if (L.K == 8) {
+          launch_quad<8, V, X, ACC>(a, quad->template args<V>(), val, x, epi, st());
+          return;
+        }
+      }
+      launch_quad<4, V, X, ACC>(a, quad->template args<V>(), val, x, epi, st());
+      return;
+    }
+    launch_sell<V, X, ACC>(L.K, a, val, x, epi, st(), grid);
+  }
+  // blocks of a product with A's values V that leaves block sums
+  template <class V> int dots_blocks() const {
+    return quad ? quad_blocks(argsv<V>(), quad->template args<V>()) : sell_blocks(argsv<V>(), spmv_grid);
+  }
   SellArgs args() const { return sell_args(*sh, false); }
   // the layout of the matrix with value type V (the fp16 copy may differ in K)
   template <class V> const SellShared &shv() const {
@@ -828,12 +916,12 @@ struct Solver {
     EpiDots<T, NV> epi{L.w(), c, j + 1, L.Hp() + (int64_t)j * L.ldh(), partial<T>(), counter(0)};
     if (!L.Zh.empty()) {
       epi.xs = (T)(1.0 / range_s);
-      launch_sell<V, half_t, T>(shv<V>().K, argsv<V>(), val, L.Zh[j], epi, st(), spmv_grid);
+      product<V, half_t, T>(val, L.Zh[j], epi, spmv_grid);
     } else {
-      launch_sell<V, T, T>(shv<V>().K, argsv<V>(), val, L.Z[j], epi, st(), spmv_grid);
+      product<V, T, T>(val, L.Z[j], epi, spmv_grid);
     }
     // block sums the SpMV + dots kernel wrote per dot: its grid
-    finish_dots<T>(sell_blocks(argsv<V>(), spmv_grid), j, L.Hp() + (int64_t)j * L.ldh());
+    finish_dots<T>(dots_blocks<V>(), j, L.Hp() + (int64_t)j * L.ldh());
   }
   template <class T> void finish_dots(int G, int j, T *Hcol) {
     if (G > kDirectDots)
@@ -922,7 +1010,7 @@ struct Solver {
   // in ACC (FLOAT / DOUBLE: the fp64 A summed in fp64, work/src/f3r-gpu.cpp:
   // 123-152, 174-203).  The result goes to `hz` (S), or h / s to `out` (F).
   template <class S, class F, class MV, class ACC>
-  void richardson(const F *in, F *out, S *hz, const MV *aval, const SellShared &lay) {
+  void richardson(const F *in, F *out, S *hz, const MV *aval) {
     ++cnt;
     ++calls;
     const bool probe = p.static_weight <= 0 && (cnt % p.c) == 0;
@@ -931,7 +1019,6 @@ struct Solver {
     RichDev *rs = rich->as<RichDev>();
     const F inv_s = (F)(1.f / range_s);
     const bool diag = P->kind == 0 && P->diag;
-    const SellArgs a = sell_args(lay, false);
     constexpr bool kSame = std::is_same<S, F>::value;
     S *hi = hin->as<S>(), *ho = hout->as<S>(), *ho2 = hout2->as<S>();
     S *hr_ = hr->as<S>(), *t2 = tmp2->as<S>(), *t = tt->as<S>();
@@ -946,15 +1033,13 @@ struct Solver {
     io.out = ho;
     io.w = probe ? nullptr : &rs->ome[0];
     prec_apply_io<S, F>(P.get(), io, st());
-    auto product = [&](const S *x, S *y) {
-      launch_sell<MV, S, ACC>(lay.K, a, aval, x, EpiStore<S, ACC>{y, nullptr}, st());
-    };
+    auto apply_a = [&](const S *x, S *y) { product<MV, S, ACC>(aval, x, EpiStore<S, ACC>{y, nullptr}); };
     auto probe_dots = [&](const S *ts, const S *r, int k) {
       hipLaunchKernelGGL(k_probe<S>, dim3(dots_grid), b, 0, st(), nn, ts, r, rs, k,
                          partial<typename Acc<S>::type>(), counter(2));
     };
     if (probe) {
-      product(ho, t);
+      apply_a(ho, t);
       probe_dots(t, hi, 0);
       hipLaunchKernelGGL(k_l4_scale<S>, g, b, 0, st(), nn, ho, (const double *)&rs->alpha[0]);
     }
@@ -965,9 +1050,9 @@ struct Solver {
       if (diag) {
         EpiL4Diag<S, F, ACC> epi{hi, ho, diag_wz<S>(*P), &rs->ome[k], probe ? hr_ : nullptr, probe ? t2 : nullptr,
                                  hn, of, inv_s};
-        launch_sell<MV, S, ACC>(lay.K, a, aval, ho, epi, st());
+        product<MV, S, ACC>(aval, (const S *)ho, epi);
       } else {
-        launch_sell<MV, S, ACC>(lay.K, a, aval, ho, EpiResid<S, S, ACC>{hr_, hi, nullptr}, st());
+        product<MV, S, ACC>(aval, (const S *)ho, EpiResid<S, S, ACC>{hr_, hi, nullptr});
         MIo<S, F> up;
         up.in = hr_;
         up.out = t2;
@@ -982,7 +1067,7 @@ struct Solver {
         prec_apply_io<S, F>(P.get(), up, st());
       }
       if (probe) {
-        product(t2, t);
+        apply_a(t2, t);
         probe_dots(t, hr_, k);
         hipLaunchKernelGGL((k_l4_update<S, F>), g, b, 0, st(), nn, (const S *)t2, (const S *)ho,
                            (const double *)&rs->alpha[k], hn, of, inv_s);
@@ -1007,11 +1092,11 @@ struct Solver {
     }
     if constexpr (std::is_same<T, float>::value) {
       if (p.variant == 0)
-        richardson<half_t, float, half_t, float>(in, out, hz, A16->as<half_t>(), *sh16);
+        richardson<half_t, float, half_t, float>(in, out, hz, A16->as<half_t>());
       else
-        richardson<float, float, double, double>(in, out, nullptr, A64->as<double>(), *sh);
+        richardson<float, float, double, double>(in, out, nullptr, A64->as<double>());
     } else {
-      richardson<double, double, double, double>(in, out, nullptr, A64->as<double>(), *sh);
+      richardson<double, double, double, double>(in, out, nullptr, A64->as<double>());
     }
   }
 
@@ -1244,12 +1329,11 @@ struct Solver {
       Cols<float, NV> c{};
       for (int k = 0; k <= j; ++k) c.p[k] = L.Vc<float>(k);
       EpiDots<float, NV> epi{w, c, j + 1, Hcol, partial<float>(), counter(0)};
-      const SellArgs a = L.mat == F3R_F16 ? argsv<half_t>() : args();
       if (L.mat == F3R_F16)
-        launch_sell<half_t, float, float>(sh16->K, a, A16->as<half_t>(), L.Zc<float>(j), epi, st(), spmv_grid);
+        product<half_t, float, float>(A16->as<half_t>(), L.Zc<float>(j), epi, spmv_grid);
       else
-        launch_sell<float, float, float>(sh->K, a, A32->as<float>(), L.Zc<float>(j), epi, st(), spmv_grid);
-      finish_dots<float>(sell_blocks(a, spmv_grid), j, Hcol);
+        product<float, float, float>(A32->as<float>(), L.Zc<float>(j), epi, spmv_grid);
+      finish_dots<float>(L.mat == F3R_F16 ? dots_blocks<half_t>() : dots_blocks<float>(), j, Hcol);
       update_launch<float, NV>(w, c, j, Hcol, j + 1 < L.m);
     });
     if (j + 1 < L.m) pending = {w, Hcol + j + 1, L.Vc<float>(j + 1)};
@@ -1290,10 +1374,9 @@ struct Solver {
     const int64_t nn = n;
     double *V = V1->as<double>(), *Z = Z1->as<double>(), *H = H1->as<double>();
     double *stat = arm_scalar(ctx.get());  // |e| for the convergence test
-    SellArgs a = args();
     EpiResidNorm<double> er{V, b_int->as<double>(), e1->as<double>(), inv1->as<double>(), stat,
                             partial<double>(), counter(3)};
-    launch_sell<double, double, double>(sh->K, a, A64->as<double>(), x_int->as<double>(), er, st(), spmv_grid);
+    product<double, double, double>(A64->as<double>(), (const double *)x_int->as<double>(), er, spmv_grid);
     hipLaunchKernelGGL(k_vscale<double>, dim3(grid()), dim3(kBlock), 0, st(), nn, V, (const double *)inv1->as<double>());
     double e = wait_scalar(ctx.get());
     // |e| / ||b||; a zero right-hand side is met only by a zero residual (its
@@ -1309,8 +1392,8 @@ struct Solver {
     for (; j < m1; ++j) {
       level2_any(V + (int64_t)j * nn, Z + (int64_t)j * nn);
       stat = arm_scalar(ctx.get());
-      launch_sell<double, double, double>(sh->K, a, A64->as<double>(), Z + (int64_t)j * nn,
-                                          EpiStore<double, double>{V + (int64_t)(j + 1) * nn, nullptr}, st());
+      product<double, double, double>(A64->as<double>(), (const double *)(Z + (int64_t)j * nn),
+                                      EpiStore<double, double>{V + (int64_t)(j + 1) * nn, nullptr});
       const int ncols = j + 1;
       // one grid row of NV columns up to 8 columns (counter slot 8), then
       // rows of 16 (slots 8.. 8 + (m1 + 15) / 16 - 1)
@@ -1447,6 +1530,9 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
     S->sh->lanes = S->sh->K;
     S->sh16->lanes = S->sh16->K;
   }
+  // the values as codes, where the layouts' K is one k_quad is built for
+  if (S->sh->K == 4 && (p.variant != 0 || S->sh16->K == 4 || S->sh16->K == 8))
+    S->quad = build_quads(ctx.get(), *S->sh, S->A64->as<double>());
   bool ident = true;
   for (int32_t r = 0; r < A.n && ident; ++r) ident = hs.perm[r] == r;
   F3R_CHECK(!nest || nest->inner != 2 || ident, F3R_ERR_UNSUPPORTED,
@@ -1482,7 +1568,8 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
   // flags bit 1 caps them like the others.
   const int64_t full = (n + kBlock - 1) / kBlock, per = (full + kDirectDots - 1) / kDirectDots;
   S->spmv_grid = (p.flags & 2) ? S->dots_grid : (int)std::min<int64_t>(per <= 2 ? (full + per - 1) / per : full, kMaxReduceGrid);
-  auto dd = [](int64_t cnt) { return dev_alloc(sizeof(double) * std::max<int64_t>(cnt, 1)); };
+  // vectors end in 64 bytes of padding: a product's windows of x reach past the last row
+  auto dd = [](int64_t cnt) { return dev_alloc(sizeof(double) * std::max<int64_t>(cnt, 1) + 64); };
   S->V1 = dd(n * (p.m1 + 1));
   S->Z1 = dd(n * p.m1);
   S->H1 = dd((int64_t)(p.m1 + 1) * p.m1);
@@ -1499,8 +1586,8 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
     L.m = m;
     // columns 64-element aligned, so the streaming kernels can use 16-byte accesses
     const int64_t ld = (n + 63) / 64 * 64;
-    L.Vbuf = dev_alloc(sizeof(E) * ld * (m + 1));
-    L.Zbuf = dev_alloc(sizeof(E) * ld * m);
+    L.Vbuf = dev_alloc(sizeof(E) * ld * (m + 1) + 64);
+    L.Zbuf = dev_alloc(sizeof(E) * ld * m + 64);
     L.wbuf = dev_alloc(sizeof(E) * ld);
     L.H = dev_alloc(sizeof(E) * (m + 1) * m);
     L.V.resize(m + 1);
@@ -1541,8 +1628,8 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
       L.s = q.store == F3R_F16 ? S->range_s : 1.f;
       L.ld = ld;
       const size_t es = q.store == F3R_F16 ? sizeof(half_t) : sizeof(float);
-      L.V = dev_alloc(es * ld * (q.m + 1));
-      L.Z = dev_alloc(es * ld * q.m);
+      L.V = dev_alloc(es * ld * (q.m + 1) + 64);
+      L.Z = dev_alloc(es * ld * q.m + 64);
       L.H = dev_alloc(sizeof(float) * (q.m + 1) * q.m);
       L.cs = dev_alloc(sizeof(float) * q.m);
       L.sn = dev_alloc(sizeof(float) * q.m);
@@ -1560,13 +1647,13 @@ Solver *solver_create(std::shared_ptr<Context> ctx, const HostCSR &A, const Prec
     int e2 = 0;
     if (p.variant == 0 && std::frexp(S->range_s, &e2) == 0.5f) {  // exact only for a power-of-two scale
       const int64_t ld = (n + 63) / 64 * 64;
-      S->L3f.Zhbuf = dev_alloc(sizeof(half_t) * ld * p.m3);
+      S->L3f.Zhbuf = dev_alloc(sizeof(half_t) * ld * p.m3 + 64);
       S->L3f.Zh.resize(p.m3);
       for (int k = 0; k < p.m3; ++k) S->L3f.Zh[k] = S->L3f.Zhbuf->as<half_t>() + (int64_t)k * ld;
     }
   }
   const size_t wsz = p.variant == 0 ? sizeof(half_t) : p.variant == 1 ? sizeof(float) : sizeof(double);
-  auto dh = [&](void) { return dev_alloc(wsz * n); };
+  auto dh = [&](void) { return dev_alloc(wsz * n + 64); };
   S->hin = dh();
   S->hout = dh();
   S->hout2 = dh();
@@ -1882,7 +1969,6 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
             "time_kernel: the Arnoldi-step kernels need the HALF variant with m3 <= 4");
   Solver *s = S->s;
   F3R_CHECK(which < 4 || s->p.depth == 0, F3R_ERR_UNSUPPORTED, "time_kernel: the Arnoldi-step kernels of the F3R nest");
-  SellArgs a = s->args(), a16 = s->argsv<half_t>();
   F3R_CHECK(s->p.variant == 0 || which == 3, F3R_ERR_UNSUPPORTED, "time_kernel: fp16/fp32 kernels need the HALF variant");
   half_t *x16 = s->hout->as<half_t>(), *y16 = s->tt->as<half_t>();
   float *x32 = s->L2f.V.empty() ? nullptr : s->L2f.V[0], *y32 = s->L2f.V.empty() ? nullptr : s->L2f.V[1];
@@ -1896,23 +1982,23 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
   auto launch = [&]() {
     switch (which) {
       case 0:  // fp16 values, fp16 x and y (the metric's fp16 SpMV)
-        launch_sell<half_t, half_t, float>(s->sh16->K, a16, s->A16->as<half_t>(), x16,
-                                           EpiStore<half_t, float>{y16, nullptr}, s->st());
+        s->product<half_t, half_t, float>(s->A16->as<half_t>(), (const half_t *)x16,
+                                          EpiStore<half_t, float>{y16, nullptr});
         by = s->sh16->algo_bytes(2, 2, 2);
         break;
       case 1:  // fp16 values, fp32 x and y (level 3)
-        launch_sell<half_t, float, float>(s->sh16->K, a16, s->A16->as<half_t>(), x32,
-                                          EpiStore<float, float>{y32, nullptr}, s->st());
+        s->product<half_t, float, float>(s->A16->as<half_t>(), (const float *)x32,
+                                         EpiStore<float, float>{y32, nullptr});
         by = s->sh16->algo_bytes(2, 4, 4);
         break;
       case 2:  // fp32 (level 2)
-        launch_sell<float, float, float>(s->sh->K, a, s->A32->as<float>(), x32,
-                                         EpiStore<float, float>{y32, nullptr}, s->st());
+        s->product<float, float, float>(s->A32->as<float>(), (const float *)x32,
+                                        EpiStore<float, float>{y32, nullptr});
         by = s->sh->algo_bytes(4, 4, 4);
         break;
       case 3:  // fp64 (outer level)
-        launch_sell<double, double, double>(s->sh->K, a, s->A64->as<double>(), x64,
-                                            EpiStore<double, double>{y64, nullptr}, s->st());
+        s->product<double, double, double>(s->A64->as<double>(), (const double *)x64,
+                                           EpiStore<double, double>{y64, nullptr});
         by = s->sh->algo_bytes(8, 8, 8);
         break;
       case 4:  // level-3 Arnoldi step j = m3 - 1: fp16 SpMV of Z_j + CGS dots with V_0..V_j, and their finish
@@ -1933,11 +2019,9 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
                                 s->template partial<float>(), s->counter(0)};
           if (!s->L3f.Zh.empty()) {
             epi.xs = 1.f / s->range_s;
-            launch_sell<half_t, half_t, float>(s->sh16->K, a16, s->A16->as<half_t>(), s->L3f.Zh[j], epi, s->st(),
-                                               s->spmv_grid);
+            s->product<half_t, half_t, float>(s->A16->as<half_t>(), (const half_t *)s->L3f.Zh[j], epi, s->spmv_grid);
           } else {
-            launch_sell<half_t, float, float>(s->sh16->K, a16, s->A16->as<half_t>(), s->L3f.Z[j], epi, s->st(),
-                                              s->spmv_grid);
+            s->product<half_t, float, float>(s->A16->as<half_t>(), (const float *)s->L3f.Z[j], epi, s->spmv_grid);
           }
           // values, Z_j gathered, w written, V_0 .. V_j read
           by += s->sh16->algo_bytes(2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * (j + 1);
@@ -1961,8 +2045,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
         EpiL4Diag<half_t, float, float> epi{s->hin->as<half_t>(), s->hout->as<half_t>(), diag_wz<half_t>(*s->P),
                                             &rs->ome[1], nullptr, nullptr, s->hout2->as<half_t>(), nullptr,
                                             1.f / s->range_s};
-        launch_sell<half_t, half_t, float>(s->sh16->K, a16, s->A16->as<half_t>(), s->hout->as<half_t>(), epi,
-                                           s->st());
+        s->product<half_t, half_t, float>(s->A16->as<half_t>(), (const half_t *)s->hout->as<half_t>(), epi);
         // values, h gathered, hin / h / (w, z) read per row, h' written
         by = s->sh16->algo_bytes(2, 2, 2) + (double)s->n * (2 + 2 + 4);
         break;

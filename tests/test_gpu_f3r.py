@@ -374,3 +374,56 @@ def test_solve_variants_match_oracle(ctx, variant, kind):
     assert res.is_solved and ro.is_solved
     assert _true_res(A, xv.download(), b) <= 1e-8
     assert abs(res.res_iter - ro.res_iter) <= max(1, int(np.ceil(0.1 * ro.res_iter))), (res.res_iter, ro.res_iter)
+
+
+def _banded(n, offs, vals, seed):
+    """rows coupled at the given offsets, values drawn from a few numbers"""
+    import scipy.sparse as sp
+    import f3r_amd as F
+    rng = np.random.default_rng(seed)
+    M = sp.diags([np.full(n, 3.0) if o == 0 else rng.choice(vals, n - abs(o)) for o in offs], offs, format="csr")
+    M.sort_indices()
+    return F.CSR(n, M.indptr, M.indices, M.data)
+
+
+@pytest.mark.parametrize("kind", ["27pt", "27pt-ragged", "7pt", "7pt-dominant", "runs", "32 slots", "16 values",
+                                  "17 values"])
+@pytest.mark.parametrize("variant", ["half", "float", "double"])
+def test_value_codes(ctx, kind, variant):
+    """matrices of few distinct values are summed from 4-bit codes, four rows a
+    lane (from 131072 rows): the innermost level's bits are those of the
+    int32-index layout, which has no codes; level 3 agrees to its reductions"""
+    import f3r_amd as F
+    if kind == "27pt":
+        A = F.CSR.stencil27(64, 64, 33, beta=0.5)
+    elif kind == "27pt-ragged":
+        A = F.CSR.stencil27(53, 51, 49, beta=0.5)  # n not a multiple of 4
+    elif kind == "7pt":
+        A = F.CSR.dominant(7, 67, 45, 44, margin=1.0)
+    elif kind == "7pt-dominant":
+        A = F.CSR.dominant(7, 52, 51, 50, margin=0.7)
+    else:
+        n = 131072 + 77
+        offs, vals = {"runs": ([-700, -302, -301, -2, -1, 0, 1, 2, 3, 4, 301, 900], [-.25, .125]),
+                      "32 slots": (list(range(-40, -24)) + list(range(-7, 9)), [-.03, .02, .01]),
+                      "16 values": ([-300, -1, 0, 1, 300], np.linspace(-.5, .5, 14)),
+                      "17 values": ([-300, -1, 0, 1, 300], np.linspace(-.5, .5, 15))}[kind]
+        A = _banded(n, offs, vals, 5)
+    if kind[:2] in ("27", "7p"):
+        F.algorithm.scaling(A)
+    dt = {"half": "f16", "float": "f32", "double": "f64"}[variant]
+    P = F.SDAINV(A, 0.1, 1.0, dt, ctx=ctx)
+    b = F.uniform(A.n, -1.0, 1.0, seed=3)
+    vin = F.vector.from_numpy(ctx, b / np.linalg.norm(b))
+    out = {}
+    for index in (1, 0):
+        S = F.F3R(ctx, A, P, variant=variant, index=index, K=0 if index else 4, use_graph=False, device_build=True)
+        for level in (4, 3):
+            v = F.vector(ctx, "f64", A.n)
+            print(f"value codes {kind} {variant} index={index} level={level}", flush=True)
+            S.level_apply(level, vin, v)
+            out[index, level] = v.download()
+    assert np.array_equal(out[1, 4], out[0, 4])
+    # fp32 dots of 4 columns in another order (2^-24 n^0.5 at most), then fp16 roundings that may flip
+    tol = {"half": 2e-3, "float": 1e-4, "double": 1e-10}[variant]
+    assert np.linalg.norm(out[1, 3] - out[0, 3]) <= tol * np.linalg.norm(out[0, 3])
