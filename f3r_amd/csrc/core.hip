@@ -225,11 +225,16 @@ __global__ __launch_bounds__(1024) void k_bj_trsv_u(const int32_t *__restrict__ 
 // four waves and a barrier per batch.  Records read level by level from
 // global memory, four levels ahead, took 87 us at 64^3 / 112 blocks: 0.43 us
 // a level, the memory latency over four.
-constexpr uint16_t kBjNone = 0xffff;  // column of an unused entry
+// The wave's own instructions then count (about 40 a batch), so a record is
+// ready to use: byte offsets into xs, the end of a batch in bit 0 of the row's
+// (found by a ballot, no batch sizes to fetch), unused entries reading a zero
+// slot behind xs with value 0 (s + -0 = s: no test), and L's records carrying
+// dinv = 1, so L and U are one stream.  Measured at 64^3 / 112 blocks: 43 us
+// with batch sizes, tests and two streams.
 template <class S, int R> struct alignas(8) BjRecord {
-  uint16_t row, col[R];
+  uint16_t row, col[R];  // byte offsets into xs; bit 0 of row: last of its batch (one wave) or no row (four)
   S val[R];
-  S dinv;  // U only
+  S dinv;
 };
 // records per segment: a power of two of batches, about 16 KB
 template <class S, int R, int NW> constexpr int bj_segment() {
@@ -237,32 +242,29 @@ template <class S, int R, int NW> constexpr int bj_segment() {
   while (2 * m * (int)sizeof(BjRecord<S, R>) <= 16384) m *= 2;
   return m;
 }
-struct BjSide {
-  const void *rec;        // segments of all blocks
-  const int32_t *seg;     // block b: segments seg[b] .. seg[b + 1] - 1
-  const int32_t *bat;     // block b: batch sizes cnt[bat[b]] .. cnt[bat[b + 1] - 1]
-  const uint16_t *cnt;    // (64 entries of zero padding at the end)
-};
 // Barrier for LDS traffic only: this wave's LDS operations complete, then
 // s_barrier.  __syncthreads() would also wait for every outstanding global
 // load (its release fence), i.e. for the segment on its way.  The memory
 // clobber keeps the compiler from moving LDS accesses across it.
 __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Solves the block's stream of nseg segments at `src`; the first two are in
+// the ring already.  NW = 1: batches end where a record says so.  NW = 4: a
+// batch is 256 records (levels padded by records without a row).
 template <class S, int R, int NW>
-__device__ __forceinline__ void bj_side(const BjSide &sd, bool upper, S *xs, unsigned char *ring) {
+__device__ __forceinline__ void bj_solve(const BjRecord<S, R> *__restrict__ srec, int nseg, int nrec, S *xs,
+                                         unsigned char *ring) {
   using A = typename Acc<S>::type;
   using Rec = BjRecord<S, R>;
   using Unit = typename std::conditional<sizeof(Rec) % 16 == 0, u32x4, u32x2>::type;
   constexpr int SR = bj_segment<S, R, NW>(), T = 64 * NW;
   constexpr int kUnits = SR * (int)sizeof(Rec) / (int)sizeof(Unit) / T;  // of one thread
   static_assert(SR * sizeof(Rec) == (size_t)kUnits * T * sizeof(Unit), "a segment is whole units per thread");
-  const int tid = threadIdx.x, lane = tid & (kWave - 1);
-  const int32_t s0 = sd.seg[blockIdx.x], nseg = sd.seg[blockIdx.x + 1] - s0;
-  const int32_t b0 = sd.bat[blockIdx.x], nb = sd.bat[blockIdx.x + 1] - b0;
-  const Unit *src = reinterpret_cast<const Unit *>(static_cast<const Rec *>(sd.rec) + (int64_t)s0 * SR);
+  const int tid = threadIdx.x;
+  const Unit *src = reinterpret_cast<const Unit *>(srec);
   Unit *const lring = reinterpret_cast<Unit *>(ring);
   const Rec *const recs = reinterpret_cast<const Rec *>(ring);
+  char *const xb = reinterpret_cast<char *>(xs);
   Unit stage[kUnits];
   auto issue = [&](int k) {
     if (k < nseg) {
@@ -276,26 +278,27 @@ __device__ __forceinline__ void bj_side(const BjSide &sd, bool upper, S *xs, uns
       for (int p = 0; p < kUnits; ++p) lring[((k & 1) * kUnits + p) * T + tid] = stage[p];
     }
   };
-  issue(0);
-  commit(0);
-  issue(1);
-  commit(1);
   issue(2);
-  if constexpr (NW > 1) lds_barrier();
-  int32_t cnts = sd.cnt[b0 + lane], cntn = sd.cnt[b0 + kWave + lane];  // the next 64 batch sizes ahead
   int k = 0, t0 = 0;
   Rec rec = recs[tid];
-  for (int b = 0; b < nb; ++b) {
-    const int c = __builtin_amdgcn_readlane(cnts, b & (kWave - 1));
+  while (t0 < nrec) {
     const Rec cur = rec;
-    // xs of this batch: every read is issued before the first is used
-    const int32_t row = tid < c ? cur.row : 0;
-    A s = to_acc(xs[row]);
+    // every read of xs is issued before the first is used
+    const int row = cur.row & ~1;
+    A s = to_acc(*reinterpret_cast<const S *>(xb + row));
     S xv[R];
 #pragma unroll
-    for (int q = 0; q < R; ++q) xv[q] = xs[tid < c && cur.col[q] != kBjNone ? cur.col[q] : 0];
+    for (int q = 0; q < R; ++q) xv[q] = *reinterpret_cast<const S *>(xb + cur.col[q]);
+    bool active;
+    if constexpr (NW == 1) {
+      const int c = __builtin_ctzll(__ballot((cur.row & 1) != 0)) + 1;
+      active = tid < c;
+      t0 += c;
+    } else {
+      active = (cur.row & 1) == 0;
+      t0 += T;
+    }
     // the next batch's records, past the segment boundary if it is crossed
-    t0 += c;
     if (t0 >= (k + 1) * SR) {
       if constexpr (NW > 1) lds_barrier();  // segment k is read by every wave
       commit(k + 2);
@@ -304,24 +307,36 @@ __device__ __forceinline__ void bj_side(const BjSide &sd, bool upper, S *xs, uns
       if constexpr (NW > 1) lds_barrier();
     }
     rec = recs[(t0 + tid) & (2 * SR - 1)];
-    if (((b + 1) & (kWave - 1)) == 0) {
-      cnts = cntn;
-      cntn = b + 1 + kWave < nb ? sd.cnt[b0 + b + 1 + kWave + lane] : 0;
-    }
 #pragma unroll
-    for (int q = 0; q < R; ++q)
-      if (cur.col[q] != kBjNone) s = fma_<A>(-to_acc(cur.val[q]), to_acc(xv[q]), s);
-    if (tid < c) xs[row] = upper ? cvt<S>(s * to_acc(cur.dinv)) : cvt<S>(s);
+    for (int q = 0; q < R; ++q) s = fma_<A>(-to_acc(cur.val[q]), to_acc(xv[q]), s);
+    if (active) *reinterpret_cast<S *>(xb + row) = cvt<S>(s * to_acc(cur.dinv));
     if constexpr (NW > 1) lds_barrier();
   }
 }
 
 template <class S, class F, int R, int NW>
-__global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, BjSide L, BjSide U, MIo<S, F> io) {
+__global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, const BjRecord<S, R> *__restrict__ recs,
+                                                   const int2 *__restrict__ blk, MIo<S, F> io) {
   extern __shared__ __align__(16) unsigned char bj_smem[];
   constexpr int kRing = 2 * bj_segment<S, R, NW>() * (int)sizeof(BjRecord<S, R>);
   S *xs = reinterpret_cast<S *>(bj_smem + kRing);
   const int32_t r0 = blockIdx.x * bsz, nr = n - r0 < bsz ? n - r0 : bsz;
+  // the block's stream: first segment and records (its segments: whole ones)
+  constexpr int SR = bj_segment<S, R, NW>();
+  const int2 bk = blk[blockIdx.x];
+  const int nseg = (bk.y + SR - 1) / SR;
+  const BjRecord<S, R> *srec = recs + (int64_t)bk.x * SR;
+  // the first two segments (the second slot never stays unwritten: any lane
+  // may read a record there before its batch's end is known)
+  {
+    using Unit = u32x2;
+    constexpr int kSegUnits = SR * (int)sizeof(BjRecord<S, R>) / (int)sizeof(Unit);
+    const Unit *src = reinterpret_cast<const Unit *>(srec);
+    Unit *dst = reinterpret_cast<Unit *>(bj_smem);
+#pragma unroll 8
+    for (int i = threadIdx.x; i < 2 * kSegUnits; i += kBlock) dst[i] = src[nseg > 1 || i < kSegUnits ? i : i - kSegUnits];
+  }
+  if (threadIdx.x == 0) xs[bsz] = S(0);  // the zero slot
   // all waves move the vector, 8 rows in flight each
   if (io.raw) {
     const MEntry<S, F> en(io);
@@ -351,11 +366,7 @@ __global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, BjSid
     }
   }
   __syncthreads();
-  if (threadIdx.x < 64 * NW) {
-    bj_side<S, R, NW>(L, false, xs, bj_smem);
-    if constexpr (NW > 1) lds_barrier();
-    bj_side<S, R, NW>(U, true, xs, bj_smem);
-  }
+  if (threadIdx.x < 64 * NW) bj_solve<S, R, NW>(srec, nseg, bk.y, xs, bj_smem);
   __syncthreads();
   const MExit<S, F> mo(io);
   for (int32_t i = threadIdx.x; i < nr; i += kBlock) mo.put(r0 + i, xs[i], mo.pre(r0 + i));
@@ -992,22 +1003,20 @@ static void group_by_block(const std::vector<int32_t> &rows, const std::vector<i
   bstart[nb] = (int32_t)blptr.size();
 }
 
-// Record stream of a triangular factor for k_bj_lds: the rows of each block
-// in the grouped order (`brows`, block by block and level by level), padded to
-// whole segments, and the sizes of the batches (at most 64 NW rows of one
-// level) they are solved in.
-struct BjStream {
-  std::vector<unsigned char> rec;
-  std::vector<int32_t> seg, bat;
-  std::vector<uint16_t> cnt;
+// Record streams of the triangular factors for k_bj_lds: the rows of each
+// block in the grouped order (`brows`, block by block and level by level), L's
+// and then U's, padded to whole segments.  A batch is at most 64 NW rows of
+// one level (NW = 4: padded to 256 records).
+struct BjRows {
+  const HostCSR &M;
+  const std::vector<int32_t> &brows, &blptr, &bstart;
 };
 template <class S, int R, int NW>
-static void bj_stream(const HostCSR &M, bool upper, const std::vector<int32_t> &brows,
-                      const std::vector<int32_t> &blptr, const std::vector<int32_t> &bstart, int32_t bsz,
-                      BjStream &out) {
+static void bj_stream(const BjRows &L, const BjRows &U, int32_t bsz, std::vector<BjRecord<S, R>> &rec,
+                      std::vector<int2> &blk) {
   using Rec = BjRecord<S, R>;
-  constexpr int SR = bj_segment<S, R, NW>();
-  const int32_t nb = (int32_t)bstart.size() - 1;
+  constexpr int SR = bj_segment<S, R, NW>(), T = 64 * NW;
+  const int32_t nb = (int32_t)L.bstart.size() - 1;
   auto bits = [](double v) {
     S s;
     if constexpr (std::is_same<S, half_t>::value) {
@@ -1018,41 +1027,61 @@ static void bj_stream(const HostCSR &M, bool upper, const std::vector<int32_t> &
     }
     return s;
   };
-  out.seg.assign(1, 0);
-  out.bat.assign(1, 0);
-  for (int32_t b = 0; b < nb; ++b) {
-    const int32_t rows = blptr[bstart[b + 1] - 1] - blptr[bstart[b]];
-    out.seg.push_back(out.seg.back() + (rows + SR - 1) / SR);
-  }
+  // unused entries read the zero slot behind xs, or with a vector of exactly
+  // 64 KB, behind which an offset does not reach, the row's own element (the
+  // same sum while that is finite)
+  const bool slot = bsz * sizeof(S) < 65536;
+  const uint16_t zero = (uint16_t)(slot ? bsz * sizeof(S) : 0);
   Rec none{};
-  for (int q = 0; q < R; ++q) none.col[q] = kBjNone;
-  std::vector<Rec> rec((size_t)out.seg.back() * SR, none);
+  none.row = 1;
+  for (int q = 0; q < R; ++q) none.col[q] = zero;
+  // records of a block
+  auto count = [&](const BjRows &s, int32_t b) {
+    int32_t c = 0;
+    for (int32_t q = s.bstart[b]; q + 1 < s.bstart[b + 1]; ++q) {
+      const int32_t w = s.blptr[q + 1] - s.blptr[q];
+      c += NW == 1 ? w : (w + T - 1) / T * T;
+    }
+    return c;
+  };
+  int32_t seg = 0;
   for (int32_t b = 0; b < nb; ++b) {
-    Rec *r = rec.data() + (size_t)out.seg[b] * SR;
+    const int32_t c = count(L, b) + count(U, b);
+    blk.push_back(int2{seg, c});
+    seg += (c + SR - 1) / SR;
+  }
+  rec.assign((size_t)seg * SR, none);
+  for (int32_t b = 0; b < nb; ++b) {
+    Rec *r = rec.data() + (size_t)blk[b].x * SR;
     const int32_t base = b * bsz;
-    for (int32_t t = blptr[bstart[b]]; t < blptr[bstart[b + 1] - 1]; ++t, ++r) {
-      const int32_t i = brows[t];
-      r->row = (uint16_t)(i - base);
-      int c = 0;
-      auto put = [&](int32_t k) {
-        r->col[c] = (uint16_t)(M.idx[k] - base);
-        r->val[c++] = bits(M.val[k]);
-      };
-      if (upper) {
-        for (int32_t k = M.rptr[i + 1] - 1; k > M.rptr[i]; --k) put(k);
-        r->dinv = bits(1. / M.val[M.rptr[i]]);
-      } else {
-        for (int32_t k = M.rptr[i]; k < M.rptr[i + 1] - 1; ++k) put(k);
+    for (int side = 0; side < 2; ++side) {
+      const BjRows &s = side == 0 ? L : U;
+      const HostCSR &M = s.M;
+      for (int32_t q = s.bstart[b]; q + 1 < s.bstart[b + 1]; ++q) {
+        const int32_t t1 = s.blptr[q + 1];
+        int32_t w = 0;
+        for (int32_t t = s.blptr[q]; t < t1; ++t, ++r, ++w) {
+          const int32_t i = s.brows[t];
+          r->row = (uint16_t)((i - base) * sizeof(S)) | (NW == 1 && (t + 1 == t1 || w % 64 == 63) ? 1 : 0);
+          if (!slot)
+            for (int k = 0; k < R; ++k) r->col[k] = (uint16_t)((i - base) * sizeof(S));
+          int c = 0;
+          auto put = [&](int32_t k) {
+            r->col[c] = (uint16_t)((M.idx[k] - base) * sizeof(S));
+            r->val[c++] = bits(M.val[k]);
+          };
+          if (side == 1) {
+            for (int32_t k = M.rptr[i + 1] - 1; k > M.rptr[i]; --k) put(k);
+            r->dinv = bits(1. / M.val[M.rptr[i]]);
+          } else {
+            for (int32_t k = M.rptr[i]; k < M.rptr[i + 1] - 1; ++k) put(k);
+            r->dinv = bits(1.);
+          }
+        }
+        if (NW > 1) r += (T - w % T) % T;
       }
     }
-    for (int32_t q = bstart[b]; q + 1 < bstart[b + 1]; ++q)
-      for (int32_t w = blptr[q + 1] - blptr[q]; w > 0; w -= 64 * NW) out.cnt.push_back((uint16_t)std::min(w, 64 * NW));
-    out.bat.push_back((int32_t)out.cnt.size());
   }
-  // the kernel reads batch sizes 64 at a time, two groups ahead
-  out.cnt.insert(out.cnt.end(), 2 * kWave, 0);
-  out.rec.resize(rec.size() * sizeof(Rec));
-  std::memcpy(out.rec.data(), rec.data(), out.rec.size());
 }
 
 // f(S tag, R, NW) for the preconditioner's record shape
@@ -1204,8 +1233,9 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
         maxe = std::max(maxe, L.rptr[i + 1] - L.rptr[i] - 1);
         maxe = std::max(maxe, U.rptr[i + 1] - U.rptr[i] - 1);
       }
-      const size_t lds = (size_t)maxrows * dtype_size(P->dtype);
-      if (maxe <= 16 && lds <= kBjLdsBytes) {
+      const size_t es = dtype_size(P->dtype), lds = (size_t)(bsz + 1) * es;
+      // byte offsets in xs are 16-bit numbers
+      if (maxe <= 16 && maxrows > 0 && (size_t)bsz * es <= kBjLdsBytes) {
         P->bj_R = maxe <= 3 ? 3 : maxe <= 7 ? 7 : 16;
         // one wave up to 128 rows per level on average (two batches); wider
         // levels on four waves with a barrier per batch
@@ -1214,22 +1244,17 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
         bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
           using S = decltype(s);
           constexpr int R = decltype(r)::value, NW = decltype(w)::value;
-          for (int side = 0; side < 2; ++side) {
-            BjStream bt;
-            if (side == 0) bj_stream<S, R, NW>(L, false, lbr, lbl, lbs, bsz, bt);
-            else bj_stream<S, R, NW>(U, true, ubr, ubl, ubs, bsz, bt);
-            Prec::BjData &d = P->bj[side];
-            auto up = [&](DevPtr &p, const void *h, size_t bytes) {
-              p = dev_alloc(std::max<size_t>(bytes, 16));
-              if (bytes) F3R_HIP(hipMemcpyAsync(p->p, h, bytes, hipMemcpyHostToDevice, c->stream));
-            };
-            up(d.rec, bt.rec.data(), bt.rec.size());
-            up(d.cnt, bt.cnt.data(), 2 * bt.cnt.size());
-            up(d.seg, bt.seg.data(), 4 * bt.seg.size());
-            up(d.bat, bt.bat.data(), 4 * bt.bat.size());
-            F3R_HIP(hipStreamSynchronize(c->stream));
-          }
-          P->bj_lds = lds + 2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>);
+          std::vector<BjRecord<S, R>> rec;
+          std::vector<int2> blk;
+          bj_stream<S, R, NW>({L, lbr, lbl, lbs}, {U, ubr, ubl, ubs}, bsz, rec, blk);
+          auto up = [&](DevPtr &p, const void *h, size_t bytes) {
+            p = dev_alloc(std::max<size_t>(bytes, 16));
+            if (bytes) F3R_HIP(hipMemcpyAsync(p->p, h, bytes, hipMemcpyHostToDevice, c->stream));
+          };
+          up(P->bj_rec, rec.data(), sizeof(rec[0]) * rec.size());
+          up(P->bj_blk, blk.data(), sizeof(int2) * blk.size());
+          F3R_HIP(hipStreamSynchronize(c->stream));
+          P->bj_lds = (lds + 2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>) + 15) / 16 * 16;
           // up to 154 KB of the CU's 160 KB
           F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, typename Acc<S>::type, R, NW>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->bj_lds));
@@ -1250,14 +1275,12 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
 
 // the fused block-Jacobi solve
 template <class S, class F> static void bj_apply(Prec *P, const MIo<S, F> &io, hipStream_t st) {
-  auto side = [&](const Prec::BjData &d) {
-    return BjSide{d.rec->p, d.seg->as<int32_t>(), d.bat->as<int32_t>(), d.cnt->as<uint16_t>()};
-  };
   const int32_t blocks = P->bj_blocks, bsz = (P->n + blocks - 1) / blocks;
   bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
     if constexpr (std::is_same<decltype(s), S>::value)
       hipLaunchKernelGGL((k_bj_lds<S, F, decltype(r)::value, decltype(w)::value>), dim3(P->bj_groups), dim3(kBlock),
-                         P->bj_lds, st, P->n, bsz, side(P->bj[0]), side(P->bj[1]), io);
+                         P->bj_lds, st, P->n, bsz, P->bj_rec->as<BjRecord<S, decltype(r)::value>>(),
+                         P->bj_blk->as<int2>(), io);
   });
 }
 

@@ -33,12 +33,11 @@ struct Prec {
   int32_t bj_blocks = 0, bj_groups = 0;
   DevPtr lb_rows, lb_ptr, lb_start, ub_rows, ub_ptr, ub_start;
   // fused L+U solve with the block's vector in LDS (bj_R entries per record;
-  // 0: not used), on bj_waves wavefronts: the record streams of L and U
+  // 0: not used), on bj_waves wavefronts: the record streams and, per block,
+  // its first segment and its records
   int32_t bj_R = 0, bj_waves = 1;
   size_t bj_lds = 0;
-  struct BjData {
-    DevPtr rec, seg, bat, cnt;
-  } bj[2];
+  DevPtr bj_rec, bj_blk;
   // its kernels take the entry themselves (no vector for its result needed)
   bool has_fused_entry() const { return kind == 0 || bj_R != 0; }
 };

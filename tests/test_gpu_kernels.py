@@ -265,6 +265,8 @@ def _coupled(n, dists, seed):
     (40007, 32, [300, 301, 302, 303, 304]),
     (40009, 37, [290 + k for k in range(16)]),
     (4096, 64, []),                            # diagonal blocks: one level
+    (32 * 16384, 32, [128]),                   # a block's fp32 vector fills 64 KB exactly
+    (32 * 8192, 32, [1, 90]),                  # its fp64 vector
     (127, 64, [1])])                           # 2 rows a block, 1 in the last
 @pytest.mark.parametrize("dtype", ["f64", "f32", "f16"])
 def test_bjilu0_record_streams(ctx, n, blocks, dists, dtype):
