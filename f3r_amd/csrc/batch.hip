@@ -29,6 +29,7 @@
 #include "common.hpp"
 #include "device.hpp"
 #include "internal.hpp"
+#include "quad.hpp"
 #include "sell_kernel.hpp"
 
 namespace f3r {
@@ -438,90 +439,149 @@ __global__ __launch_bounds__(kBlock) void k_b_l4_update(const half_t *__restrict
 // per-lane byte offset is the row's, the chunk offset and the copy's stride
 // ride in the scalar offset (no per-lane address arithmetic per gather).
 template <class V, class X, class ACC, int K, int NR, class Y>
+__device__ __forceinline__ void sell_mr_row(const SellArgs &a, int r, const V *__restrict__ val,
+                                            const X *__restrict__ x, int64_t nx, const int32_t *__restrict__ cshift,
+                                            const int32_t *__restrict__ cstride, Y *__restrict__ y,
+                                            const Y *__restrict__ b, const int32_t *__restrict__ cseg,
+                                            const float *__restrict__ ysc) {
+  typedef const __attribute__((address_space(4))) int32_t *const_i32;
+  const int s = r >> a.log2C;
+  const int j = r - (s << a.log2C);
+  const int C = 1 << a.log2C;
+  const int rem = a.n - (s << a.log2C);
+  const int tc = rem < C ? rem : C;
+  const int su = __builtin_amdgcn_readfirstlane(s);  // C >= 64: one chunk per wavefront
+  const int cw = a.cwidth[su];
+  const int groups = chunk_groups(cw);
+  const int32_t shift = cshift[su], stride = cstride[su];
+  int64_t pos = (int64_t)a.cptr[su] + (int64_t)j * K;
+  const int64_t step = (int64_t)tc * K;
+  ACC acc[NR];
+#pragma unroll
+  for (int c = 0; c < NR; ++c) acc[c] = 0;
+  const int64_t vr = (int64_t)r + shift;
+  const int32_t start = a.iptr ? a.iptr[su] : 0;
+  if (a.iptr && start < 0) {
+    const const_i32 off = (const_i32)(a.coff + (-start - 1));
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)((uintptr_t)x - (uintptr_t)a.off_bias * sizeof(X)), (short)0,
+        (int)((nx + a.off_bias) * (int64_t)sizeof(X)), kBufferWord3);
+    const int vo = (int)(vr * (int64_t)sizeof(X));
+    const int bias = a.off_bias, cst = stride * (int)sizeof(X);
+#pragma unroll 2
+    for (int g = 0; g < groups; ++g, pos += step) {
+      const Pack<V, K> pv = load_pack<V, K>(val + pos);
+      X xv[K][NR];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int so = (off[g * K + k] + bias) * (int)sizeof(X);
+#pragma unroll
+        for (int c = 0; c < NR; ++c) xv[k][c] = buffer_gather<X>(rs, vo, so + c * cst);
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int c = 0; c < NR; ++c) acc[c] = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xv[k][c]), acc[c]);
+    }
+    if constexpr (K >= 2) {
+      if (cw & kHalfTail) {  // the half group (K / 2 slots per row, rows consecutive)
+        constexpr int H = K / 2;
+        const Pack<V, H> pv = load_pack<V, H>(val + ((int64_t)a.cptr[su] + (int64_t)groups * step + (int64_t)j * H));
+        X xv[H][NR];
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+          const int so = (off[groups * K + k] + bias) * (int)sizeof(X);
+#pragma unroll
+          for (int c = 0; c < NR; ++c) xv[k][c] = buffer_gather<X>(rs, vo, so + c * cst);
+        }
+#pragma unroll
+        for (int k = 0; k < H; ++k)
+#pragma unroll
+          for (int c = 0; c < NR; ++c) acc[c] = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xv[k][c]), acc[c]);
+      }
+    }
+  } else {
+    const int32_t *__restrict__ ip = a.idx + (a.iptr ? (int64_t)start : (int64_t)a.cptr[su]) + (int64_t)j * K;
+    for (int g = 0; g < groups; ++g, pos += step, ip += step) {
+      const Pack<V, K> pv = load_pack<V, K>(val + pos);
+      const Pack<int32_t, K> pi = load_pack<int32_t, K>(ip);
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int64_t col = (int64_t)pi.v[k] + shift;
+#pragma unroll
+        for (int c = 0; c < NR; ++c)
+          acc[c] = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(x[col + (int64_t)c * stride]), acc[c]);
+      }
+    }
+  }
+  // ysc: x held z * s (fp16 storage, s a power of two per segment), so
+  // y = sum * (1/s) is the sum over z exactly
+#pragma unroll
+  for (int c = 0; c < NR; ++c) {
+    const int64_t o = vr + (int64_t)c * stride;
+    const ACC sum = ysc ? acc[c] * (ACC)ysc[cseg[su] + c] : acc[c];
+    y[o] = b ? cvt<Y>((ACC)to_acc(b[o]) - sum) : cvt<Y>(sum);
+  }
+}
+
+template <class V, class X, class ACC, int K, int NR, class Y>
 __global__ __launch_bounds__(kBlock) void k_sell_mr(SellArgs a, const V *__restrict__ val, const X *__restrict__ x,
                                                     int64_t nx, const int32_t *__restrict__ cshift,
                                                     const int32_t *__restrict__ cstride, Y *__restrict__ y,
                                                     const Y *__restrict__ b, const int32_t *__restrict__ cseg,
                                                     const float *__restrict__ ysc) {
-  typedef const __attribute__((address_space(4))) int32_t *const_i32;
-  for (int r = xcd_block() * kBlock + threadIdx.x; r < a.n; r += gridDim.x * kBlock) {
-    const int s = r >> a.log2C;
-    const int j = r - (s << a.log2C);
-    const int C = 1 << a.log2C;
-    const int rem = a.n - (s << a.log2C);
-    const int tc = rem < C ? rem : C;
-    const int su = __builtin_amdgcn_readfirstlane(s);  // C >= 64: one chunk per wavefront
-    const int cw = a.cwidth[su];
-    const int groups = chunk_groups(cw);
-    const int32_t shift = cshift[su], stride = cstride[su];
-    int64_t pos = (int64_t)a.cptr[su] + (int64_t)j * K;
-    const int64_t step = (int64_t)tc * K;
-    ACC acc[NR];
-#pragma unroll
-    for (int c = 0; c < NR; ++c) acc[c] = 0;
-    const int64_t vr = (int64_t)r + shift;
-    const int32_t start = a.iptr ? a.iptr[su] : 0;
-    if (a.iptr && start < 0) {
-      const const_i32 off = (const_i32)(a.coff + (-start - 1));
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-          (void *)((uintptr_t)x - (uintptr_t)a.off_bias * sizeof(X)), (short)0,
-          (int)((nx + a.off_bias) * (int64_t)sizeof(X)), kBufferWord3);
-      const int vo = (int)(vr * (int64_t)sizeof(X));
-      const int bias = a.off_bias, cst = stride * (int)sizeof(X);
-#pragma unroll 2
-      for (int g = 0; g < groups; ++g, pos += step) {
-        const Pack<V, K> pv = load_pack<V, K>(val + pos);
-        X xv[K][NR];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          const int so = (off[g * K + k] + bias) * (int)sizeof(X);
-#pragma unroll
-          for (int c = 0; c < NR; ++c) xv[k][c] = buffer_gather<X>(rs, vo, so + c * cst);
-        }
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-#pragma unroll
-          for (int c = 0; c < NR; ++c) acc[c] = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xv[k][c]), acc[c]);
-      }
-      if constexpr (K >= 2) {
-        if (cw & kHalfTail) {  // the half group (K / 2 slots per row, rows consecutive)
-          constexpr int H = K / 2;
-          const Pack<V, H> pv = load_pack<V, H>(val + ((int64_t)a.cptr[su] + (int64_t)groups * step + (int64_t)j * H));
-          X xv[H][NR];
-#pragma unroll
-          for (int k = 0; k < H; ++k) {
-            const int so = (off[groups * K + k] + bias) * (int)sizeof(X);
-#pragma unroll
-            for (int c = 0; c < NR; ++c) xv[k][c] = buffer_gather<X>(rs, vo, so + c * cst);
-          }
-#pragma unroll
-          for (int k = 0; k < H; ++k)
-#pragma unroll
-            for (int c = 0; c < NR; ++c) acc[c] = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(xv[k][c]), acc[c]);
-        }
-      }
-    } else {
-      const int32_t *__restrict__ ip = a.idx + (a.iptr ? (int64_t)start : (int64_t)a.cptr[su]) + (int64_t)j * K;
-      for (int g = 0; g < groups; ++g, pos += step, ip += step) {
-        const Pack<V, K> pv = load_pack<V, K>(val + pos);
-        const Pack<int32_t, K> pi = load_pack<int32_t, K>(ip);
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          const int64_t col = (int64_t)pi.v[k] + shift;
-#pragma unroll
-          for (int c = 0; c < NR; ++c)
-            acc[c] = fma_<ACC>((ACC)to_acc(pv.v[k]), (ACC)to_acc(x[col + (int64_t)c * stride]), acc[c]);
-        }
-      }
+  for (int r = xcd_block() * kBlock + threadIdx.x; r < a.n; r += gridDim.x * kBlock)
+    sell_mr_row<V, X, ACC, K, NR, Y>(a, r, val, x, nx, cshift, cstride, y, b, cseg, ysc);
+}
+
+// The same product by value codes (quad.hpp), where every system has few
+// distinct values: a lane takes four matrix rows of NR copies, so codes are
+// decoded once for all copies and x is read in windows.  The gathers and their
+// latency, not the bytes, were the plain product's cost (0.32 of the memory
+// rate for 4 copies).
+template <class V, class X, class ACC, int K, int NR, class Y>
+__global__ __launch_bounds__(kBlock) void k_quad_mr(SellArgs a, QuadArgs qa, const V *__restrict__ val,
+                                                    const X *__restrict__ x, int64_t nx,
+                                                    const int32_t *__restrict__ cshift,
+                                                    const int32_t *__restrict__ cstride, Y *__restrict__ y,
+                                                    const Y *__restrict__ b, const int32_t *__restrict__ cseg,
+                                                    const float *__restrict__ ysc) {
+  __shared__ QuadPair<V> lut[256];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  if ((int)blockIdx.x < qa.nfb) {  // blocks that are not coded: a chunk per wave
+    const int c = (int)blockIdx.x * kWavesPerBlock + wave;
+    if (c < qa.nfc) {
+      const int r = qa.fchunk[c] * 64 + lane;
+      if (r < a.n) sell_mr_row<V, X, ACC, K, NR, Y>(a, r, val, x, nx, cshift, cstride, y, b, cseg, ysc);
     }
-    // ysc: x held z * s (fp16 storage, s a power of two per segment), so
-    // y = sum * (1/s) is the sum over z exactly
+    return;
+  }
+  const int blk = quad_block<V>(a, qa, lut);
+  if ((int64_t)blk * kQuadBlock >= a.n) return;
+  const int4 e = qa.blk[blk];
+  const int tab = __builtin_amdgcn_readfirstlane(e.x), unit = __builtin_amdgcn_readfirstlane(e.y);
+  if (tab < 0) return;
+  // the block's rows lie in one tile: one shift and stride (its first chunk's)
+  const int su = blk * (kQuadBlock / 64);
+  const int32_t shift = cshift[su], stride = cstride[su], seg = cseg[su];
+  const int64_t vr = (int64_t)blk * kQuadBlock + 4 * lane + shift;
+  V4<Y> bv[NR];
+  if (b)
 #pragma unroll
-    for (int c = 0; c < NR; ++c) {
-      const int64_t o = vr + (int64_t)c * stride;
-      const ACC sum = ysc ? acc[c] * (ACC)ysc[cseg[su] + c] : acc[c];
-      y[o] = b ? cvt<Y>((ACC)to_acc(b[o]) - sum) : cvt<Y>(sum);
+    for (int c = 0; c < NR; ++c) bv[c] = ld4(b + vr + (int64_t)c * stride);
+  ACC acc[NR][4];
+  quad_rows<NR, V, X, ACC>(qa, tab, unit, lut, quad_rsrc<X>(x, nx, qa.bias), (int)(vr * (int64_t)sizeof(X)),
+                           stride * (int)sizeof(X), acc);
+#pragma unroll
+  for (int c = 0; c < NR; ++c) {
+    const ACC sc = ysc ? (ACC)ysc[seg + c] : (ACC)1;
+    V4<Y> o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const ACC sum = ysc ? acc[c][q] * sc : acc[c][q];
+      o.v[q] = b ? cvt<Y>((ACC)to_acc(bv[c].v[q]) - sum) : cvt<Y>(sum);
     }
+    st4(y + vr + (int64_t)c * stride, o);
   }
 }
 
@@ -802,6 +862,7 @@ struct BatchSolver {
   std::vector<int32_t> nrow;
   DevPtr bseg, sb0, snb, scale, iscale;
   std::shared_ptr<SellShared> sh, sh16;
+  std::shared_ptr<QuadSet> quad;  // NR > 1: value codes, a table per system (null: too many values)
   DevPtr A64, A32, A16;
   // NR > 1: each system's matrix is stored once for its NR right-hand sides
   // (chunk -> vector-row shift and copy stride, per layout)
@@ -891,6 +952,14 @@ struct BatchSolver {
           return;
         }
       }
+      if constexpr (K >= 4) {
+        if (quad) {
+          const QuadArgs qa = quad->template args<V>();
+          hipLaunchKernelGGL((k_quad_mr<V, X, ACC, K, R, Y>), dim3(quad_blocks(a, qa)), dim3(kBlock), 0, st(), a, qa,
+                             val, x, (int64_t)N, shf, str, y, b, (const int32_t *)cseg->as<int32_t>(), ysc);
+          return;
+        }
+      }
       hipLaunchKernelGGL((k_sell_mr<V, X, ACC, K, R, Y>), g, dim3(kBlock), 0, st(), a, val, x, (int64_t)N, shf, str, y,
                          b, (const int32_t *)cseg->as<int32_t>(), ysc);
     };
@@ -910,8 +979,9 @@ struct BatchSolver {
 
   template <class T> void alloc_level(BLevel<T> &L, int m) {
     L.m = m;
-    L.V = dev_alloc(sizeof(T) * N * (m + 1));
-    L.Z = dev_alloc(sizeof(T) * N * m);
+    // vectors end in 64 bytes of padding: a product's windows of x reach past the last row
+    L.V = dev_alloc(sizeof(T) * N * (m + 1) + 64);
+    L.Z = dev_alloc(sizeof(T) * N * m + 64);
     L.H = dev_alloc(sizeof(T) * nseg * L.hs());
     L.cs = dev_alloc(sizeof(T) * nseg * m);
     L.sn = dev_alloc(sizeof(T) * nseg * m);
@@ -1405,6 +1475,7 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
       B->sh16 = upload_sell_shared(c, h16, false);
       B->A16 = upload_sell_values(c, h16, F3R_F16);
     }
+    if (NR > 1 && !B->lanes && K >= 4 && K16 >= 4) B->quad = build_quads(c, *B->sh, B->A64->as<double>(), moff);
     // k_sell_mr gathers x (fp64 at most) of offset chunks through a buffer
     // resource whose size and byte offsets are 32-bit
     const int64_t bias = std::max(B->sh->off_bias, B->sh16->off_bias);
@@ -1478,9 +1549,9 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
       pow2 = pow2 && std::frexp(v, &e) == 0.5f;
     }
     B->zh = NR > 1 && pow2;
-    if (B->zh) B->Zh3 = dev_alloc(sizeof(half_t) * N * p.m3);
+    if (B->zh) B->Zh3 = dev_alloc(sizeof(half_t) * N * p.m3 + 64);
   }
-  auto hv = [&]() { return dev_alloc(sizeof(half_t) * N); };
+  auto hv = [&]() { return dev_alloc(sizeof(half_t) * N + 64); };
   B->hin = hv();
   B->hout = hv();
   B->hout2 = hv();
@@ -1489,7 +1560,7 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
   B->tt = hv();
   B->t2 = hv();
   B->b_int = dev_alloc(sizeof(double) * N);
-  B->x_int = dev_alloc(sizeof(double) * N);
+  B->x_int = dev_alloc(sizeof(double) * N + 64);
   B->partial = dev_alloc(sizeof(double) * (int64_t)B->G * (p.m1 + 1 + 16));
   B->rows = up32(B->nrow);
   B->alloc_pinned();

@@ -17,6 +17,8 @@
 // solver.hip.
 #pragma once
 
+#include <utility>
+
 #include "sell_kernel.hpp"
 
 namespace f3r {
@@ -37,10 +39,12 @@ template <class V> struct QuadPair {
   V v[2];
 };
 struct QuadArgs {
-  const int2 *__restrict__ blk;      // per 256-row block: table (-1: not coded), first 16-byte unit of its codes
+  // per 256-row block: table (-1: not coded), first 16-byte unit of its codes,
+  // value table (one per system of a batch; the blocks of a workgroup share it)
+  const int4 *__restrict__ blk;
   const u32x4 *__restrict__ codes;   // unit w * 64 + l of a block: code word w of the rows of lane l
   const QuadTab *__restrict__ tabs;
-  const void *__restrict__ lut;      // 256 pairs of V
+  const void *__restrict__ lut;      // 256 pairs of V per value table
   const int32_t *__restrict__ fchunk;  // 64-row chunks of the blocks that are not coded
   int32_t nfb, nfc;                  // workgroups that take them (four each), and their number
   int32_t bias;                      // > -(smallest offset), even
@@ -53,20 +57,20 @@ template <class X, int N> struct QuadWindow {
     if constexpr (sizeof(L) == 16) return __builtin_bit_cast(L, __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0));
     else return __builtin_bit_cast(L, __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0));
   }
-  __device__ __forceinline__ QuadWindow(__amdgpu_buffer_rsrc_t rs, int vo, int u, int bias) {
+  __device__ __forceinline__ QuadWindow(__amdgpu_buffer_rsrc_t rs, int vo, int u, int bias, int cs) {
     constexpr int kBytes = N * (int)sizeof(X);
     if constexpr (sizeof(X) == 2) {
       // dword-aligned loads: one element more when u is odd, dropped by a
       // funnel shift (the parity is the wave's: r0 is a multiple of four)
       const int odd = u & 1;
-      const u32x4 d = load<u32x4>(rs, vo, (u - odd + bias) * 2);
+      const u32x4 d = load<u32x4>(rs, vo, (u - odd + bias) * 2 + cs);
       const unsigned sh = odd ? 16u : 0u;
       uint32_t w[3] = {__builtin_amdgcn_alignbit(d[1], d[0], sh), __builtin_amdgcn_alignbit(d[2], d[1], sh),
                        __builtin_amdgcn_alignbit(d[3], d[2], sh)};
       static_assert(N <= 6, "eight halves are loaded");
       __builtin_memcpy(v, w, kBytes);
     } else {
-      const int so = (u + bias) * (int)sizeof(X);
+      const int so = (u + bias) * (int)sizeof(X) + cs;
 #pragma unroll
       for (int b = 0; b + 16 <= kBytes; b += 16) {
         const u32x4 d = load<u32x4>(rs, vo, so + b);
@@ -81,44 +85,60 @@ template <class X, int N> struct QuadWindow {
   }
 };
 
-// acc[q] += the run's M slots (codes of slots T .. T + M - 1 of each row)
-template <int T, int M, class V, class X, class ACC, int N, class Pair>
-__device__ __forceinline__ void quad_run(const QuadWindow<X, N> &w, const Pair &pair, ACC (&acc)[4]) {
+// the windows of one run in NR copies of the vector, `cs` bytes apart
+template <class X, int N, int NR> struct QuadWindows {
+  QuadWindow<X, N> w[NR];
+  template <int... C>
+  __device__ __forceinline__ QuadWindows(__amdgpu_buffer_rsrc_t rs, int vo, int u, int bias, int cs,
+                                         std::integer_sequence<int, C...>)
+      : w{QuadWindow<X, N>(rs, vo, u, bias, C * cs)...} {}
+  __device__ __forceinline__ QuadWindows(__amdgpu_buffer_rsrc_t rs, int vo, int u, int bias, int cs)
+      : QuadWindows(rs, vo, u, bias, cs, std::make_integer_sequence<int, NR>()) {}
+};
+
+// acc[c][q] += the run's M slots (codes of slots T .. T + M - 1 of each row)
+template <int T, int M, class X, class ACC, int N, int NR, class Pair>
+__device__ __forceinline__ void quad_run(const QuadWindows<X, N, NR> &w, const Pair &pair, ACC (&acc)[NR][4]) {
 #pragma unroll
   for (int j = 0; j < M; ++j)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      acc[q] = fma_<ACC>((ACC)to_acc(pair(q, T + j)), (ACC)to_acc(w.v[q + j]), acc[q]);
+    for (int q = 0; q < 4; ++q) {
+      const ACC v = (ACC)to_acc(pair(q, T + j));
+#pragma unroll
+      for (int c = 0; c < NR; ++c) acc[c][q] = fma_<ACC>(v, (ACC)to_acc(w.w[c].v[q + j]), acc[c][q]);
+    }
 }
 
-// sums of rows r0 .. r0 + 3 of a coded block
-template <class V, class X, class ACC>
+// sums of rows r0 .. r0 + 3 of a coded block, for NR copies of x whose rows
+// lie cs bytes apart; rs: a buffer resource over x - bias, vo: the byte offset
+// of row r0
+template <int NR, class V, class X, class ACC>
 __device__ __forceinline__ void quad_rows(const QuadArgs &qa, int tab, int unit, const QuadPair<V> *lut,
-                                          const X *__restrict__ x, int n, int r0, ACC (&acc)[4]) {
+                                          __amdgpu_buffer_rsrc_t rs, int vo, int cs, ACC (&acc)[NR][4]) {
   typedef const __attribute__((address_space(4))) QuadTab *const_tab;
   const const_tab tb = (const_tab)(qa.tabs + tab);
   const int lane = threadIdx.x & (kWave - 1);
   const u32x4 *__restrict__ cp = qa.codes + unit + lane;
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)((uintptr_t)x - (uintptr_t)qa.bias * sizeof(X)), (short)0,
-      (int)(((int64_t)n + qa.bias) * (int64_t)sizeof(X)) + 64, kBufferWord3);
-  // lanes past the last row read where the last row's lane does
-  const int vo = (r0 < n ? r0 : (n - 1) & ~3) * (int)sizeof(X);
+  const int bias = qa.bias;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) acc[q] = 0;
+  for (int c = 0; c < NR; ++c)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[c][q] = 0;
+  using W6 = QuadWindows<X, 6, NR>;
+  using W4 = QuadWindows<X, 4, NR>;
   if (tb->kind == kQuad27) {
     u32x4 c[4];
 #pragma unroll
     for (int w = 0; w < 4; ++w) c[w] = cp[w * kWave];
     auto pair = [&](int q, int t) { return lut[(c[t / 8][q] >> (8 * (t / 2 % 4))) & 255u].v[t & 1]; };
-    // three lines of a plane at a time: their nine windows in flight together
+    // three lines of a plane at a time: their windows in flight together
     auto plane = [&](auto pt) {
       constexpr int P = decltype(pt)::value;
-      const QuadWindow<X, 6> w0(rs, vo, tb->u[3 * P], qa.bias), w1(rs, vo, tb->u[3 * P + 1], qa.bias),
-          w2(rs, vo, tb->u[3 * P + 2], qa.bias);
-      quad_run<9 * P, 3, V>(w0, pair, acc);
-      quad_run<9 * P + 3, 3, V>(w1, pair, acc);
-      quad_run<9 * P + 6, 3, V>(w2, pair, acc);
+      const W6 w0(rs, vo, tb->u[3 * P], bias, cs), w1(rs, vo, tb->u[3 * P + 1], bias, cs),
+          w2(rs, vo, tb->u[3 * P + 2], bias, cs);
+      quad_run<9 * P, 3>(w0, pair, acc);
+      quad_run<9 * P + 3, 3>(w1, pair, acc);
+      quad_run<9 * P + 6, 3>(w2, pair, acc);
     };
     plane(std::integral_constant<int, 0>());
     plane(std::integral_constant<int, 1>());
@@ -126,31 +146,51 @@ __device__ __forceinline__ void quad_rows(const QuadArgs &qa, int tab, int unit,
   } else if (tb->kind == kQuad7) {
     const u32x4 c = cp[0];
     auto pair = [&](int q, int t) { return lut[(c[q] >> (8 * (t / 2))) & 255u].v[t & 1]; };
-    const QuadWindow<X, 4> w0(rs, vo, tb->u[0], qa.bias), w1(rs, vo, tb->u[1], qa.bias), w3(rs, vo, tb->u[3], qa.bias),
-        w4(rs, vo, tb->u[4], qa.bias);
-    const QuadWindow<X, 6> w2(rs, vo, tb->u[2], qa.bias);
-    quad_run<0, 1, V>(w0, pair, acc);
-    quad_run<1, 1, V>(w1, pair, acc);
-    quad_run<2, 3, V>(w2, pair, acc);
-    quad_run<5, 1, V>(w3, pair, acc);
-    quad_run<6, 1, V>(w4, pair, acc);
+    const W4 w0(rs, vo, tb->u[0], bias, cs), w1(rs, vo, tb->u[1], bias, cs), w3(rs, vo, tb->u[3], bias, cs),
+        w4(rs, vo, tb->u[4], bias, cs);
+    const W6 w2(rs, vo, tb->u[2], bias, cs);
+    quad_run<0, 1>(w0, pair, acc);
+    quad_run<1, 1>(w1, pair, acc);
+    quad_run<2, 3>(w2, pair, acc);
+    quad_run<5, 1>(w3, pair, acc);
+    quad_run<6, 1>(w4, pair, acc);
   } else {
     int t = 0;
     u32x4 c = cp[0];
     for (int i = 0; i < tb->nruns; ++i) {
-      const QuadWindow<X, 6> w(rs, vo, tb->u[i], qa.bias);
+      const W6 w(rs, vo, tb->u[i], bias, cs);
       const int m = tb->m[i];
 #pragma unroll
       for (int j = 0; j < 3; ++j)
         if (j < m) {
           if ((t & 7) == 0) c = cp[(t >> 3) * kWave];
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            acc[q] = fma_<ACC>((ACC)to_acc(lut[(c[q] >> (4 * (t & 7))) & 15u].v[0]), (ACC)to_acc(w.v[q + j]), acc[q]);
+          for (int q = 0; q < 4; ++q) {
+            const ACC v = (ACC)to_acc(lut[(c[q] >> (4 * (t & 7))) & 15u].v[0]);
+#pragma unroll
+            for (int k = 0; k < NR; ++k) acc[k][q] = fma_<ACC>(v, (ACC)to_acc(w.w[k].v[q + j]), acc[k][q]);
+          }
           ++t;
         }
     }
   }
+}
+// nx elements of x behind a fictitious x - bias, and the padding behind them
+template <class X>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t quad_rsrc(const X *x, int64_t nx, int bias) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)((uintptr_t)x - (uintptr_t)bias * sizeof(X)), (short)0,
+                                           (int)((nx + bias) * (int64_t)sizeof(X)) + 64, kBufferWord3);
+}
+// the 256-row block of this wave, and its workgroup's value table into LDS
+template <class V>
+__device__ __forceinline__ int quad_block(const SellArgs &a, const QuadArgs &qa, QuadPair<V> *lut) {
+  static_assert(kBlock == 256, "a thread per pair of the table");
+  // XCD k takes the k-th contiguous eighth of the rows (xcd_block)
+  const int g = (int)gridDim.x - qa.nfb, b0 = (int)blockIdx.x - qa.nfb;
+  const int b = g % kXcds ? b0 : b0 % kXcds * (g / kXcds) + b0 / kXcds;
+  lut[threadIdx.x] = static_cast<const QuadPair<V> *>(qa.lut)[qa.blk[b * kWavesPerBlock].z * 256 + threadIdx.x];
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(b * kWavesPerBlock + (int)threadIdx.x / kWave);
 }
 
 // An epilogue (sell_kernel.hpp) may also provide, for four consecutive rows of
@@ -177,33 +217,30 @@ __global__ __launch_bounds__(kBlock) void k_quad(SellArgs a, QuadArgs qa, const 
       }
     }
   } else {
-    static_assert(kBlock == 256, "a thread per pair of the table");
-    lut[threadIdx.x] = static_cast<const QuadPair<V> *>(qa.lut)[threadIdx.x];
-    __syncthreads();
-    // XCD k takes the k-th contiguous eighth of the rows (xcd_block)
-    const int g = (int)gridDim.x - qa.nfb, b0 = (int)blockIdx.x - qa.nfb;
-    const int b = g % kXcds ? b0 : b0 % kXcds * (g / kXcds) + b0 / kXcds;
-    const int blk = __builtin_amdgcn_readfirstlane(b * kWavesPerBlock + wave);
+    const int blk = quad_block<V>(a, qa, lut);
     if ((int64_t)blk * kQuadBlock < a.n) {
-      const int2 e = qa.blk[blk];
+      const int4 e = qa.blk[blk];
       const int tab = __builtin_amdgcn_readfirstlane(e.x), unit = __builtin_amdgcn_readfirstlane(e.y);
       if (tab >= 0) {
         const int r0 = blk * kQuadBlock + 4 * lane;
-        ACC acc[4];
+        const __amdgpu_buffer_rsrc_t rs = quad_rsrc<X>(x, a.n, qa.bias);
+        // lanes past the last row read where the last row's lane does
+        const int vo = (r0 < a.n ? r0 : (a.n - 1) & ~3) * (int)sizeof(X);
+        ACC acc[1][4];
         bool done = false;
         if constexpr (HasRow4<Epi>::value) {
           if (vec && (blk + 1) * kQuadBlock <= a.n) {
             const typename Epi::Pre4 p = epi.pre4(r0);
-            quad_rows<V, X, ACC>(qa, tab, unit, lut, x, a.n, r0, acc);
-            epi.row4(r0, acc, p, st);
+            quad_rows<1, V, X, ACC>(qa, tab, unit, lut, rs, vo, 0, acc);
+            epi.row4(r0, acc[0], p, st);
             done = true;
           }
         }
         if (!done) {
-          quad_rows<V, X, ACC>(qa, tab, unit, lut, x, a.n, r0, acc);
+          quad_rows<1, V, X, ACC>(qa, tab, unit, lut, rs, vo, 0, acc);
 #pragma unroll
           for (int q = 0; q < 4; ++q)
-            if (r0 + q < a.n) epi.row(r0 + q, acc[q], epi.pre(r0 + q), st);
+            if (r0 + q < a.n) epi.row(r0 + q, acc[0][q], epi.pre(r0 + q), st);
         }
       }
     }
@@ -230,14 +267,17 @@ struct QuadSet {
   int32_t nfb = 0, nfc = 0, bias = 0;
   template <class V> QuadArgs args() const {
     const DevPtr &l = sizeof(V) == 8 ? lut64 : sizeof(V) == 4 ? lut32 : lut16;
-    return {blk->as<int2>(), codes->as<u32x4>(), tabs->as<QuadTab>(), l->p, fchunk->as<int32_t>(), nfb, nfc, bias};
+    return {blk->as<int4>(), codes->as<u32x4>(), tabs->as<QuadTab>(), l->p, fchunk->as<int32_t>(), nfb, nfc, bias};
   }
 };
 // Fewer rows than this leave k_quad's waves (256 rows each) too few for the
 // GPU's 1024 SIMDs to hide their latency.
 constexpr int32_t kQuadMinRows = 1 << 17;
 // null when the matrix has more than 16 distinct values (0 among them), its
-// chunks are not 64 rows of offset form, or it has too few rows
-std::shared_ptr<QuadSet> build_quads(Context *c, const SellShared &sh, const double *val64);
+// chunks are not 64 rows of offset form, or it has too few rows.  systems: the
+// first rows of the diagonal blocks with value tables of their own (multiples
+// of 1024; empty: one table), the last entry the end
+std::shared_ptr<QuadSet> build_quads(Context *c, const SellShared &sh, const double *val64,
+                                     const std::vector<int64_t> &systems = {});
 
 }  // namespace f3r

@@ -397,3 +397,33 @@ def test_lockstep_many_small_segments():
     worst = max(_true_res(A, x.download(), b) for A, x, b in zip(As, xv, bs))
     assert worst <= 1e-8, worst
     ctx.close()
+
+
+@pytest.mark.parametrize("nrhs", [2, 4])
+@pytest.mark.parametrize("sizes", [[(7, 48), (27, 33), (7, 21), (27, 17)],   # 131072 matrix rows and more: coded
+                                   [(27, 51), (7, 16)]])
+def test_lockstep_value_codes(nrhs, sizes):
+    """systems of few distinct values each, one matrix for several right-hand
+    sides: products by value codes, with a table per system, give the bits of
+    the int32-index layout, which has none"""
+    import f3r_amd as F
+    ctx = F.Context(0)
+    As, Ps, bs = [], [], []
+    for s, (npts, m) in enumerate(sizes):
+        A = F.CSR.dominant(npts, m, m + 1, m - 1, margin=0.6 + 0.3 * s)
+        F.algorithm.scaling(A)
+        P = F.SDAINV(A, 0.1, 1.0, "f16", ctx=ctx)
+        for r in range(nrhs):
+            As.append(A)
+            Ps.append(P)
+            bs.append(F.uniform(A.n, -1.0, 1.0, seed=100 * s + r))
+    out = []
+    for kw in ({"index": 1}, {"index": 0, "K": 4}):
+        print(f"lockstep value codes nrhs={nrhs} sizes={sizes} {kw}", flush=True)
+        B = F.Batch(ctx, As, Ps, m=(100, 3, 2, 2), **kw)
+        xs = [F.vector(ctx, "f64", A.n).fill(0.0) for A in As]
+        res = B.solve([F.vector.from_numpy(ctx, b) for b in bs], xs)
+        assert all(r.is_solved for r in res)
+        out.append([x.download() for x in xs])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
