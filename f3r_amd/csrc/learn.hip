@@ -841,8 +841,7 @@ int f3r_mlp_grad_zero(f3r_mlp m) {
   F3R_API_BEGIN
   F3R_CHECK(m, F3R_ERR_ARG, "null argument");
   Context *c = m->m->ctx.get();
-  F3R_HIP(hipMemsetAsync(m->m->grad->p, 0, 4 * kNParams, c->stream));
-  sync(c);
+  F3R_HIP(hipMemsetAsync(m->m->grad->p, 0, 4 * kNParams, c->stream));  // ordered before the stream's later work
   F3R_API_END
 }
 
