@@ -377,27 +377,34 @@ __global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, const
 // vectors (4 rows per lane with VEC: every array 4-element aligned).
 template <class S, class F, bool VEC>
 __global__ __launch_bounds__(kBlock) void k_m_diag(int64_t n, DiagWZ<S> d, MIo<S, F> io) {
+  const int64_t gid = blockIdx.x * (int64_t)kBlock + threadIdx.x, gstride = (int64_t)gridDim.x * kBlock;
+  const int64_t n4 = VEC ? n / 4 : 0;
+  V4<F> v;
+  V4<S> w4, z4;
+  auto rows = [&](int64_t q) {
+    v = ld4(io.raw + 4 * q);
+    if constexpr (std::is_same<S, half_t>::value) {
+      const V4<uint32_t> wz = ld4(d.wz + 4 * q);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const typename DiagWZ<S>::V e = DiagWZ<S>::unpack(wz.v[c]);
+        w4.v[c] = e.w;
+        z4.v[c] = e.z;
+      }
+    } else {
+      w4 = ld4(d.w + 4 * q);
+      z4 = ld4(d.z + 4 * q);
+    }
+  };
+  // the first rows' loads before the norm is added up
+  if (VEC && gid < n4) rows(gid);
   const MEntry<S, F> en(io);
   const MExit<S, F> mo(io);
-  const int64_t gid = blockIdx.x * (int64_t)kBlock + threadIdx.x, gstride = (int64_t)gridDim.x * kBlock;
   int64_t i0 = 0;
   if constexpr (VEC) {
-    const int64_t n4 = n / 4;
     for (int64_t q = gid; q < n4; q += gstride) {
-      V4<F> v = ld4(io.raw + 4 * q);
-      V4<S> h, o, w4, z4;
-      if constexpr (std::is_same<S, half_t>::value) {
-        const V4<uint32_t> wz = ld4(d.wz + 4 * q);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const typename DiagWZ<S>::V e = DiagWZ<S>::unpack(wz.v[c]);
-          w4.v[c] = e.w;
-          z4.v[c] = e.z;
-        }
-      } else {
-        w4 = ld4(d.w + 4 * q);
-        z4 = ld4(d.z + 4 * q);
-      }
+      if (q != gid) rows(q);
+      V4<S> h, o;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         v.v[c] = en.norm(v.v[c]);
