@@ -98,9 +98,10 @@ __device__ __forceinline__ int64_t tile_row(int q) { return (int64_t)blockIdx.x 
 // 8- or 16-byte access per vector and group; segments and vectors start on
 // tile boundaries, so every group is aligned)
 constexpr int kQuads = kRows / 4;
-__device__ __forceinline__ int64_t tile_quad(int q) {
-  return (int64_t)blockIdx.x * kTile + ((int64_t)threadIdx.x + (int64_t)q * kBlock) * 4;
+__device__ __forceinline__ int64_t tile_quad(int q, int b) {
+  return (int64_t)b * kTile + ((int64_t)threadIdx.x + (int64_t)q * kBlock) * 4;
 }
+__device__ __forceinline__ int64_t tile_quad(int q) { return tile_quad(q, (int)blockIdx.x); }
 
 // block partial sums of <w, V_k> for the NV columns of blockIdx.y (k < ncols):
 // partial[k * gridDim.x + block]
@@ -641,7 +642,8 @@ __global__ __launch_bounds__(kBlock) void k_sell_mr_lanes(SellArgs a, const V *_
 // An SDAINV factor split by row kind: a row whose only entry is its diagonal
 // is an elementwise product (dval), any other row is a CSR row summed in
 // column order with fp32 accumulation, as the SELL SpMV sums it; dval holds
-// an fp16 NaN for those rows.  M = Z W^T x runs as two launches:
+// an fp16 NaN for those rows.  M = Z W^T x is k_b_m where all rows are short,
+// else two launches:
 //   k_b_mw: t = W^T x for every row (tile blocks: diagonal rows; row blocks:
 //           the CSR rows), and y = Z t for the rows where Z is diagonal;
 //   k_b_mz: y = Z t for the CSR rows of Z.  They read t of other rows: t of
@@ -737,52 +739,140 @@ struct FacArgs {
   int32_t nr;
 };
 
+// the rows of tile block b that are diagonal in both factors
+__device__ __forceinline__ void b_m_tile(int b, const MIn &xin, const half_t *__restrict__ wd,
+                                         const half_t *__restrict__ zd, const int64_t *__restrict__ dsh,
+                                         const int32_t *__restrict__ bseg, const MOut &o) {
+  // every load of the thread's rows first, then the stores (a branch
+  // between a row's loads would keep one row's loads in flight at a time)
+  const int seg = bseg[b];
+  const float w = o.weight(seg);
+  const float sc = xin.in ? xin.sc[seg] : 0.f, iv = xin.iv(seg);
+  const int64_t sh = dsh[seg];
+  V4<half_t> xi[kQuads], dw[kQuads], dz[kQuads], hov[kQuads];
+#pragma unroll
+  for (int q = 0; q < kQuads; ++q) {
+    const int64_t i = tile_quad(q, b);
+    if (xin.in) {
+      const V4<float> f = ld4(xin.in + i);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) xi[q].v[c] = cvt<half_t>((f.v[c] * iv) * sc);
+    } else {
+      xi[q] = ld4(xin.x + i);
+    }
+    dw[q] = ld4(wd + i + sh);
+    dz[q] = ld4(zd + i + sh);
+    if (o.mode >= 2) hov[q] = ld4(o.ho + i);
+  }
+#pragma unroll
+  for (int q = 0; q < kQuads; ++q) {
+    const int64_t i = tile_quad(q, b);
+    if (xin.in) st4(xin.hin + i, xi[q]);
+    bool plain = true;  // all four rows diagonal in W and Z
+    V4<half_t> yv;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      plain = plain && !is_nan16(dw[q].v[c]) && !is_nan16(dz[q].v[c]);
+      const half_t ti = cvt<half_t>(to_acc(dw[q].v[c]) * to_acc(xi[q].v[c]));
+      yv.v[c] = cvt<half_t>(to_acc(dz[q].v[c]) * to_acc(ti));
+    }
+    if (plain) {
+      o.put4(i, seg, yv, o.mode >= 2 ? hov[q] : yv, w);
+      continue;
+    }
+    // a CSR row of W or Z is not a tile block's
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (!is_nan16(dw[q].v[c]) && !is_nan16(dz[q].v[c])) o.put(i + c, seg, yv.v[c], hov[q].v[c], w);
+  }
+}
+
+// A row that is not diagonal in W or Z, both of at most kMRow entries a row:
+// y_i = sum_g z_g fp16(sum_u w_gu x_c(gu)), g over Z's row i and u over W's
+// row of Z's column g (one entry where that row is diagonal; one g where Z's
+// row i is).  Slot u of group g of row r is at wc / wv[(g * nr + r) * kMRow +
+// u], column -1 where there is none; meta: {vector row of the first copy, its
+// segment, the copies' stride, groups}.
+constexpr int kMRow = 4;
+struct MRows {
+  const int4 *__restrict__ meta;
+  const int4 *__restrict__ wc;
+  const half_t *__restrict__ wv, *__restrict__ z;
+  int32_t nr;
+};
+
+// y = M x in one launch, where the rows of W and Z have at most kMRow entries:
+// blocks below GR take rows of `R`, one thread for the NR copies of a row, and
+// work t = W^T x of their columns out again; the rest are tile blocks.  The
+// second launch for Z's rows and the indexes read once per copy were a third
+// of M's time; the row blocks come first, so that their chain of three loads
+// runs beside the tile blocks' streaming, which is what bounds M then.
+// 5.93 M rows, 4 copies, 9% of the rows not diagonal: 30.3 -> 17.8 us.
+template <int NR, bool IN>
+__global__ __launch_bounds__(kBlock) void k_b_m(MIn xin, MRows R, int GR, const half_t *__restrict__ wd,
+                                                const half_t *__restrict__ zd, const int64_t *__restrict__ dsh,
+                                                const int32_t *__restrict__ bseg, MOut o) {
+  if ((int)blockIdx.x >= GR) {
+    b_m_tile((int)blockIdx.x - GR, xin, wd, zd, dsh, bseg, o);
+    return;
+  }
+  const int32_t r = (int32_t)blockIdx.x * kBlock + threadIdx.x;
+  if (r >= R.nr) return;
+  const int4 m = R.meta[r];
+  int4 wc[kMRow];
+  V4<half_t> wv[kMRow];
+#pragma unroll
+  for (int g = 0; g < kMRow; ++g) {
+    wc[g] = R.wc[(int64_t)g * R.nr + r];
+    wv[g] = ld4(R.wv + ((int64_t)g * R.nr + r) * kMRow);
+  }
+  const V4<half_t> z = ld4(R.z + (int64_t)r * kMRow);
+  float iv[NR], sc[NR], acc[NR];
+#pragma unroll
+  for (int c = 0; c < NR; ++c) {
+    iv[c] = IN ? xin.iv(m.y + c) : 1.f;
+    sc[c] = IN ? xin.sc[m.y + c] : 1.f;
+    acc[c] = 0.f;
+  }
+#pragma unroll
+  for (int g = 0; g < kMRow; ++g) {
+    if (g >= m.w) break;
+    const int32_t col[kMRow] = {wc[g].x, wc[g].y, wc[g].z, wc[g].w};
+    typename std::conditional<IN, float, half_t>::type xv[kMRow][NR];
+#pragma unroll
+    for (int u = 0; u < kMRow; ++u)
+#pragma unroll
+      for (int c = 0; c < NR; ++c) {
+        const int64_t q = (int64_t)(col[u] < 0 ? m.x : col[u]) + (int64_t)c * m.z;
+        if constexpr (IN)
+          xv[u][c] = xin.in[q];
+        else
+          xv[u][c] = xin.x[q];
+      }
+#pragma unroll
+    for (int c = 0; c < NR; ++c) {
+      float t = 0.f;
+#pragma unroll
+      for (int u = 0; u < kMRow; ++u) {
+        half_t xu;
+        if constexpr (IN)
+          xu = cvt<half_t>((xv[u][c] * iv[c]) * sc[c]);
+        else
+          xu = xv[u][c];
+        if (col[u] >= 0) t = fma_<float>(to_acc(wv[g].v[u]), to_acc(xu), t);
+      }
+      acc[c] = fma_<float>(to_acc(z.v[g]), to_acc(cvt<half_t>(t)), acc[c]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NR; ++c) o.put((int64_t)m.x + (int64_t)c * m.z, m.y + c, cvt<half_t>(acc[c]));
+}
+
 __global__ __launch_bounds__(kBlock) void k_b_mw(MIn xin, FacArgs W, const half_t *__restrict__ zd,
                                                  const int64_t *__restrict__ dsh, half_t *__restrict__ t, int G,
                                                  const int32_t *__restrict__ bseg, MOut o) {
   if ((int)blockIdx.x < G) {
-    // every load of the thread's rows first, then the stores (a branch
-    // between a row's loads would keep one row's loads in flight at a time)
-    const int seg = bseg[blockIdx.x];
-    const float w = o.weight(seg);
-    const float sc = xin.in ? xin.sc[seg] : 0.f, iv = xin.iv(seg);
-    const int64_t sh = dsh[seg];
-    V4<half_t> xi[kQuads], dw[kQuads], dz[kQuads], hov[kQuads];
-#pragma unroll
-    for (int q = 0; q < kQuads; ++q) {
-      const int64_t i = tile_quad(q);
-      if (xin.in) {
-        const V4<float> f = ld4(xin.in + i);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) xi[q].v[c] = cvt<half_t>((f.v[c] * iv) * sc);
-      } else {
-        xi[q] = ld4(xin.x + i);
-      }
-      dw[q] = ld4(W.d + i + sh);
-      dz[q] = ld4(zd + i + sh);
-      if (o.mode >= 2) hov[q] = ld4(o.ho + i);
-    }
-#pragma unroll
-    for (int q = 0; q < kQuads; ++q) {
-      const int64_t i = tile_quad(q);
-      if (xin.in) st4(xin.hin + i, xi[q]);
-      bool plain = true;  // all four rows diagonal in W and Z
-      V4<half_t> yv;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        plain = plain && !is_nan16(dw[q].v[c]) && !is_nan16(dz[q].v[c]);
-        const half_t ti = cvt<half_t>(to_acc(dw[q].v[c]) * to_acc(xi[q].v[c]));
-        yv.v[c] = cvt<half_t>(to_acc(dz[q].v[c]) * to_acc(ti));
-      }
-      if (plain) {
-        o.put4(i, seg, yv, o.mode >= 2 ? hov[q] : yv, w);
-        continue;
-      }
-      // a CSR row of W is the row blocks' (and a CSR row of Z k_b_mz's)
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (!is_nan16(dw[q].v[c]) && !is_nan16(dz[q].v[c])) o.put(i + c, seg, yv.v[c], hov[q].v[c], w);
-    }
+    b_m_tile((int)blockIdx.x, xin, W.d, zd, dsh, bseg, o);
     return;
   }
   const int32_t r = (int32_t)(blockIdx.x - G) * kBlock + threadIdx.x;
@@ -871,6 +961,10 @@ struct BatchSolver {
   bool lanes = false;
   DevPtr csh, cst, csh16, cst16;
   Factor16 W, Z;
+  // the rows that are not diagonal, where k_b_m takes them (mr_nr < 0: k_b_mw and k_b_mz do)
+  DevPtr mr_meta, mr_wc, mr_wv, mr_z;
+  int32_t mr_nr = -1;
+  int mr_copies = 1;
   DevPtr dsh;  // per segment: vector row -> row of the factor diagonals
   DevPtr cseg;  // NR > 1: per chunk, the segment of its first copy
   // level 3's Z as the fp16 Richardson output h (Z = h / s exactly, s the
@@ -1031,6 +1125,23 @@ struct BatchSolver {
   // y = M x with M = Z W^T (ainv.hpp:110-114): W^T first, then Z; x given
   // by `xin`, y consumed by `o`
   void precond(const MIn &xin, const MOut &o) {
+    if (mr_nr >= 0) {
+      const MRows R{mr_meta->as<int4>(), mr_wc->as<int4>(), mr_wv->as<half_t>(), mr_z->as<half_t>(), mr_nr};
+      const int gr = (mr_nr + kBlock - 1) / kBlock;
+      auto go = [&](auto nt) {
+        constexpr int NC = decltype(nt)::value;
+        hipLaunchKernelGGL((xin.in ? k_b_m<NC, true> : k_b_m<NC, false>), dim3(G + gr), dim3(kBlock), 0, st(), xin, R,
+                           gr, (const half_t *)W.dval->as<half_t>(), (const half_t *)Z.dval->as<half_t>(),
+                           (const int64_t *)dsh->as<int64_t>(), (const int32_t *)bs(), o);
+      };
+      if (mr_copies == 4)
+        go(std::integral_constant<int, 4>());
+      else if (mr_copies == 2)
+        go(std::integral_constant<int, 2>());
+      else
+        go(std::integral_constant<int, 1>());
+      return;
+    }
     half_t *t = tmp->as<half_t>();
     const int gw = (W.nr + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(k_b_mw, dim3(G + gw), dim3(kBlock), 0, st(), xin, fac(W), (const half_t *)Z.dval->as<half_t>(),
@@ -1490,17 +1601,28 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
   std::vector<int64_t> dshift(nseg, 0);
   if (share_d)
     for (int s = 0; s < nseg; ++s) dshift[s] = moff[s / NR] - B->off[s];
-  auto factor = [&](const std::vector<const HostCSR *> &parts) {
-    HostCSR M = concat(parts, B->off, N);
+  const HostCSR Wm = concat(pw, B->off, N), Zm = concat(pz, B->off, N);
+  auto plain = [](const HostCSR &M, int32_t i) { return M.rptr[i + 1] - M.rptr[i] == 1 && M.idx[M.rptr[i]] == i; };
+  auto csr_row = [&](const HostCSR &M, int32_t i) { return M.rptr[i + 1] > M.rptr[i] && !plain(M, i); };
+  // k_b_m works t of a Z row's columns out again for each row: that is up to
+  // kMRow^2 gathers a row where the two launches have 2 kMRow, so it is for
+  // short rows (a 7-point matrix's factors have at most 4 entries a row).
+  // Solves of 7-point systems only, every row with 2 to 4 entries: 8 of 48^3
+  // rows by 4 right-hand sides 19.8 -> 9.1 ms, by one 6.7 -> 5.6 ms
+  bool one = true;
+  for (int32_t i = 0; i < (int32_t)N && one; ++i)
+    one = Wm.rptr[i + 1] - Wm.rptr[i] <= kMRow && Zm.rptr[i + 1] - Zm.rptr[i] <= kMRow;
+  auto factor = [&](const HostCSR &M) {
     std::vector<double> d(N, 0.0);
     std::vector<int32_t> rows, rp(1, 0), cl;
     std::vector<double> vl;
     for (int32_t i = 0; i < M.n; ++i) {
       const int32_t b = M.rptr[i], e = M.rptr[i + 1];
-      if (e - b == 1 && M.idx[b] == i) {
+      if (plain(M, i)) {
         d[i] = M.val[b];
       } else if (e > b) {
         d[i] = std::numeric_limits<double>::quiet_NaN();  // marks a CSR row
+        if (one) continue;
         rows.push_back(i);
         for (int32_t k = b; k < e; ++k) {
           cl.push_back(M.idx[k]);
@@ -1535,8 +1657,44 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
     F3R_HIP(hipStreamSynchronize(c->stream));
     B->dsh = d;
   }
-  B->W = factor(pw);
-  B->Z = factor(pz);
+  B->W = factor(Wm);
+  B->Z = factor(Zm);
+  if (one) {
+    B->mr_copies = share_d ? NR : 1;
+    std::vector<int32_t> rows;
+    for (int s = 0; s < nseg; s += B->mr_copies)
+      for (int64_t i = B->off[s]; i < B->off[s + 1]; ++i)
+        if (csr_row(Wm, (int32_t)i) || csr_row(Zm, (int32_t)i)) rows.push_back((int32_t)i);
+    const size_t nr = rows.size(), ns = std::max<size_t>(1, nr);
+    std::vector<int32_t> meta(4 * ns, 0), wc(ns * kMRow * kMRow, -1);
+    std::vector<double> wv(ns * kMRow * kMRow, 0.0), zv(ns * kMRow, 0.0);
+    int s = 0;
+    for (size_t q = 0; q < nr; ++q) {
+      const int32_t i = rows[q];
+      while (i >= B->off[s + 1]) ++s;
+      const int32_t zb = Zm.rptr[i], ng = Zm.rptr[i + 1] - zb;
+      meta[4 * q] = i;
+      meta[4 * q + 1] = s;
+      meta[4 * q + 2] = (int32_t)(B->off[s + 1] - B->off[s]);
+      meta[4 * q + 3] = ng;
+      for (int32_t g = 0; g < ng; ++g) {
+        zv[q * kMRow + g] = Zm.val[zb + g];
+        const int32_t k = Zm.idx[zb + g], wb = Wm.rptr[k], nw = Wm.rptr[k + 1] - wb;
+        const size_t at = ((size_t)g * nr + q) * kMRow;
+        for (int32_t u = 0; u < nw; ++u) {
+          wc[at + u] = Wm.idx[wb + u];
+          wv[at + u] = Wm.val[wb + u];
+        }
+        if (nw == 0) wc[at] = k;  // an empty row: 0 * x
+      }
+    }
+    B->mr_meta = up32(meta);
+    B->mr_wc = up32(wc);
+    B->mr_wv = upload_values(c, wv, F3R_F16);
+    B->mr_z = upload_values(c, zv, F3R_F16);
+    B->mr_nr = (int32_t)nr;
+    F3R_HIP(hipStreamSynchronize(c->stream));  // the host arrays above are released here
+  }
   F3R_HIP(hipStreamSynchronize(c->stream));
   // work space
   B->alloc_level(B->L1, p.m1);

@@ -427,3 +427,36 @@ def test_lockstep_value_codes(nrhs, sizes):
         out.append([x.download() for x in xs])
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("nrhs", [1, 2, 4])
+@pytest.mark.parametrize("sizes", [[(7, 3), (27, 9), (7, 13)], [(7, 24), (7, 17)]])
+def test_lockstep_short_factor_rows(nrhs, sizes):
+    """M in one launch where no factor row has more than four entries: the bits
+    of the two launches, which a further system with longer rows brings in"""
+    import f3r_amd as F
+    ctx = F.Context(0)
+    extra = F.CSR.dominant(27, 10, 11, 9, margin=0.6)
+    F.algorithm.scaling(extra)
+    systems = []
+    for s, (npts, m) in enumerate(sizes):
+        A = F.CSR.dominant(npts, m, m + 1, m - 1, margin=0.6 + 0.3 * s)
+        F.algorithm.scaling(A)
+        systems.append((A, F.SDAINV(A, 0.1, 1.0, "f16", ctx=ctx)))
+        assert max(np.diff(f[0]).max() for f in systems[-1][1].factors()) <= 4
+    long = F.SDAINV(extra, 0.05, 1.0, "f16", ctx=ctx)
+    assert max(np.diff(f[0]).max() for f in long.factors()) > 4
+    out = []
+    for sys_ in (systems, systems + [(extra, long)]):
+        print(f"lockstep short factor rows nrhs={nrhs} sizes={sizes} systems={len(sys_)}", flush=True)
+        As = [A for A, _ in sys_ for _ in range(nrhs)]
+        Ps = [P for _, P in sys_ for _ in range(nrhs)]
+        B = F.Batch(ctx, As, Ps, m=(100, 3, 2, 2))
+        xs = [F.vector(ctx, "f64", A.n).fill(0.0) for A in As]
+        bs = [F.vector.from_numpy(ctx, F.uniform(A.n, -1.0, 1.0, seed=7 + k)) for k, A in enumerate(As)]
+        res = B.solve(bs, xs)
+        assert all(r.is_solved for r in res)
+        out.append([x.download() for x in xs])
+    for a, b in zip(out[0], out[1]):
+        assert np.array_equal(a, b)
+    ctx.close()
