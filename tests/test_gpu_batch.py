@@ -460,3 +460,27 @@ def test_lockstep_short_factor_rows(nrhs, sizes):
     for a, b in zip(out[0], out[1]):
         assert np.array_equal(a, b)
     ctx.close()
+
+
+@pytest.mark.parametrize("m", [64, 65])   # 128 tiles of 2048 rows, and 135
+def test_lockstep_dots_added_up_by_the_update(m):
+    """segments of at most 128 tiles: the update adds their dots up itself"""
+    import f3r_amd as F
+    ctx = F.Context(0)
+    As, Ps, bs = [], [], []
+    for s, k in enumerate((m, 12)):
+        A = F.CSR.dominant(7, k, margin=0.7)
+        F.algorithm.scaling(A)
+        As.append(A)
+        Ps.append(F.SDAINV(A, 0.1, 1.0, "f16", ctx=ctx))
+        bs.append(F.uniform(A.n, -1.0, 1.0, seed=40 + s))
+    print(f"lockstep dots m={m}", flush=True)
+    xs = [F.vector(ctx, "f64", A.n).fill(0.0) for A in As]
+    res = F.Batch(ctx, As, Ps).solve([F.vector.from_numpy(ctx, b) for b in bs], xs)
+    assert all(r.is_solved for r in res)
+    for A, P, b, x, r in zip(As, Ps, bs, xs, res):
+        assert _true_res(A, x.download(), b) <= 1e-8
+        y = F.vector(ctx, "f64", A.n).fill(0.0)
+        one = F.F3R(ctx, A, P).solve(F.vector.from_numpy(ctx, b), y)
+        assert abs(one.res_iter - r.res_iter) <= 1
+    ctx.close()
