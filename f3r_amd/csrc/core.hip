@@ -461,6 +461,120 @@ template <class S, class F> struct EpiMExit {
   }
   __device__ void finish(State &) const {}
 };
+// General SDAINV in one launch, both factors of at most kBand diagonals (the
+// 7-point stencils): row i's t = W^T h of the rows i + oz that Z takes are
+// worked out again, from W's values of those rows and h at i + oz + ow.  Two
+// launches with t between them took 8.4 + 5.5 us (entry) and 5.3 + 5.5 us at
+// 885 K rows, most of it the launches themselves, their first loads and t's
+// way through memory: 12 more gathers a row, all in flight together, cost
+// less (9.7 and 7.5 us; the 7-point solve at 96^3 9.3 -> 7.9 ms).  A diagonal without an entry in a row holds a zero.
+// SYM: Z's diagonals are W's mirrored (W^T's pattern), so that one of the four
+// terms of each t is h_i itself.
+constexpr int kBand = 4;
+template <class S> struct Band {
+  const S *w, *z;
+  int32_t ow[kBand], oz[kBand];
+  int32_t lo, hi;  // smallest and largest row reached from row 0
+};
+template <class S, class F, bool RAW, bool SYM>
+__global__ __launch_bounds__(kBlock) void k_m_band(int32_t n, Band<S> bd, MIo<S, F> io) {
+  using ACC = typename Acc<S>::type;
+  using X = typename std::conditional<RAW, F, S>::type;
+  const X *x;
+  if constexpr (RAW) x = io.raw; else x = io.in;
+  const int32_t row = xcd_block() * kBlock + threadIdx.x;
+  const int32_t r = row < n ? row : n - 1;
+  const int32_t r0 = __builtin_amdgcn_readfirstlane(row);
+  V4<S> w[kBand];
+  X xv[kBand][kBand];
+  const V4<S> z = ld4(bd.z + (int64_t)r * kBand);
+  const X own = x[r];
+  const S add = io.add ? io.add[r] : S(0);
+  if (r0 + bd.lo >= 0 && r0 + kWave - 1 + bd.hi < n) {  // every row the wave reaches exists
+    const int bias = -bd.lo;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)((uintptr_t)x - (uintptr_t)bias * sizeof(X)), (short)0, (int)(((int64_t)n + bias) * (int64_t)sizeof(X)),
+        kBufferWord3);
+    const int vo = r * (int)sizeof(X);
+#pragma unroll
+    for (int a = 0; a < kBand; ++a) {
+      w[a] = ld4(bd.w + (int64_t)(r + bd.oz[a]) * kBand);
+#pragma unroll
+      for (int b = 0; b < kBand; ++b)
+        xv[a][b] = SYM && b == kBand - 1 - a ? own
+                                             : buffer_gather<X>(rs, vo, (bd.oz[a] + bd.ow[b] + bias) * (int)sizeof(X));
+    }
+  } else {  // a row that does not exist has a zero entry
+#pragma unroll
+    for (int a = 0; a < kBand; ++a) {
+      const int32_t ka = r + bd.oz[a], k = ka >= 0 && ka < n ? ka : r;
+      w[a] = ld4(bd.w + (int64_t)k * kBand);
+#pragma unroll
+      for (int b = 0; b < kBand; ++b) {
+        const int32_t l = k + bd.ow[b];
+        xv[a][b] = x[l >= 0 && l < n ? l : r];
+      }
+    }
+  }
+  const MEntry<S, F> en(io);
+  const MExit<S, F> mo(io);
+  ACC acc = 0;
+#pragma unroll
+  for (int a = 0; a < kBand; ++a) {
+    ACC t = 0;
+#pragma unroll
+    for (int b = 0; b < kBand; ++b) {
+      if constexpr (RAW) t = fma_<ACC>(to_acc(w[a].v[b]), (ACC)en(xv[a][b]), t);
+      else t = fma_<ACC>(to_acc(w[a].v[b]), to_acc(xv[a][b]), t);
+    }
+    acc = fma_<ACC>(to_acc(z.v[a]), to_acc(cvt<S>(t)), acc);
+  }
+  if (row >= n) return;
+  if constexpr (RAW) {
+    const F v = en.norm(own);
+    if (io.vout) io.vout[r] = v;
+    if (io.hin) io.hin[r] = en.store(v);
+  }
+  mo.put(r, cvt<S>(acc), add);
+}
+template <class S> static Band<S> band(const Prec &P) {
+  const S *w = P.bwz->as<S>();
+  Band<S> b{w, w + (int64_t)P.n * kBand, {}, {}, 0, 0};
+  for (int k = 0; k < kBand; ++k) {
+    b.ow[k] = P.bow[k];
+    b.oz[k] = P.boz[k];
+  }
+  for (int a = 0; a < kBand; ++a) {
+    b.lo = std::min(b.lo, b.oz[a]);
+    b.hi = std::max(b.hi, b.oz[a]);
+    for (int k = 0; k < kBand; ++k) {
+      b.lo = std::min(b.lo, b.oz[a] + b.ow[k]);
+      b.hi = std::max(b.hi, b.oz[a] + b.ow[k]);
+    }
+  }
+  return b;
+}
+// n elements at p and at q do not overlap (a null pointer overlaps nothing)
+template <class A, class B> static bool apart(const A *p, const B *q, int64_t n) {
+  const uintptr_t a = (uintptr_t)p, b = (uintptr_t)q;
+  return !p || !q || a + n * sizeof(A) <= b || b + n * sizeof(B) <= a;
+}
+// rows gather x, so nothing that is written may lie over it
+template <class S, class F> static bool band_apply(Prec *P, const MIo<S, F> &io, hipStream_t st) {
+  if (!P->bwz) return false;
+  const int64_t n = P->n;
+  const bool ok = io.raw ? apart(io.raw, io.out, n) && apart(io.raw, io.outf, n) && apart(io.raw, io.hin, n) &&
+                               apart(io.raw, io.vout, n)
+                         : apart(io.in, io.out, n) && apart(io.in, io.outf, n);
+  if (!ok) return false;
+  bool sym = true;
+  for (int k = 0; k < kBand; ++k) sym = sym && P->boz[k] == -P->bow[kBand - 1 - k];
+  auto kern = io.raw ? (sym ? k_m_band<S, F, true, true> : k_m_band<S, F, true, false>)
+                     : (sym ? k_m_band<S, F, false, true> : k_m_band<S, F, false, false>);
+  hipLaunchKernelGGL(kern, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, (int32_t)n, band<S>(*P), io);
+  return true;
+}
+
 // element-wise entry and output for kinds of M without fused kernels
 template <class S, class F> __global__ void k_m_entry(int64_t n, MIo<S, F> io, S *__restrict__ h) {
   const MEntry<S, F> en(io);
@@ -1166,6 +1280,28 @@ HostCSR permute_csr(const HostCSR &M, const std::vector<int32_t> &perm) {
   return R;
 }
 
+// the band form of k_m_band, when each factor has at most kBand diagonals and
+// the rows keep their order (a sort scatters the diagonals); values in
+// ascending column order, as the row sums take them
+static void build_band(Prec *P, const HostCSR &W, const HostCSR &Z, bool sorted) {
+  if (sorted || P->diag || P->n == 0) return;
+  std::vector<int32_t> ow, oz;
+  if (!band_offsets(W, kBand, ow) || !band_offsets(Z, kBand, oz)) return;
+  int64_t reach = 0;
+  for (int32_t a : ow)
+    for (int32_t b : oz) reach = std::max(reach, std::abs((int64_t)a) + std::abs((int64_t)b));
+  if ((P->n + reach) * (int64_t)sizeof(double) >= ((int64_t)1 << 31)) return;  // 32-bit byte offsets
+  std::copy(ow.begin(), ow.end(), P->bow);
+  std::copy(oz.begin(), oz.end(), P->boz);
+  const size_t half = dtype_size(P->dtype) * kBand * (size_t)P->n;
+  std::vector<unsigned char> v(2 * half);
+  band_values(W, ow, kBand, P->dtype, v.data());
+  band_values(Z, oz, kBand, P->dtype, v.data() + half);
+  P->bwz = dev_alloc(v.size());
+  F3R_HIP(hipMemcpyAsync(P->bwz->p, v.data(), v.size(), hipMemcpyHostToDevice, P->ctx->stream));
+  F3R_HIP(hipStreamSynchronize(P->ctx->stream));  // v is released at scope end
+}
+
 void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int32_t K, bool offsets) {
   Context *c = P->ctx.get();
   const int32_t n = P->host.f[0].n;
@@ -1195,6 +1331,7 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
         F3R_HIP(hipStreamSynchronize(c->stream));  // wz is released at scope end
       }
     }
+    build_band(P, W, Z, perm != nullptr);
     for (int w = 0; w < 2; ++w) {
       const HostCSR &M = w == 0 ? W : Z;
       HostSell hs = build_sell(M, C, 1, K, perm, perm != nullptr, offsets);
@@ -1328,6 +1465,10 @@ template <class S> static void ilu_apply_t(Prec *P, const S *in, S *out, hipStre
 
 template <class S> static void sdainv_apply_t(Prec *P, const S *in, S *out, hipStream_t st) {
   using ACC = typename Acc<S>::type;
+  MIo<S, ACC> io;
+  io.in = in;
+  io.out = out;
+  if (band_apply<S, ACC>(P, io, st)) return;
   S *tmp = P->tmp->as<S>();
   const bool wp = !P->W->sh->internal;
   SellArgs aw = sell_args(*P->W->sh, wp), az = sell_args(*P->Z->sh, wp);
@@ -1375,6 +1516,7 @@ template <class S, class F> void prec_apply_io(Prec *P, const MIo<S, F> &io, hip
     else vec = vec && align4(d.w) && align4(d.z);
     auto kern = vec ? k_m_diag<S, F, true> : k_m_diag<S, F, false>;
     hipLaunchKernelGGL(kern, dim3(vec ? grid_for((n + 3) / 4, P->ctx->num_cu) : g.x), b, 0, st, n, d, io);
+  } else if (P->kind == 0 && band_apply<S, F>(P, io, st)) {
   } else if (P->kind == 0) {
     S *tmp = P->tmp->as<S>();
     SellArgs aw = sell_args(*P->W->sh, false), az = sell_args(*P->Z->sh, false);

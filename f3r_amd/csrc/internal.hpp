@@ -25,6 +25,10 @@ struct Prec {
   bool diag = false;
   DevPtr dw, dz;              // diagonals when `diag`
   DevPtr dwz;                 // fp16 only: (dw[i], dz[i]) interleaved, one 4-byte load per row
+  // at most 4 diagonals in each factor: band form (kBand values a row, W's
+  // then Z's)
+  DevPtr bwz;
+  int32_t bow[4] = {}, boz[4] = {};
   // ILU(0)
   std::vector<int32_t> l_lptr, u_lptr;  // level pointers into *_rows
   DevPtr l_rows, u_rows, l_rptr, l_idx, l_val, u_rptr, u_idx, u_val, u_dinv;

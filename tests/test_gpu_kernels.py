@@ -597,3 +597,26 @@ def test_bf16_spmv_bitexact(ctx, fmt):
             M.compute_residual(bv, xv, yv)
             ref = O.spmv(A.n, A.rptr, A.idx, A.val, xh, 3, xp, yp, 1, b=bv.download())
             assert np.array_equal(yv.download().view(np.uint8), ref.view(np.uint8)), (name, fmt, "resid")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32", "f64"])
+@pytest.mark.parametrize("dims", [(9, 1, 1), (3, 3, 3), (4, 4, 4), (13, 1, 17), (2, 31, 5), (17, 16, 19), (40, 33, 29)])
+def test_sdainv_band_form(ctx, dims, dtype):
+    """factors of at most four diagonals each: M in one launch gives the bits of
+    the two products, which an application in place still takes"""
+    import f3r_amd as F
+    A = F.CSR.convdiff7(*dims, sigma=0.5, corr=4.0, peclet=0.0, seed=2)
+    F.algorithm.scaling(A)
+    P = F.SDAINV(A, 0.1, 1.0, dtype, ctx=ctx)
+    diagonals = [len(np.unique(i - np.repeat(np.arange(A.n), np.diff(r)))) for r, i, v in P.factors()]
+    assert max(diagonals) <= 4
+    print(f"band form dims={dims} {dtype} diagonals={diagonals}", flush=True)
+    b = F.uniform(A.n, -1.0, 1.0, seed=3)
+    x = F.vector(ctx, dtype, A.n)
+    x.upload(b)
+    y = F.vector(ctx, dtype, A.n).fill(0.0)
+    P.operate(x, y)
+    P.operate(x, x)
+    got, want = y.download(), x.download()
+    assert np.all(np.isfinite(got.astype(np.float64))) and np.any(got != 0)
+    assert np.array_equal(got, want)
