@@ -210,12 +210,6 @@ struct HostFactors {
 HostFactors sdainv_host(const HostCSR &A, double tol, double acc);
 HostFactors ilu0_host(const HostCSR &A, int32_t blocks, double acc);
 HostCSR csr_transpose(const HostCSR &A);
-// the diagonals (column - row, ascending) that M has entries on; false when
-// there are more than `most`
-bool band_offsets(const HostCSR &M, int32_t most, std::vector<int32_t> &off);
-// M's values by row and diagonal (`width` a row, in off's order, zero without
-// an entry), converted to dtype
-void band_values(const HostCSR &M, const std::vector<int32_t> &off, int32_t width, int dtype, void *out);
 // pieces of ilu0_host: the block-diagonal part of A, the position of each
 // row's diagonal entry in it, and the split of the eliminated rows into L, U
 HostCSR ilu0_restrict(const HostCSR &A, int32_t blocks);

@@ -1280,26 +1280,72 @@ HostCSR permute_csr(const HostCSR &M, const std::vector<int32_t> &perm) {
   return R;
 }
 
-// the band form of k_m_band, when each factor has at most kBand diagonals and
-// the rows keep their order (a sort scatters the diagonals); values in
-// ascending column order, as the row sums take them
-static void build_band(Prec *P, const HostCSR &W, const HostCSR &Z, bool sorted) {
-  if (sorted || P->diag || P->n == 0) return;
-  std::vector<int32_t> ow, oz;
-  if (!band_offsets(W, kBand, ow) || !band_offsets(Z, kBand, oz)) return;
+// the diagonals (column - row, ascending) of M, laid out as hs in its own row
+// order; false when there are more than kBand.  Offset chunks list theirs.
+static bool band_offsets(const HostCSR &M, const HostSell &hs, std::vector<int32_t> &off) {
+  off.clear();
+  auto add = [&](int32_t o) {
+    if (std::find(off.begin(), off.end(), o) == off.end()) off.push_back(o);
+    return off.size() <= kBand;
+  };
+  for (int32_t o : hs.coff)
+    if (!add(o)) return false;
+  for (int32_t s = 0; s < hs.nchunks; ++s) {
+    if (!hs.iptr.empty() && hs.iptr[s] < 0) continue;
+    const int32_t r1 = std::min(hs.n, (s + 1) * hs.C);
+    for (int32_t i = s * hs.C; i < r1; ++i)
+      for (int32_t k = M.rptr[i]; k < M.rptr[i + 1]; ++k)
+        if (!add(M.idx[k] - i)) return false;
+  }
+  std::sort(off.begin(), off.end());
+  return true;
+}
+// a factor by row and diagonal from its SELL layout (padding slots hold zeros)
+template <class S>
+__global__ __launch_bounds__(kBlock) void k_band_fill(SellArgs a, int K, const S *__restrict__ val, int4 off,
+                                                      S *__restrict__ out) {
+  const int32_t r = blockIdx.x * kBlock + threadIdx.x;
+  if (r >= a.n) return;
+  const int32_t s = r >> a.log2C, r0 = s << a.log2C, c0 = a.cptr[s], cw = a.cwidth[s];
+  const int32_t tc = min(a.n - r0, 1 << a.log2C), width = chunk_slots(cw, K);
+  const int32_t start = a.iptr ? a.iptr[s] : c0;
+  S v[kBand] = {S(0), S(0), S(0), S(0)};
+  for (int32_t t = 0; t < width; ++t) {
+    const int64_t pos = chunk_slot_pos(c0, cw, tc, r - r0, t, K);
+    const S e = val[pos];
+    if (to_acc(e) == 0) continue;
+    const int32_t o = a.iptr && start < 0 ? a.coff[-start - 1 + t] : a.idx[start + (pos - c0)] - r;
+    if (o == off.x) v[0] = e;
+    else if (o == off.y) v[1] = e;
+    else if (o == off.z) v[2] = e;
+    else if (o == off.w) v[3] = e;
+  }
+  for (int k = 0; k < kBand; ++k) out[(int64_t)r * kBand + k] = v[k];
+}
+// the band form of k_m_band: values in ascending column order, as the row sums
+// take them
+template <class S> static void band_fill(Prec *P) {
+  P->bwz = dev_alloc(2 * sizeof(S) * kBand * (size_t)P->n);
+  for (int m = 0; m < 2; ++m) {
+    const Mat &M = m == 0 ? *P->W : *P->Z;
+    const int32_t *o = m == 0 ? P->bow : P->boz;
+    hipLaunchKernelGGL(k_band_fill<S>, dim3((P->n + kBlock - 1) / kBlock), dim3(kBlock), 0, P->ctx->stream,
+                       sell_args(*M.sh, false), M.sh->K, (const S *)M.s_val->as<S>(), make_int4(o[0], o[1], o[2], o[3]),
+                       P->bwz->as<S>() + (int64_t)m * P->n * kBand);
+  }
+  F3R_HIP(hipGetLastError());
+  F3R_HIP(hipStreamSynchronize(P->ctx->stream));  // as the uploads: ready for any stream
+}
+static void build_band(Prec *P, const std::vector<int32_t> &ow, const std::vector<int32_t> &oz) {
   int64_t reach = 0;
   for (int32_t a : ow)
     for (int32_t b : oz) reach = std::max(reach, std::abs((int64_t)a) + std::abs((int64_t)b));
   if ((P->n + reach) * (int64_t)sizeof(double) >= ((int64_t)1 << 31)) return;  // 32-bit byte offsets
   std::copy(ow.begin(), ow.end(), P->bow);
   std::copy(oz.begin(), oz.end(), P->boz);
-  const size_t half = dtype_size(P->dtype) * kBand * (size_t)P->n;
-  std::vector<unsigned char> v(2 * half);
-  band_values(W, ow, kBand, P->dtype, v.data());
-  band_values(Z, oz, kBand, P->dtype, v.data() + half);
-  P->bwz = dev_alloc(v.size());
-  F3R_HIP(hipMemcpyAsync(P->bwz->p, v.data(), v.size(), hipMemcpyHostToDevice, P->ctx->stream));
-  F3R_HIP(hipStreamSynchronize(P->ctx->stream));  // v is released at scope end
+  if (P->dtype == F3R_F64) band_fill<double>(P);
+  else if (P->dtype == F3R_F32) band_fill<float>(P);
+  else band_fill<half_t>(P);
 }
 
 void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int32_t K, bool offsets) {
@@ -1331,7 +1377,9 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
         F3R_HIP(hipStreamSynchronize(c->stream));  // wz is released at scope end
       }
     }
-    build_band(P, W, Z, perm != nullptr);
+    // rows in their own order only: a sort scatters the diagonals
+    bool band_form = !perm && !P->diag && n > 0;
+    std::vector<int32_t> boff[2];
     for (int w = 0; w < 2; ++w) {
       const HostCSR &M = w == 0 ? W : Z;
       HostSell hs = build_sell(M, C, 1, K, perm, perm != nullptr, offsets);
@@ -1342,7 +1390,9 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
       m->sh = upload_sell_shared(c, hs, perm != nullptr);
       m->s_val = upload_sell_values(c, hs, P->dtype);
       (w == 0 ? P->W : P->Z) = m;
+      band_form = band_form && band_offsets(M, hs, boff[w]);
     }
+    if (band_form) build_band(P, boff[0], boff[1]);
   } else {
     HostCSR L = perm ? permute_csr(P->host.f[0], *perm) : P->host.f[0];
     HostCSR U = perm ? permute_csr(P->host.f[1], *perm) : P->host.f[1];

@@ -6,11 +6,9 @@
 // Compiled with -ffp-contract=off: the factorizations must round exactly as
 // the reference's host code does (one rounding per operation).
 #include <algorithm>
-#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstring>
-#include <mutex>
 #include <numeric>
 #include <thread>
 
@@ -30,45 +28,6 @@ template <class Fn> static void parallel_ranges(int64_t n, Fn fn) {
   std::vector<std::thread> th;
   for (int64_t t = 0; t < nt; ++t) th.emplace_back(fn, n * t / nt, n * (t + 1) / nt);
   for (auto &x : th) x.join();
-}
-
-bool band_offsets(const HostCSR &M, int32_t most, std::vector<int32_t> &off) {
-  off.clear();
-  std::atomic<bool> few{true};
-  std::mutex mu;
-  auto add = [most](std::vector<int32_t> &s, int32_t o) {
-    if (std::find(s.begin(), s.end(), o) != s.end()) return true;
-    s.push_back(o);
-    return (int32_t)s.size() <= most;
-  };
-  parallel_ranges(((int64_t)M.n + 255) / 256, [&](int64_t c0, int64_t c1) {
-    std::vector<int32_t> s;
-    bool ok = true;
-    for (int64_t i = c0 * 256; i < std::min<int64_t>(M.n, c1 * 256) && ok && few.load(std::memory_order_relaxed); ++i)
-      for (int32_t k = M.rptr[i]; k < M.rptr[i + 1] && ok; ++k) ok = add(s, M.idx[k] - (int32_t)i);
-    std::lock_guard<std::mutex> lk(mu);
-    for (int32_t o : s) ok = add(off, o) && ok;
-    if (!ok) few = false;
-  });
-  std::sort(off.begin(), off.end());
-  return few;
-}
-
-void band_values(const HostCSR &M, const std::vector<int32_t> &off, int32_t width, int dtype, void *out) {
-  const size_t es = dtype_size(dtype);
-  parallel_ranges(((int64_t)M.n + 255) / 256, [&](int64_t c0, int64_t c1) {
-    for (int64_t i = c0 * 256; i < std::min<int64_t>(M.n, c1 * 256); ++i) {
-      unsigned char *row = static_cast<unsigned char *>(out) + (size_t)i * width * es;
-      std::memset(row, 0, (size_t)width * es);
-      for (int32_t k = M.rptr[i]; k < M.rptr[i + 1]; ++k) {
-        const int32_t o = M.idx[k] - (int32_t)i;
-        const size_t at = (size_t)(std::find(off.begin(), off.end(), o) - off.begin());
-        if (dtype == F3R_F64) reinterpret_cast<double *>(row)[at] = M.val[k];
-        else if (dtype == F3R_F32) reinterpret_cast<float *>(row)[at] = (float)M.val[k];
-        else reinterpret_cast<uint16_t *>(row)[at] = d2h_bits(M.val[k]);
-      }
-    }
-  });
 }
 
 // algorithm::scaling (sparse/matrix/algorithm.hpp:45-59): every entry divided
