@@ -317,11 +317,11 @@ def main():
                    "graph": not args.no_graph},
         "roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(ach / PEAK_HBM_GBS, 4), "traffic": None, "traffic_detail": None,
-                     "kernel": "k_sell<half,half,float,8,EpiDots<float,4>>: level-3 fp16 SpMV w = A16 z_j (fp16 "
-                               "values, fp16 z, fp32 sums) with the CGS dots <w, v_k>, k <= j, fused; the solve's "
-                               "mix j = 0..3, back to back; algorithmic bytes per launch = 2 nnz (values, unpadded; "
-                               "no column indices in the chunk-offset layout) + 4 B per nonzero of the int32-index "
-                               "chunks + n (2 z + 4 w + 4 (j+1) v), averaged over j",
+                     "kernel": "k_quad<half,half,float,8,EpiDots<float,4>>: level-3 fp16 SpMV w = A16 z_j (fp16 "
+                               "values by 4-bit codes, fp16 z, fp32 sums) with the CGS dots <w, v_k>, k <= j, "
+                               "fused; the solve's mix j = 0..3, back to back; algorithmic bytes per launch = 16 B "
+                               "of codes a row (instead of 2 nnz of values) + the values of the few chunks that "
+                               "are not coded + n (2 z + 4 w + 4 (j+1) v), averaged over j",
                      "us_per_launch": head["us"], "algorithmic_bytes": head["algorithmic_bytes"],
                      "metric_spmv_f16": kern["spmv_f16"]},
         "kernels": kern,

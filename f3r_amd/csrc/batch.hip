@@ -557,7 +557,8 @@ __global__ __launch_bounds__(kBlock) void k_sell_mr(SellArgs a, const V *__restr
 // distinct values: a lane takes four matrix rows of NR copies, so codes are
 // decoded once for all copies and x is read in windows.  The gathers and their
 // latency, not the bytes, were the plain product's cost (0.32 of the memory
-// rate for 4 copies).
+// rate for 4 copies; 5.93 M rows in fp16: now 17 us, and with the other steps'
+// products a solve 14.1 -> 11.1 ms).
 template <class V, class X, class ACC, int K, int NR, class Y>
 __global__ __launch_bounds__(kBlock) void k_quad_mr(SellArgs a, QuadArgs qa, const V *__restrict__ val,
                                                     const X *__restrict__ x, int64_t nx,

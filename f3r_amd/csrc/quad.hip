@@ -246,6 +246,11 @@ std::shared_ptr<QuadSet> build_quads(Context *c, const SellShared &sh, const dou
   q->bias = (-umin + 1 + 7) / 8 * 8;
   q->nfc = (int32_t)fchunk.size();
   q->nfb = ((q->nfc + kWavesPerBlock - 1) / kWavesPerBlock + kXcds - 1) / kXcds * kXcds;  // the rest keep their XCDs
+  q->code_bytes = units * (int64_t)sizeof(u32x4);
+  for (int32_t s : fchunk) {
+    q->plain_slots += cptr[s + 1] - cptr[s];
+    if (iptr[s] >= 0) q->plain_idx += cptr[s + 1] - cptr[s];
+  }
   q->blk = upload(c, blk.data(), sizeof(int4) * blk.size());
   q->tabs = upload(c, tabs.data(), sizeof(QuadTab) * tabs.size());
   q->fchunk = upload(c, fchunk.data(), 4 * fchunk.size());

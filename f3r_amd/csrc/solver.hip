@@ -5,10 +5,10 @@
 //   L4 = adaptive Richardson(A4, M, m4, c)   fp16 storage in HALF
 // as composed in work/src/f3r-gpu.cpp:210-266.
 //
-// Everything but the outer convergence test stays on the device: Hessenberg
-// columns, Givens rotations, residual estimates and the adaptive Richardson
-// weights are written by the last block of the reduction kernels that
-// produce them, so no level below the outer one synchronises with the host.
+// Everything but the outer convergence test stays on the device, so no level
+// below the outer one synchronises with the host.  The kernels of an inner
+// level leave block sums (dots, norms) that their readers add up; the Givens
+// rotations of an inner cycle run in the kernel that forms its solution.
 // The body of level 2 (m2 level-3 solves and Arnoldi steps) is captured once
 // per pattern of probe calls in a HIP graph and replayed.
 //
@@ -91,7 +91,7 @@ __device__ void hess_solve(const T *H, int ldh, const T *e, T *y, int j) {
 
 // ------------------------------------------------- Arnoldi epilogues ----
 // w = A z stored into V_{j+1}, and the dots <w, V_k>, k <= j, reduced in the
-// same pass; the last block writes H(j, 0..j).
+// same pass as block sums.
 template <class T, int NV> struct EpiDots {
   struct State {
     T v[NV];
@@ -102,9 +102,7 @@ template <class T, int NV> struct EpiDots {
   T *__restrict__ w;
   Cols<T, NV> cols;
   int ncols;
-  T *Hcol;
   T *partial;
-  unsigned *counter;
   // x = z * s with s a power of two (fp16 storage of z): the sum is scaled
   // back by xs = 1/s, exactly, so w is bit-identical to the sum over z
   T xs = 1;
@@ -147,8 +145,8 @@ template <class T, int NV> struct EpiDots {
 #pragma unroll
         for (int c = 0; c < 4; ++c) s.v[k] = fma_<T>(o.v[c], p.v[k].v[c], s.v[k]);
   }
-  // Block sums only, into partial[k * gridDim.x + block]; k_dots_finish adds
-  // them in the next launch.  A grid reduction finished in this kernel made
+  // Block sums only, into partial[k * gridDim.x + block]; the CGS update's
+  // blocks add them up, or k_dots_finish before it.  A grid reduction finished in this kernel made
   // every block wait for its stores (the w rows included) and its arrival
   // atomic before retiring, which cost more than the SpMV's tail: 53 vs
   // 34 us per launch at 128^3.
@@ -808,6 +806,10 @@ struct Solver {
   std::shared_ptr<SellShared> sh;    // layout of A64 / A32
   std::shared_ptr<SellShared> sh16;  // layout of A16 (sh itself when K agrees)
   std::shared_ptr<QuadSet> quad;     // value codes of A (null: too many distinct values)
+  // algorithmic bytes of a product with A: its values (and indexes) or their codes, x and y once
+  double product_bytes(const SellShared &l, int sv, int sx, int sy) const {
+    return quad ? quad->algo_bytes(l.n, sv, sx, sy) : l.algo_bytes(sv, sx, sy);
+  }
   DevPtr A64, A32, A16;
   std::shared_ptr<Prec> P;
   float range_s = 1.f;
@@ -924,7 +926,7 @@ struct Solver {
   void spmv_dots(InnerLevel<T> &L, const V *val, int j) {
     Cols<T, NV> c{};
     for (int k = 0; k <= j; ++k) c.p[k] = L.V[k];
-    EpiDots<T, NV> epi{L.w(), c, j + 1, L.Hp() + (int64_t)j * L.ldh(), partial<T>(), counter(0)};
+    EpiDots<T, NV> epi{L.w(), c, j + 1, partial<T>()};
     if (!L.Zh.empty()) {
       epi.xs = (T)(1.0 / range_s);
       product<V, half_t, T>(val, L.Zh[j], epi, spmv_grid);
@@ -1339,7 +1341,7 @@ struct Solver {
       constexpr int NV = decltype(nv)::value;
       Cols<float, NV> c{};
       for (int k = 0; k <= j; ++k) c.p[k] = L.Vc<float>(k);
-      EpiDots<float, NV> epi{w, c, j + 1, Hcol, partial<float>(), counter(0)};
+      EpiDots<float, NV> epi{w, c, j + 1, partial<float>()};
       if (L.mat == F3R_F16)
         product<half_t, float, float>(A16->as<half_t>(), L.Zc<float>(j), epi, spmv_grid);
       else
@@ -1995,26 +1997,26 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
       case 0:  // fp16 values, fp16 x and y (the metric's fp16 SpMV)
         s->product<half_t, half_t, float>(s->A16->as<half_t>(), (const half_t *)x16,
                                           EpiStore<half_t, float>{y16, nullptr});
-        by = s->sh16->algo_bytes(2, 2, 2);
+        by = s->product_bytes(*s->sh16, 2, 2, 2);
         break;
       case 1:  // fp16 values, fp32 x and y (level 3)
         s->product<half_t, float, float>(s->A16->as<half_t>(), (const float *)x32,
                                          EpiStore<float, float>{y32, nullptr});
-        by = s->sh16->algo_bytes(2, 4, 4);
+        by = s->product_bytes(*s->sh16, 2, 4, 4);
         break;
       case 2:  // fp32 (level 2)
         s->product<float, float, float>(s->A32->as<float>(), (const float *)x32,
                                         EpiStore<float, float>{y32, nullptr});
-        by = s->sh->algo_bytes(4, 4, 4);
+        by = s->product_bytes(*s->sh, 4, 4, 4);
         break;
       case 3:  // fp64 (outer level)
         s->product<double, double, double>(s->A64->as<double>(), (const double *)x64,
                                            EpiStore<double, double>{y64, nullptr});
-        by = s->sh->algo_bytes(8, 8, 8);
+        by = s->product_bytes(*s->sh, 8, 8, 8);
         break;
       case 4:  // level-3 Arnoldi step j = m3 - 1: fp16 SpMV of Z_j + CGS dots with V_0..V_j, and their finish
         s->template spmv_dots<float, half_t, 4>(s->L3f, s->A16->as<half_t>(), s->L3f.m - 1);
-        by = s->sh16->algo_bytes(2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * s->L3f.m;
+        by = s->product_bytes(*s->sh16, 2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * s->L3f.m;
         break;
       case 5:  // level-3 CGS update + norm of that step (the last: w is not stored)
         s->template cgs_update<float, 4>(s->L3f, s->L3f.m - 1);
@@ -2026,8 +2028,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
         for (int j = 0; j < m; ++j) {
           Cols<float, 4> c{};
           for (int k = 0; k <= j; ++k) c.p[k] = s->L3f.V[k];
-          EpiDots<float, 4> epi{s->L3f.w(), c, j + 1, s->L3f.Hp() + (int64_t)j * s->L3f.ldh(),
-                                s->template partial<float>(), s->counter(0)};
+          EpiDots<float, 4> epi{s->L3f.w(), c, j + 1, s->template partial<float>()};
           if (!s->L3f.Zh.empty()) {
             epi.xs = 1.f / s->range_s;
             s->product<half_t, half_t, float>(s->A16->as<half_t>(), (const half_t *)s->L3f.Zh[j], epi, s->spmv_grid);
@@ -2035,7 +2036,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
             s->product<half_t, float, float>(s->A16->as<half_t>(), (const float *)s->L3f.Z[j], epi, s->spmv_grid);
           }
           // values, Z_j gathered, w written, V_0 .. V_j read
-          by += s->sh16->algo_bytes(2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * (j + 1);
+          by += s->product_bytes(*s->sh16, 2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * (j + 1);
         }
         by /= m;
         break;
@@ -2058,7 +2059,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
                                             1.f / s->range_s};
         s->product<half_t, half_t, float>(s->A16->as<half_t>(), (const half_t *)s->hout->as<half_t>(), epi);
         // values, h gathered, hin / h / (w, z) read per row, h' written
-        by = s->sh16->algo_bytes(2, 2, 2) + (double)s->n * (2 + 2 + 4);
+        by = s->product_bytes(*s->sh16, 2, 2, 2) + (double)s->n * (2 + 2 + 4);
         break;
       }
       case 9: {  // the innermost entry: normalise the basis vector, fp16 input, first weighted M application
