@@ -1069,13 +1069,11 @@ struct BatchSolver {
           return;
         }
       }
-      if constexpr (K >= 4) {
-        if (quad) {
-          const QuadArgs qa = quad->template args<V>();
-          hipLaunchKernelGGL((k_quad_mr<V, X, ACC, K, R, Y>), dim3(quad_blocks(a, qa)), dim3(kBlock), 0, st(), a, qa,
-                             val, x, (int64_t)N, shf, str, y, b, (const int32_t *)cseg->as<int32_t>(), ysc);
-          return;
-        }
+      if (quad) {
+        const QuadArgs qa = quad->template args<V>();
+        hipLaunchKernelGGL((k_quad_mr<V, X, ACC, K, R, Y>), dim3(quad_blocks(a, qa)), dim3(kBlock), 0, st(), a, qa,
+                           val, x, (int64_t)N, shf, str, y, b, (const int32_t *)cseg->as<int32_t>(), ysc);
+        return;
       }
       hipLaunchKernelGGL((k_sell_mr<V, X, ACC, K, R, Y>), g, dim3(kBlock), 0, st(), a, val, x, (int64_t)N, shf, str, y,
                          b, (const int32_t *)cseg->as<int32_t>(), ysc);
@@ -1616,7 +1614,7 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
       B->sh16 = upload_sell_shared(c, h16, false);
       B->A16 = upload_sell_values(c, h16, F3R_F16);
     }
-    if (NR > 1 && !B->lanes && K >= 4 && K16 >= 4) B->quad = build_quads(c, *B->sh, B->A64->as<double>(), moff);
+    if (NR > 1 && !B->lanes) B->quad = build_quads(c, *B->sh, B->A64->as<double>(), moff);
     // k_sell_mr gathers x (fp64 at most) of offset chunks through a buffer
     // resource whose size and byte offsets are 32-bit
     const int64_t bias = std::max(B->sh->off_bias, B->sh16->off_bias);

@@ -418,15 +418,15 @@ def test_lockstep_value_codes(nrhs, sizes):
             Ps.append(P)
             bs.append(F.uniform(A.n, -1.0, 1.0, seed=100 * s + r))
     out = []
-    for kw in ({"index": 1}, {"index": 0, "K": 4}):
+    for kw in ({"index": 1}, {"index": 0, "K": 4}, {"index": 1, "K": 1}):
         print(f"lockstep value codes nrhs={nrhs} sizes={sizes} {kw}", flush=True)
         B = F.Batch(ctx, As, Ps, m=(100, 3, 2, 2), **kw)
         xs = [F.vector(ctx, "f64", A.n).fill(0.0) for A in As]
         res = B.solve([F.vector.from_numpy(ctx, b) for b in bs], xs)
         assert all(r.is_solved for r in res)
         out.append([x.download() for x in xs])
-    for a, b in zip(*out):
-        assert np.array_equal(a, b)
+    for a, b, c in zip(*out):
+        assert np.array_equal(a, b) and np.array_equal(a, c)
 
 
 @pytest.mark.parametrize("nrhs", [1, 2, 4])
