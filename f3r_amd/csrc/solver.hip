@@ -806,9 +806,17 @@ struct Solver {
   std::shared_ptr<SellShared> sh;    // layout of A64 / A32
   std::shared_ptr<SellShared> sh16;  // layout of A16 (sh itself when K agrees)
   std::shared_ptr<QuadSet> quad;     // value codes of A (null: too many distinct values)
+  // whether a product runs by the value codes: a caller with a block limit
+  // (the reductions': their readers take kMaxReduceGrid block sums, 16.7 M
+  // rows of codes, or what f3r_params.grid and flags bit 1 say) gets the
+  // plain product, whose blocks loop over the rows, where the codes' blocks
+  // are more.  The same loop in k_quad costs it 10 to 100 registers a lane.
+  bool coded(int grid) const {
+    return quad && (grid <= 0 || quad_blocks(args(), quad->args<double>()) <= grid);
+  }
   // algorithmic bytes of a product with A: its values (and indexes) or their codes, x and y once
-  double product_bytes(const SellShared &l, int sv, int sx, int sy) const {
-    return quad ? quad->algo_bytes(l.n, sv, sx, sy) : l.algo_bytes(sv, sx, sy);
+  double product_bytes(const SellShared &l, int sv, int sx, int sy, int grid = 0) const {
+    return coded(grid) ? quad->algo_bytes(l.n, sv, sx, sy) : l.algo_bytes(sv, sx, sy);
   }
   DevPtr A64, A32, A16;
   std::shared_ptr<Prec> P;
@@ -883,12 +891,12 @@ struct Solver {
     const int64_t per = vec ? 4 * kBlock : kBlock;
     return (int)std::min<int64_t>((n + per - 1) / per, (int64_t)ctx->num_cu * 16);
   }
-  // a product with A's values V: by their codes where the matrix has them
+  // a product with A's values V, on at most `grid` blocks when that is not 0
   template <class V, class X, class ACC, class Epi>
   void product(const V *val, const X *x, const Epi &epi, int grid = 0) const {
     const SellShared &L = shv<V>();
     const SellArgs a = argsv<V>();
-    if (quad) {
+    if (coded(grid)) {
       if constexpr (std::is_same<V, half_t>::value) {
         if (L.K == 8) {
           launch_quad<8, V, X, ACC>(a, quad->template args<V>(), val, x, epi, st());
@@ -902,7 +910,7 @@ struct Solver {
   }
   // blocks of a product with A's values V that leaves block sums
   template <class V> int dots_blocks() const {
-    return quad ? quad_blocks(argsv<V>(), quad->template args<V>()) : sell_blocks(argsv<V>(), spmv_grid);
+    return coded(spmv_grid) ? quad_blocks(argsv<V>(), quad->template args<V>()) : sell_blocks(argsv<V>(), spmv_grid);
   }
   SellArgs args() const { return sell_args(*sh, false); }
   // the layout of the matrix with value type V (the fp16 copy may differ in K)
@@ -937,6 +945,7 @@ struct Solver {
     finish_dots<T>(dots_blocks<V>(), j, L.Hp() + (int64_t)j * L.ldh());
   }
   template <class T> void finish_dots(int G, int j, T *Hcol) {
+    F3R_CHECK(G <= kMaxReduceGrid, F3R_ERR_RANGE, "solver: more block sums than their readers take");
     if (G > kDirectDots)
       hipLaunchKernelGGL(k_dots_finish<T>, dim3(j + 1), dim3(1024), 0, st(), (const T *)partial<T>(), G, Hcol);
     dots_parts = G > kDirectDots ? 0 : G;
@@ -2016,7 +2025,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
         break;
       case 4:  // level-3 Arnoldi step j = m3 - 1: fp16 SpMV of Z_j + CGS dots with V_0..V_j, and their finish
         s->template spmv_dots<float, half_t, 4>(s->L3f, s->A16->as<half_t>(), s->L3f.m - 1);
-        by = s->product_bytes(*s->sh16, 2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * s->L3f.m;
+        by = s->product_bytes(*s->sh16, 2, s->L3f.Zh.empty() ? 4 : 2, 4, s->spmv_grid) + 4.0 * s->n * s->L3f.m;
         break;
       case 5:  // level-3 CGS update + norm of that step (the last: w is not stored)
         s->template cgs_update<float, 4>(s->L3f, s->L3f.m - 1);
@@ -2036,7 +2045,7 @@ int f3r_solver_time_kernel(f3r_solver S, int32_t which, int32_t reps, double *ms
             s->product<half_t, float, float>(s->A16->as<half_t>(), (const float *)s->L3f.Z[j], epi, s->spmv_grid);
           }
           // values, Z_j gathered, w written, V_0 .. V_j read
-          by += s->product_bytes(*s->sh16, 2, s->L3f.Zh.empty() ? 4 : 2, 4) + 4.0 * s->n * (j + 1);
+          by += s->product_bytes(*s->sh16, 2, s->L3f.Zh.empty() ? 4 : 2, 4, s->spmv_grid) + 4.0 * s->n * (j + 1);
         }
         by /= m;
         break;

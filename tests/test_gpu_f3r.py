@@ -427,3 +427,47 @@ def test_value_codes(ctx, kind, variant):
     # fp32 dots of 4 columns in another order (2^-24 n^0.5 at most), then fp16 roundings that may flip
     tol = {"half": 2e-3, "float": 1e-4, "double": 1e-10}[variant]
     assert np.linalg.norm(out[1, 3] - out[0, 3]) <= tol * np.linalg.norm(out[0, 3])
+
+
+def _level_pair(ctx, A, levels=(3,), n_inner=(2, 3, 4, 2), **kw):
+    """level applications of the DOUBLE build with value codes and, from the
+    int32-index layout, without: {level: (coded, plain)}"""
+    import f3r_amd as F
+    P = F.SDAINV(A, 0.1, 1.0, "f64", ctx=ctx, device=True)
+    b = F.uniform(A.n, -1.0, 1.0, seed=3)
+    vin = F.vector.from_numpy(ctx, b / np.linalg.norm(b))
+    out = {}
+    for index in (1, 0):
+        S = F.F3R(ctx, A, P, m=n_inner, variant="double", index=index, K=0 if index else 4, use_graph=False,
+                  device_build=True, **kw)
+        for level in levels:
+            v = F.vector(ctx, "f64", A.n)
+            S.level_apply(level, vin, v)
+            out.setdefault(level, []).append(v.download())
+        del S
+    return out
+
+
+def test_value_codes_beyond_the_block_limit(ctx):
+    """a product by value codes of more rows than the reductions' block limit
+    has blocks of 1024 rows for: no block sum of the dots is lost"""
+    import f3r_amd as F
+    A = F.CSR.dominant(7, 256, 256, 257, margin=0.7)
+    assert (A.n + 1023) // 1024 > 16384
+    F.algorithm.scaling(A)
+    print(f"value codes n={A.n}", flush=True)
+    got, want = _level_pair(ctx, A)[3]
+    # fp64 dots of 1.7e7 rows in another order: 2^-53 n^0.5 each, through four steps
+    assert np.linalg.norm(got - want) <= 1e-10 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("grid", [24, 7])
+def test_value_codes_keep_to_the_callers_grid(ctx, grid):
+    """flags bit 1 and `grid` limit the blocks of the products that leave block
+    sums on a matrix with value codes too: the int32-index layout's bits"""
+    import f3r_amd as F
+    A = F.CSR.dominant(7, 52, 51, 50, margin=0.7)
+    F.algorithm.scaling(A)
+    print(f"value codes grid={grid}", flush=True)
+    got, want = _level_pair(ctx, A, cap_spmv=True, grid=grid)[3]
+    assert np.array_equal(got, want)
