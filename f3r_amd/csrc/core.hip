@@ -1554,6 +1554,7 @@ void prec_entry(const MIo<S, F> &io, int64_t n, S *h, int num_cu, hipStream_t st
 }
 template void prec_entry<half_t, float>(const MIo<half_t, float> &, int64_t, half_t *, int, hipStream_t);
 template void prec_entry<float, float>(const MIo<float, float> &, int64_t, float *, int, hipStream_t);
+template void prec_entry<double, double>(const MIo<double, double> &, int64_t, double *, int, hipStream_t);
 
 template <class S, class F> void prec_apply_io(Prec *P, const MIo<S, F> &io, hipStream_t st) {
   using ACC = typename Acc<S>::type;

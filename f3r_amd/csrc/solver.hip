@@ -1104,7 +1104,9 @@ struct Solver {
   template <class T> void level4(const T *in, T *out, half_t *hz = nullptr) {
     if (capturing() && calls % cap_every == 0) {
       float *dst = cap->as<float>() + (int64_t)cap_n * n;
-      // a basis vector still to be normalised is recorded as it is
+      // the HALF nest records a basis vector still to be normalised as it is;
+      // the others normalise it first, as their entry would
+      if (p.variant != 0 || !glev.empty()) normalise_pending<T>();
       const T *src = pending.col == in ? static_cast<const T *>(pending.w) : in;
       if constexpr (std::is_same<T, float>::value)
         F3R_HIP(hipMemcpyAsync(dst, src, sizeof(float) * n, hipMemcpyDeviceToDevice, st()));
@@ -1198,10 +1200,10 @@ struct Solver {
   // ------------------------------------ generic levels (depth ablations) ---
   // w and its norm written to the basis column they belong to, where the
   // column's first reader does not do it itself
-  void normalise_pending() {
+  template <class T> void normalise_pending() {
     if (!pending.col) return;
-    MIo<float, float> io = entry_io<float, float>(static_cast<const float *>(pending.col));
-    prec_entry<float, float>(io, n, nullptr, ctx->num_cu, st());
+    MIo<T, T> io = entry_io<T, T>(static_cast<const T *>(pending.col));
+    prec_entry<T, T>(io, n, nullptr, ctx->num_cu, st());
   }
   // M applied directly to a vector of the caller's storage SI, scaled by s_in
   template <class SI> void mdirect(const SI *in, SI *out, float s_in) {
@@ -1235,7 +1237,7 @@ struct Solver {
     const int64_t nn = n;
     const dim3 g(grid()), b(kBlock);
     const double s_op = op_dtype == F3R_F16 ? (double)range_s : 1.0;
-    if constexpr (std::is_same<SI, float>::value) normalise_pending();
+    if constexpr (std::is_same<SI, float>::value) normalise_pending<float>();
     auto to_op = [&](auto tag) {
       using T = decltype(tag);
       hipLaunchKernelGGL((k_g_entry<SI, T>), g, b, 0, st(), nn, in, op_in->as<T>(), s_op / s_in);

@@ -440,8 +440,9 @@ int f3r_batch_info(f3r_batch B, int64_t *rows, int32_t *segments);
 int f3r_batch_destroy(f3r_batch B);
 
 /* record copies of the innermost level's input vectors during later solves:
- * every `every`-th call, up to `max_vectors` (0 stops and frees).  Level 2
- * runs without HIP graphs while vectors are being recorded.  These are the
+ * every `every`-th call, up to `max_vectors` (0 stops and frees).  The F3R
+ * nest's HALF build records a basis vector before its normalisation (up to a
+ * scale), the others the unit vector.  Level 2 runs without HIP graphs while vectors are being recorded.  These are the
  * probe vectors of the learned correction below; the reference has no
  * counterpart (its Richardson operator receives the same vectors, src/f3r-gpu.cpp:229-231). */
 int f3r_solver_capture(f3r_solver S, int32_t max_vectors, int32_t every);

@@ -251,6 +251,34 @@ def test_capture_first_vector_is_rhs(ctx):
     assert S.captured().shape == (8, A.n)
 
 
+@pytest.mark.parametrize("build", ["half", "float", "double", "nest"])
+def test_captured_vectors_are_unit_vectors(ctx, build):
+    """the innermost level's inputs are unit vectors; only the HALF nest
+    records its basis vectors before their normalisation.  Recording changes
+    no bit of the solve"""
+    import f3r_amd as F
+    A, _ = _system(F, m=10)
+    P = F.SDAINV(A, 0.1, 1.0, {"float": "f32", "double": "f64"}.get(build, "f16"), ctx=ctx)
+    b = F.vector.from_numpy(ctx, np.random.default_rng(2).uniform(-1, 1, A.n))
+    x = [F.vector(ctx, "f64", A.n).fill(0.0) for _ in range(2)]
+    if build == "nest":
+        level = F.FGMRES("f32", F.AutoRichardson("f16", P, 2, 64), 6)
+        S = F.Restarted(ctx, A, F.FGMRES("f64", level, 100, normalize=True, T="f64"), 20)
+    else:
+        S = F.F3R(ctx, A, P, variant=build)
+    S.solve(b, x[0])
+    F.F3R.capture(S, 40)
+    S.solve(b, x[1])
+    norms = np.linalg.norm(F.F3R.captured(S).astype(np.float64), axis=1)
+    print(build, norms[:6], flush=True)
+    assert np.array_equal(x[0].download(), x[1].download())
+    assert norms.size >= 10 and abs(norms[0] - 1) <= 1e-6
+    if build == "half":
+        assert np.all(norms > 0)
+    else:  # fp32 norms of 1000 elements
+        assert np.abs(norms - 1).max() <= 1e-5
+
+
 def test_training_lowers_loss_and_learned_solve_converges(ctx):
     import f3r_amd as F
     from f3r_amd import learn
