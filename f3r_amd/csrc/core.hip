@@ -242,6 +242,11 @@ template <class S, int R, int NW> constexpr int bj_segment() {
   while (2 * m * (int)sizeof(BjRecord<S, R>) <= 16384) m *= 2;
   return m;
 }
+// LDS of a workgroup: two segments, the block's vector of `bytes` and its zero
+// slot; at most 154 KB of the CU's 160 KB
+template <class S, int R, int NW> constexpr size_t bj_lds_bytes(size_t bytes) {
+  return (2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>) + bytes + sizeof(S) + 15) / 16 * 16;
+}
 // Barrier for LDS traffic only: this wave's LDS operations complete, then
 // s_barrier.  __syncthreads() would also wait for every outstanding global
 // load (its release fence), i.e. for the segment on its way.  The memory
@@ -1427,7 +1432,7 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
         maxe = std::max(maxe, L.rptr[i + 1] - L.rptr[i] - 1);
         maxe = std::max(maxe, U.rptr[i + 1] - U.rptr[i] - 1);
       }
-      const size_t es = dtype_size(P->dtype), lds = (size_t)(bsz + 1) * es;
+      const size_t es = dtype_size(P->dtype);
       // byte offsets in xs are 16-bit numbers
       if (maxe <= 16 && maxrows > 0 && (size_t)bsz * es <= kBjLdsBytes) {
         P->bj_R = maxe <= 3 ? 3 : maxe <= 7 ? 7 : 16;
@@ -1448,10 +1453,13 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
           up(P->bj_rec, rec.data(), sizeof(rec[0]) * rec.size());
           up(P->bj_blk, blk.data(), sizeof(int2) * blk.size());
           F3R_HIP(hipStreamSynchronize(c->stream));
-          P->bj_lds = (lds + 2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>) + 15) / 16 * 16;
-          // up to 154 KB of the CU's 160 KB
+          static_assert(bj_lds_bytes<S, R, NW>(kBjLdsBytes) <= 160 * 1024, "the CU's LDS");
+          P->bj_lds = bj_lds_bytes<S, R, NW>((size_t)bsz * es);
+          // the limit is the kernel's, shared by every preconditioner of its
+          // record shape: the most that any of them takes
           F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, typename Acc<S>::type, R, NW>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)P->bj_lds));
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)bj_lds_bytes<S, R, NW>(kBjLdsBytes)));
         });
       }
     }

@@ -396,6 +396,24 @@ def test_csr_spmv_lanes_per_row(ctx, tpr, vd, xd, yd):
         assert np.all(np.abs(got - exact) <= tol), (name, float(np.max(np.abs(got - exact) - tol)))
 
 
+@pytest.mark.parametrize("dtype", ["f64", "f16"])
+def test_bjilu0_large_blocks_after_small(ctx, dtype):
+    """a preconditioner of large blocks still runs after one of small blocks
+    with the same records was built (their kernel's LDS limit is shared)"""
+    import f3r_amd as F
+    A = _coupled(32 * 8192, [600], 11)
+    x = F.vector.from_numpy(ctx, np.random.default_rng(8).uniform(-1, 1, A.n), dtype)
+    ys = [F.vector(ctx, dtype, A.n) for _ in range(2)]
+    large = F.ILU0(A, blocks=32, acc=1.0, dtype=dtype, ctx=ctx)
+    large.operate(x, ys[0])
+    small = F.ILU0(A, blocks=256, acc=1.0, dtype=dtype, ctx=ctx)
+    print(f"bjilu0 large blocks after small {dtype}", flush=True)
+    large.operate(x, ys[1])
+    assert np.array_equal(ys[0].download(), ys[1].download())
+    small.operate(x, ys[1])
+    assert not np.array_equal(ys[0].download(), ys[1].download())
+
+
 @pytest.mark.parametrize("lens", [[8] * 256,                      # one block's run fills the staging exactly
                                   [8] * 255 + [9],                # one entry more: read row by row
                                   [8] * 257, [0] * 300, [1, 0, 5] * 200,
