@@ -1599,10 +1599,11 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
   }
   {
     HostCSR big = NR > 1 ? concat(msys, moff, NM) : concat(pa, B->off, N);
+    const std::vector<int64_t> &parts = NR > 1 ? moff : B->off;
     // fp16 copy: K = 8 once rows average 12 entries (a 27-point row then
     // takes 4 slot groups instead of 7; a 7-point row takes 1 either way)
     const int K16 = p.K > 0 ? p.K : (big.nnz() >= (int64_t)12 * big.n ? 8 : 4);
-    HostSell hs = build_sell(big, C, 1, K, nullptr, false, offsets);
+    HostSell hs = build_sell(big, C, 1, K, nullptr, false, offsets, &parts);
     B->sh = upload_sell_shared(c, hs, false);
     B->A64 = upload_sell_values(c, hs, F3R_F64);
     B->A32 = upload_sell_values(c, hs, F3R_F32);
@@ -1610,7 +1611,7 @@ BatchSolver *batch_create(std::shared_ptr<Context> ctx, const std::vector<std::s
       B->sh16 = B->sh;
       B->A16 = upload_sell_values(c, hs, F3R_F16);
     } else {
-      HostSell h16 = build_sell(big, C, 1, K16, nullptr, false, offsets);
+      HostSell h16 = build_sell(big, C, 1, K16, nullptr, false, offsets, &parts);
       B->sh16 = upload_sell_shared(c, h16, false);
       B->A16 = upload_sell_values(c, h16, F3R_F16);
     }

@@ -201,9 +201,13 @@ struct HostSell {
 // inverse permutation (the matrix P A P^T in sorted order).  With `offsets`
 // (and C >= 64) every chunk whose rows share a small set of column offsets
 // col - row, all in range and in CSR order, stores that set once instead of
-// a column index per slot.
+// a column index per slot.  parts: the first rows of independent diagonal
+// blocks in row order (multiples of C), the last entry the end: no slot, empty
+// ones included, then reads a column of another block (0 times a neighbour's
+// infinity is no zero).
 HostSell build_sell(const HostCSR &A, int32_t C, int32_t sigma, int32_t K,
-                    const std::vector<int32_t> *perm_override, bool renumber, bool offsets = false);
+                    const std::vector<int32_t> *perm_override, bool renumber, bool offsets = false,
+                    const std::vector<int64_t> *parts = nullptr);
 struct HostFactors {
   HostCSR f[2];
 };

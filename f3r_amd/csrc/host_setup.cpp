@@ -76,7 +76,8 @@ int64_t sell_nslots(int32_t n, const int32_t *rptr, int32_t C, int32_t sigma, in
 }
 
 HostSell build_sell(const HostCSR &A, int32_t C, int32_t sigma, int32_t K,
-                    const std::vector<int32_t> *perm_override, bool renumber, bool offsets) {
+                    const std::vector<int32_t> *perm_override, bool renumber, bool offsets,
+                    const std::vector<int64_t> *parts) {
   F3R_CHECK(C >= 1 && K >= 1 && sigma >= 1, F3R_ERR_ARG, "SELL: C, K and sigma must be >= 1");
   HostSell S;
   const int32_t n = A.n;
@@ -112,8 +113,8 @@ HostSell build_sell(const HostCSR &A, int32_t C, int32_t sigma, int32_t K,
       int32_t width = mx;
       if (offsets && mx > 0) {
         // eligible when every row's columns ascend (CSR order = offset
-        // order), every row + offset is a row of the matrix, and the union
-        // is at most 5/4 of the widest row.  Rows repeating the previous
+        // order), every row + offset is a row of the matrix (of the chunk's
+        // part), and the union is at most 5/4 of the widest row.  Rows repeating the previous
         // row's offsets (the stencil case) skip the merge.
         u.clear();
         first.clear();
@@ -137,7 +138,13 @@ HostSell build_sell(const HostCSR &A, int32_t C, int32_t sigma, int32_t K,
         if (ok) {
           std::sort(u.begin(), u.end());
           u.erase(std::unique(u.begin(), u.end()), u.end());
-          ok = (int64_t)u.size() * 4 <= (int64_t)mx * 5 && r0 + u.front() >= 0 && r0 + tc - 1 + u.back() < n;
+          int64_t lo = 0, hi = n;
+          if (parts) {
+            const auto e = std::upper_bound(parts->begin(), parts->end(), r0);
+            lo = e[-1];
+            hi = *e;
+          }
+          ok = (int64_t)u.size() * 4 <= (int64_t)mx * 5 && r0 + u.front() >= lo && r0 + tc - 1 + u.back() < hi;
         }
         if (ok) {
           uni[s] = u;
@@ -210,7 +217,7 @@ HostSell build_sell(const HostCSR &A, int32_t C, int32_t sigma, int32_t K,
       int32_t o = S.perm[r0 + j];
       int32_t len = A.rptr[o + 1] - A.rptr[o];
       expl_nnz[s] += len;
-      int32_t last = 0;
+      int32_t last = parts ? (int32_t)(r0 + j) : 0;  // of a row without entries
       for (int32_t q = 0; q < width; ++q) {
         int64_t pos = S.cptr[s] + ((int64_t)(q / K) * tc + j) * K + (q % K);
         if (q < len) {

@@ -225,12 +225,12 @@ std::shared_ptr<QuadSet> build_quads(Context *c, const SellShared &sh, const dou
       last = key;
       last_tab = tab;
     }
-    // every row of the block reads every offset of the table
+    // every row of the block reads every offset of the table, within its system
     if (tab >= 0) {
       const QuadTab &q = tabs[tab];
       const int64_t r0 = (int64_t)b * kQuadBlock, r1 = std::min<int64_t>(sh.n, r0 + kQuadBlock);
       const int32_t lo = q.u[0], hi = q.nruns ? q.u[q.nruns - 1] + q.m[q.nruns - 1] - 1 : 0;
-      if (r0 + lo < 0 || r1 - 1 + hi >= sh.n) tab = -1;
+      if (r0 + lo < sys[g] || r1 - 1 + hi >= sys[g + 1]) tab = -1;
       else umin = std::min(umin, lo);
     }
     if (tab >= 0) {

@@ -484,3 +484,35 @@ def test_lockstep_dots_added_up_by_the_update(m):
         one = F.F3R(ctx, A, P).solve(F.vector.from_numpy(ctx, b), y)
         assert abs(one.res_iter - r.res_iter) <= 1
     ctx.close()
+
+
+@pytest.mark.parametrize("nrhs", [1, 2, 4])
+@pytest.mark.parametrize("sizes", [[(7, 64), (7, 21), (27, 33)],   # value codes with several right-hand sides
+                                   [(7, 12), (27, 9), (7, 13)]])
+@pytest.mark.parametrize("index", [1, 0])
+def test_lockstep_nonfinite_segment_stays_alone(nrhs, sizes, index):
+    """a right-hand side that is not finite leaves every bit of the other
+    segments' solutions as it was: no padding slot, offset or code of one
+    system meets another's vectors"""
+    import f3r_amd as F
+    ctx = F.Context(0)
+    As, Ps = [], []
+    for s, (npts, m) in enumerate(sizes):
+        A = F.CSR.dominant(npts, m, margin=0.6 + 0.3 * s)
+        F.algorithm.scaling(A)
+        As += [A] * nrhs
+        Ps += [F.SDAINV(A, 0.1, 1.0, "f16", ctx=ctx)] * nrhs
+    B = F.Batch(ctx, As, Ps, m=(6, 3, 2, 2), restart=1, index=index, K=0 if index else 4)
+    bs = [F.uniform(A.n, -1.0, 1.0, seed=7 + k) for k, A in enumerate(As)]
+
+    def solve(bad):
+        xs = [F.vector(ctx, "f64", A.n).fill(0.0) for A in As]
+        B.solve([F.vector.from_numpy(ctx, np.full(A.n, np.nan) if k == bad else b)
+                 for k, (A, b) in enumerate(zip(As, bs))], xs)
+        return [x.download() for x in xs]
+    want = solve(None)
+    for bad in range(len(As)):
+        print(f"lockstep nonfinite segment nrhs={nrhs} sizes={sizes} index={index} bad={bad}", flush=True)
+        got = solve(bad)
+        assert [k for k in range(len(As)) if not np.array_equal(got[k], want[k])] == [bad]
+    ctx.close()
