@@ -1792,10 +1792,13 @@ int f3r_batch_solve(f3r_batch B, const f3r_vec *b, f3r_vec *x, f3r_result *res) 
   hipStream_t st = S->ctx->stream;
   const int nseg = S->nseg;
   std::vector<double> nrm_b(nseg);
+  // kernels reach the callers' vectors on this GPU; those on another are copied
+  bool here = true;
   for (int s = 0; s < nseg; ++s) {
     Vec *bv = vec_of(b[s]), *xv = vec_of(x[s]);
     F3R_CHECK(bv && xv && bv->dtype == F3R_F64 && xv->dtype == F3R_F64 && bv->n == S->nrow[s] && xv->n == S->nrow[s],
               F3R_ERR_ARG, "batch_solve: b and x of each segment: fp64 vectors of its matrix size");
+    here = here && bv->ctx->device == S->ctx->device && xv->ctx->device == S->ctx->device;
   }
   F3R_HIP(hipStreamSynchronize(st));  // the last solve's reads of the pinned pointers
   for (int s = 0; s < nseg; ++s) {
@@ -1803,8 +1806,20 @@ int f3r_batch_solve(f3r_batch B, const f3r_vec *b, f3r_vec *x, f3r_result *res) 
     S->xp[s] = static_cast<double *>(vec_of(x[s])->ptr());
   }
   const int32_t *rows = S->rows->as<int32_t>(), *bseg = S->bs(), *sb0 = S->sb0->as<int32_t>();
-  hipLaunchKernelGGL(k_b_take, dim3(S->G), dim3(kBlock), 0, st, S->bp, (const double *const *)S->xp, rows, bseg, sb0,
-                     S->b_int->as<double>(), S->x_int->as<double>(), S->partial->as<double>());
+  if (here) {
+    hipLaunchKernelGGL(k_b_take, dim3(S->G), dim3(kBlock), 0, st, S->bp, (const double *const *)S->xp, rows, bseg, sb0,
+                       S->b_int->as<double>(), S->x_int->as<double>(), S->partial->as<double>());
+  } else {
+    F3R_HIP(hipMemsetAsync(S->b_int->p, 0, sizeof(double) * S->N, st));
+    F3R_HIP(hipMemsetAsync(S->x_int->p, 0, sizeof(double) * S->N, st));
+    for (int s = 0; s < nseg; ++s) {
+      const size_t bytes = sizeof(double) * S->nrow[s];
+      F3R_HIP(hipMemcpyAsync(S->b_int->as<double>() + S->off[s], S->bp[s], bytes, hipMemcpyDeviceToDevice, st));
+      F3R_HIP(hipMemcpyAsync(S->x_int->as<double>() + S->off[s], S->xp[s], bytes, hipMemcpyDeviceToDevice, st));
+    }
+    hipLaunchKernelGGL(k_b_norm2<double>, dim3(S->G), dim3(kBlock), 0, st, (const double *)S->b_int->as<double>(),
+                       S->partial->as<double>());
+  }
   // no rotation (j = -1), no Hessenberg column: the norm itself
   hipLaunchKernelGGL(k_b_norm_finish<double>, dim3(nseg), dim3(kBlock), 0, st, (const double *)S->partial->as<double>(),
                      sb0, (const int32_t *)S->snb->as<int32_t>(), S->L1.e->as<double>(), (int64_t)(S->L1.m + 1),
@@ -1817,8 +1832,13 @@ int f3r_batch_solve(f3r_batch B, const f3r_vec *b, f3r_vec *x, f3r_result *res) 
   S->solve(nrm_b, r);
   F3R_HIP(hipStreamSynchronize(st));
   const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-  hipLaunchKernelGGL(k_b_give, dim3(S->G), dim3(kBlock), 0, st, (const double *)S->x_int->as<double>(), S->xp, rows,
-                     bseg, sb0);
+  if (here)
+    hipLaunchKernelGGL(k_b_give, dim3(S->G), dim3(kBlock), 0, st, (const double *)S->x_int->as<double>(), S->xp, rows,
+                       bseg, sb0);
+  else
+    for (int s = 0; s < nseg; ++s)
+      F3R_HIP(hipMemcpyAsync(S->xp[s], S->x_int->as<double>() + S->off[s], sizeof(double) * S->nrow[s],
+                             hipMemcpyDeviceToDevice, st));
   F3R_HIP(hipGetLastError());
   for (int s = 0; s < nseg; ++s) {
     r[s].solve_s = secs;

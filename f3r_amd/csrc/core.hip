@@ -743,9 +743,9 @@ void vec_copy(Vec *s, Vec *d) {
   hipStream_t st = d->ctx->stream;
   if (s->dtype == d->dtype) {
     // a copy kernel costs the host a third of a copy command; beyond 1 MB the
-    // copy itself is what counts
+    // copy itself is what counts, and a kernel may not reach another GPU's memory
     const size_t es = dtype_size(s->dtype);
-    if (s->n && s->n * es <= (1 << 20)) {
+    if (s->n && s->n * es <= (1 << 20) && s->ctx->device == d->ctx->device) {
       const dim3 g(grid_for(s->n, d->ctx->num_cu)), b(kBlock);
       if (es == 8) hipLaunchKernelGGL(k_copy<uint64_t>, g, b, 0, st, (const uint64_t *)s->ptr(), (uint64_t *)d->ptr(), s->n);
       else if (es == 4) hipLaunchKernelGGL(k_copy<uint32_t>, g, b, 0, st, (const uint32_t *)s->ptr(), (uint32_t *)d->ptr(), s->n);

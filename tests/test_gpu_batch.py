@@ -516,3 +516,34 @@ def test_lockstep_nonfinite_segment_stays_alone(nrhs, sizes, index):
         got = solve(bad)
         assert [k for k in range(len(As)) if not np.array_equal(got[k], want[k])] == [bad]
     ctx.close()
+
+
+def test_vectors_of_another_gpu():
+    """copies and lockstep solves take vectors of a context on another GPU,
+    made by the thread that uses that GPU"""
+    from concurrent.futures import ThreadPoolExecutor
+    import f3r_amd as F
+    if F.device_count() < 2:
+        pytest.skip("needs two GPUs")
+    ctx = F.Context(0)
+    As = [F.CSR.dominant(7, m, margin=0.7) for m in (12, 9)]
+    for A in As:
+        F.algorithm.scaling(A)
+    B = F.Batch(ctx, As, [F.SDAINV(A, 0.1, 1.0, "f16", ctx=ctx) for A in As])
+
+    def vectors(c):
+        out = ([F.vector.from_numpy(c, F.uniform(A.n, -1.0, 1.0, seed=k)) for k, A in enumerate(As)],
+               [F.vector(c, "f64", A.n).fill(0.0) for A in As])
+        c.sync()
+        return out
+
+    with ThreadPoolExecutor(1) as other:
+        far = other.submit(F.Context, 1).result()
+        fb, fx = other.submit(vectors, far).result()
+        nb, nx = vectors(ctx)
+        assert np.array_equal(F.vector(ctx, "f64", As[0].n).copy(fb[0]).download(), nb[0].download())
+        for b, x in ((nb, nx), (fb, fx)):
+            assert all(r.is_solved for r in B.solve(b, x))
+        got = other.submit(lambda: [x.download() for x in fx]).result()
+    for a, b in zip(got, nx):
+        assert np.array_equal(a, b.download())
