@@ -1708,6 +1708,7 @@ void solver_solve(Solver *S, Vec *b, Vec *x, f3r_result *res) {
     F3R_HIP(hipMemcpyAsync(S->b_int->p, b->ptr(), 8 * n, hipMemcpyDeviceToDevice, c->stream));
     F3R_HIP(hipMemcpyAsync(S->x_int->p, x->ptr(), 8 * n, hipMemcpyDeviceToDevice, c->stream));
   }
+  S->pending = {};  // of a call that ended with an error
   // reset the adaptive weights (src/f3r-gpu.cpp:277-281)
   S->cnt = S->p.c;
   S->calls = 0;
@@ -1958,6 +1959,7 @@ int f3r_solver_level_apply(f3r_solver S, int32_t level, f3r_vec in, f3r_vec out)
             "level_apply: a depth ablation applies its whole nest as level 2 only");
   const int64_t n = s->n;
   const dim3 g(s->grid()), b(kBlock);
+  s->pending = {};
   s->cnt = s->p.c;
   hipLaunchKernelGGL(k_rich_reset, dim3(1), dim3(64), 0, s->st(), s->rich->as<RichDev>(), s->p.static_weight);
   if (level == 2) {
