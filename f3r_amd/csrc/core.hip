@@ -221,8 +221,8 @@ __global__ __launch_bounds__(1024) void k_bj_trsv_u(const int32_t *__restrict__ 
 // values in visiting order, 1/u_ii) form one stream per block in solving
 // order.  It passes through LDS in segments of SR records: two are resident,
 // the third is on its way in registers, so the memory latency overlaps two
-// segments of work however narrow the levels are.  Wide levels (NW = 4) use
-// four waves and a barrier per batch.  Records read level by level from
+// segments of work however narrow the levels are.  Wide levels take a batch on
+// NW = 4, 8 or 16 waves, with a barrier per batch.  Records read level by level from
 // global memory, four levels ahead, took 87 us at 64^3 / 112 blocks: 0.43 us
 // a level, the memory latency over four.
 // The wave's own instructions then count (about 40 a batch), so a record is
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(1024) void k_bj_trsv_u(const int32_t *__restrict__ 
 // dinv = 1, so L and U are one stream.  Measured at 64^3 / 112 blocks: 43 us
 // with batch sizes, tests and two streams.
 template <class S, int R> struct alignas(8) BjRecord {
-  uint16_t row, col[R];  // byte offsets into xs; bit 0 of row: last of its batch (one wave) or no row (four)
+  uint16_t row, col[R];  // byte offsets into xs; bit 0 of row: last of its batch (one wave) or no row (more)
   S val[R];
   S dinv;
 };
@@ -243,7 +243,9 @@ template <class S, int R, int NW> constexpr int bj_segment() {
   return m;
 }
 // LDS of a workgroup: two segments, the block's vector of `bytes` and its zero
-// slot; at most 154 KB of the CU's 160 KB
+// slot (at most 154 KB with one or four waves).  The CU's 160 KB less what the
+// kernel declares:
+constexpr size_t kCuLds = 160 * 1024 - 256;
 template <class S, int R, int NW> constexpr size_t bj_lds_bytes(size_t bytes) {
   return (2 * bj_segment<S, R, NW>() * sizeof(BjRecord<S, R>) + bytes + sizeof(S) + 15) / 16 * 16;
 }
@@ -254,8 +256,8 @@ template <class S, int R, int NW> constexpr size_t bj_lds_bytes(size_t bytes) {
 __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Solves the block's stream of nseg segments at `src`; the first two are in
-// the ring already.  NW = 1: batches end where a record says so.  NW = 4: a
-// batch is 256 records (levels padded by records without a row).
+// the ring already.  NW = 1: batches end where a record says so.  NW > 1: a
+// batch is 64 NW records (levels padded by records without a row).
 template <class S, int R, int NW>
 __device__ __forceinline__ void bj_solve(const BjRecord<S, R> *__restrict__ srec, int nseg, int nrec, S *xs,
                                          unsigned char *ring) {
@@ -319,9 +321,13 @@ __device__ __forceinline__ void bj_solve(const BjRecord<S, R> *__restrict__ srec
   }
 }
 
+// threads of a workgroup: all move the vector, 64 NW solve
+constexpr int bj_threads(int NW) { return NW * kWave > kBlock ? NW * kWave : kBlock; }
 template <class S, class F, int R, int NW>
-__global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, const BjRecord<S, R> *__restrict__ recs,
-                                                   const int2 *__restrict__ blk, MIo<S, F> io) {
+__global__ __launch_bounds__(bj_threads(NW)) void k_bj_lds(int32_t n, int32_t bsz,
+                                                           const BjRecord<S, R> *__restrict__ recs,
+                                                           const int2 *__restrict__ blk, MIo<S, F> io) {
+  constexpr int kT = bj_threads(NW);
   extern __shared__ __align__(16) unsigned char bj_smem[];
   constexpr int kRing = 2 * bj_segment<S, R, NW>() * (int)sizeof(BjRecord<S, R>);
   S *xs = reinterpret_cast<S *>(bj_smem + kRing);
@@ -339,20 +345,20 @@ __global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, const
     const Unit *src = reinterpret_cast<const Unit *>(srec);
     Unit *dst = reinterpret_cast<Unit *>(bj_smem);
 #pragma unroll 8
-    for (int i = threadIdx.x; i < 2 * kSegUnits; i += kBlock) dst[i] = src[nseg > 1 || i < kSegUnits ? i : i - kSegUnits];
+    for (int i = threadIdx.x; i < 2 * kSegUnits; i += kT) dst[i] = src[nseg > 1 || i < kSegUnits ? i : i - kSegUnits];
   }
   if (threadIdx.x == 0) xs[bsz] = S(0);  // the zero slot
   // all waves move the vector, 8 rows in flight each
   if (io.raw) {
     const MEntry<S, F> en(io);
-    for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kBlock) {
+    for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kT) {
       F v[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = i0 + q * kBlock < nr ? io.raw[r0 + i0 + q * kBlock] : F(0);
+      for (int q = 0; q < 8; ++q) v[q] = i0 + q * kT < nr ? io.raw[r0 + i0 + q * kT] : F(0);
 #pragma unroll
       for (int q = 0; q < 8; ++q)
-        if (i0 + q * kBlock < nr) {
-          const int32_t i = i0 + q * kBlock;
+        if (i0 + q * kT < nr) {
+          const int32_t i = i0 + q * kT;
           const F vn = en.norm(v[q]);
           const S h = en.store(vn);
           if (io.vout) io.vout[r0 + i] = vn;
@@ -361,20 +367,20 @@ __global__ __launch_bounds__(kBlock) void k_bj_lds(int32_t n, int32_t bsz, const
         }
     }
   } else {
-    for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kBlock) {
+    for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kT) {
       S v[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = i0 + q * kBlock < nr ? io.in[r0 + i0 + q * kBlock] : S(0);
+      for (int q = 0; q < 8; ++q) v[q] = i0 + q * kT < nr ? io.in[r0 + i0 + q * kT] : S(0);
 #pragma unroll
       for (int q = 0; q < 8; ++q)
-        if (i0 + q * kBlock < nr) xs[i0 + q * kBlock] = v[q];
+        if (i0 + q * kT < nr) xs[i0 + q * kT] = v[q];
     }
   }
   __syncthreads();
   if (threadIdx.x < 64 * NW) bj_solve<S, R, NW>(srec, nseg, bk.y, xs, bj_smem);
   __syncthreads();
   const MExit<S, F> mo(io);
-  for (int32_t i = threadIdx.x; i < nr; i += kBlock) mo.put(r0 + i, xs[i], mo.pre(r0 + i));
+  for (int32_t i = threadIdx.x; i < nr; i += kT) mo.put(r0 + i, xs[i], mo.pre(r0 + i));
 }
 
 // ------------------------------------------ M with its entry and update ---
@@ -1132,7 +1138,7 @@ static void group_by_block(const std::vector<int32_t> &rows, const std::vector<i
 // Record streams of the triangular factors for k_bj_lds: the rows of each
 // block in the grouped order (`brows`, block by block and level by level), L's
 // and then U's, padded to whole segments.  A batch is at most 64 NW rows of
-// one level (NW = 4: padded to 256 records).
+// one level (NW > 1: padded to 64 NW records).
 struct BjRows {
   const HostCSR &M;
   const std::vector<int32_t> &brows, &blptr, &bstart;
@@ -1214,7 +1220,9 @@ static void bj_stream(const BjRows &L, const BjRows &U, int32_t bsz, std::vector
 template <class F> static void bj_dispatch(int dtype, int R, int NW, F f) {
   auto by_nw = [&](auto s, auto r) {
     if (NW == 1) f(s, r, std::integral_constant<int, 1>());
-    else f(s, r, std::integral_constant<int, 4>());
+    else if (NW == 4) f(s, r, std::integral_constant<int, 4>());
+    else if (NW == 8) f(s, r, std::integral_constant<int, 8>());
+    else f(s, r, std::integral_constant<int, 16>());
   };
   auto by_r = [&](auto s) {
     if (R == 3) by_nw(s, std::integral_constant<int, 3>());
@@ -1433,13 +1441,29 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
         maxe = std::max(maxe, U.rptr[i + 1] - U.rptr[i] - 1);
       }
       const size_t es = dtype_size(P->dtype);
-      // byte offsets in xs are 16-bit numbers
-      if (maxe <= 16 && maxrows > 0 && (size_t)bsz * es <= kBjLdsBytes) {
+      // byte offsets in xs are 16-bit numbers; diagonal blocks have no chain to
+      // shorten, and their records are mostly unused entries (917 K rows in
+      // fp32: 11.7 us by k_bj_trsv, 15.7 with records)
+      if (maxe > 0 && maxe <= 16 && maxrows > 0 && (size_t)bsz * es <= kBjLdsBytes) {
         P->bj_R = maxe <= 3 ? 3 : maxe <= 7 ? 7 : 16;
         // one wave up to 128 rows per level on average (two batches); wider
-        // levels on four waves with a barrier per batch
-        const double levels = (double)(lbl.size() + ubl.size()) - 2.0 * P->bj_groups;
-        P->bj_waves = 2.0 * n <= 128.0 * levels ? 1 : 4;
+        // levels on as many waves as take the average level in one batch, with
+        // a barrier per batch.  917 K rows in 112 blocks, 3 entries a row, us
+        // with 4 / 8 / 16 waves, fp16 and fp64: 200 rows a level 30 / 29 / 36
+        // and 44 / 52 / 106, 512 rows 22 / 16 / 18 and 37 / 26 / 36, 910 rows
+        // 24 / 17 / 13 and 38 / 27 / 24; k_bj_trsv 2731 rows 25 and 28, here
+        // 13 and 24
+        const double levels = (double)(lbl.size() + ubl.size()) - 2.0 * P->bj_groups, width = 2.0 * n / levels;
+        P->bj_waves = width <= 128 ? 1 : width <= 256 ? 4 : width <= 512 ? 8 : 16;
+        // as many waves as the CU's LDS holds segments for
+        auto fits = [&] {
+          bool ok = false;
+          bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
+            ok = bj_lds_bytes<decltype(s), decltype(r)::value, decltype(w)::value>((size_t)bsz * es) <= kCuLds;
+          });
+          return ok;
+        };
+        while (P->bj_waves > 4 && !fits()) P->bj_waves /= 2;
         bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
           using S = decltype(s);
           constexpr int R = decltype(r)::value, NW = decltype(w)::value;
@@ -1453,13 +1477,12 @@ void prec_build_device(Prec *P, const std::vector<int32_t> *perm, int32_t C, int
           up(P->bj_rec, rec.data(), sizeof(rec[0]) * rec.size());
           up(P->bj_blk, blk.data(), sizeof(int2) * blk.size());
           F3R_HIP(hipStreamSynchronize(c->stream));
-          static_assert(bj_lds_bytes<S, R, NW>(kBjLdsBytes) <= 160 * 1024, "the CU's LDS");
           P->bj_lds = bj_lds_bytes<S, R, NW>((size_t)bsz * es);
           // the limit is the kernel's, shared by every preconditioner of its
           // record shape: the most that any of them takes
           F3R_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_bj_lds<S, typename Acc<S>::type, R, NW>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)bj_lds_bytes<S, R, NW>(kBjLdsBytes)));
+                                      (int)std::min(kCuLds, bj_lds_bytes<S, R, NW>(kBjLdsBytes))));
         });
       }
     }
@@ -1480,9 +1503,9 @@ template <class S, class F> static void bj_apply(Prec *P, const MIo<S, F> &io, h
   const int32_t blocks = P->bj_blocks, bsz = (P->n + blocks - 1) / blocks;
   bj_dispatch(P->dtype, P->bj_R, P->bj_waves, [&](auto s, auto r, auto w) {
     if constexpr (std::is_same<decltype(s), S>::value)
-      hipLaunchKernelGGL((k_bj_lds<S, F, decltype(r)::value, decltype(w)::value>), dim3(P->bj_groups), dim3(kBlock),
-                         P->bj_lds, st, P->n, bsz, P->bj_rec->as<BjRecord<S, decltype(r)::value>>(),
-                         P->bj_blk->as<int2>(), io);
+      hipLaunchKernelGGL((k_bj_lds<S, F, decltype(r)::value, decltype(w)::value>), dim3(P->bj_groups),
+                         dim3(bj_threads(decltype(w)::value)), P->bj_lds, st, P->n, bsz,
+                         P->bj_rec->as<BjRecord<S, decltype(r)::value>>(), P->bj_blk->as<int2>(), io);
   });
 }
 

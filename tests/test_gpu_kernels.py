@@ -261,8 +261,11 @@ def _coupled(n, dists, seed):
     (33 * 97, 33, [1, 2, 5, 30, 31]),          # 7 entries a row at most
     (20000, 40, list(range(1, 14))),           # 13 entries: the widest records
     (20011, 40, list(range(1, 17))),           # 16
-    (40007, 32, [600]),                        # 600 rows per level: four waves
-    (40007, 32, [300, 301, 302, 303, 304]),
+    (40007, 32, [200]),                        # 200 rows per level: four waves
+    (40007, 32, [300, 301, 302, 303, 304]),    # eight
+    (40007, 32, [600]),                        # sixteen
+    (32 * 8192, 32, [900]),                    # with the fp64 vector of 64 KB
+    (40009, 37, [700 + k for k in range(16)]), # the widest records: fewer waves fit the LDS
     (40009, 37, [290 + k for k in range(16)]),
     (4096, 64, []),                            # diagonal blocks: one level
     (32 * 16384, 32, [128]),                   # a block's fp32 vector fills 64 KB exactly
