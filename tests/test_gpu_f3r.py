@@ -129,6 +129,43 @@ def test_level3_close(ctx, kind):
     assert err < 1e-3, err
 
 
+@pytest.mark.parametrize("kind", ["diagonal", "band", "general", "ilu0", "bjilu0", "bjilu0-wide"])
+@pytest.mark.parametrize("variant", ["half", "float", "double"])
+def test_level3_entries(ctx, kind, variant):
+    """level 3's steps after the first enter M with a basis vector still to be
+    normalised (its norm as block sums): every kind of M against the oracle"""
+    import f3r_amd as F
+    if kind == "diagonal":
+        A = _problem("27pt", 20)
+    elif kind in ("band", "bjilu0", "ilu0"):
+        A = _problem("lognormal", 20)
+    elif kind == "general":
+        A = _problem("convdiff", 20)
+    else:  # 700 rows a level
+        A = _banded(40 * 4200, [-700, 0, 700], [-0.5, -0.75], 4)
+        F.algorithm.scaling(A)
+    dt = {"half": "f16", "float": "f32", "double": "f64"}[variant]
+    kw = {"variant": {"half": 0, "float": 1, "double": 2}[variant], "ref_arith": 0}
+    if kind[:2] == "bj" or kind == "ilu0":
+        kw.update(precond=1, bj_blocks=8 if kind == "ilu0" else 40)
+        P = F.ILU0(A, blocks=kw["bj_blocks"], acc=1.0, dtype=dt, ctx=ctx)
+    else:
+        kw["tol"] = 0.02 if kind == "general" else 0.1
+        P = F.SDAINV(A, kw["tol"], 1.0, dt, ctx=ctx)
+    if variant == "half":
+        kw["range_scale"] = _scale(A.n)
+    S = F.F3R(ctx, A, P, variant=variant, range_scale=kw.get("range_scale", 0.0), use_graph=False)
+    v = np.random.default_rng(2).uniform(-1, 1, A.n)
+    v /= np.linalg.norm(v)
+    vin, vout = F.vector.from_numpy(ctx, v), F.vector(ctx, "f64", A.n)
+    print(f"level 3 entries {kind} {variant} n={A.n}", flush=True)
+    S.level_apply(3, vin, vout)
+    ref = O.level_apply(A.n, A.rptr, A.idx, A.val, 3, v, **kw)
+    err = np.linalg.norm(vout.download() - ref) / np.linalg.norm(ref)
+    # sums of at most 1.7e5 products in another order (2^-24 or 2^-53 n^0.5), through four steps
+    assert err < {"half": 1e-3, "float": 1e-4, "double": 1e-11}[variant], err
+
+
 def _true_res(A, x, b):
     r = b - O.spmv_ld(A.n, A.rptr, A.idx, A.val, x)
     return np.linalg.norm(r) / np.linalg.norm(b)
