@@ -467,8 +467,8 @@ def test_value_codes(ctx, kind, variant):
 
 
 def _level_pair(ctx, A, levels=(3,), n_inner=(2, 3, 4, 2), **kw):
-    """level applications of the DOUBLE build with value codes and, from the
-    int32-index layout, without: {level: (coded, plain)}"""
+    """level applications of the DOUBLE build with value codes (where the matrix
+    has them) and, from the int32-index layout, without: {level: (first, second)}"""
     import f3r_amd as F
     P = F.SDAINV(A, 0.1, 1.0, "f64", ctx=ctx, device=True)
     b = F.uniform(A.n, -1.0, 1.0, seed=3)
@@ -508,3 +508,32 @@ def test_value_codes_keep_to_the_callers_grid(ctx, grid):
     print(f"value codes grid={grid}", flush=True)
     got, want = _level_pair(ctx, A, cap_spmv=True, grid=grid)[3]
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("dims", [(104, 104, 98), (104, 101, 100)])   # 1,059,968 and 1,050,400 rows
+def test_value_codes_with_finished_dots(ctx, dims):
+    """above 1024 blocks of 1024 rows k_dots_finish adds the coded products'
+    block sums up"""
+    import f3r_amd as F
+    A = F.CSR.dominant(7, *dims, margin=0.7)
+    assert A.n > 1024 * 1024
+    F.algorithm.scaling(A)
+    print(f"value codes, finished dots n={A.n}", flush=True)
+    out = _level_pair(ctx, A, levels=(4, 3))
+    assert np.array_equal(*out[4])
+    # fp64 dots of 1.1e6 rows in another order: 2^-53 n^0.5 each, through four steps
+    assert np.linalg.norm(out[3][0] - out[3][1]) <= 1e-10 * np.linalg.norm(out[3][1])
+
+
+@pytest.mark.parametrize("n", [1024 * 256 + 1, 2048 * 256, 2048 * 256 + 1])
+def test_plain_dots_by_row_count(ctx, n):
+    """the plain product with dots: one row a thread up to 1024 blocks, two up
+    to 2048, then one again with the sums finished in a launch of their own;
+    against the same level on a grid of one row a thread"""
+    import f3r_amd as F
+    A = _banded(n, [-300, -1, 0, 1, 300], np.linspace(-.25, .25, 40), 5)
+    F.algorithm.scaling(A)
+    print(f"plain dots n={n}", flush=True)
+    want = _level_pair(ctx, A, cap_spmv=True, grid=4096)[3]
+    for got in _level_pair(ctx, A)[3]:
+        assert np.linalg.norm(got - want[0]) <= 1e-10 * np.linalg.norm(want[0])
