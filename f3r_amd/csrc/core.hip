@@ -350,7 +350,7 @@ __global__ __launch_bounds__(bj_threads(NW)) void k_bj_lds(int32_t n, int32_t bs
   if (threadIdx.x == 0) xs[bsz] = S(0);  // the zero slot
   // all waves move the vector, 8 rows in flight each
   if (io.raw) {
-    const MEntry<S, F> en(io);
+    const MEntry<S, F> en(io, std::bool_constant<(kT > kBlock)>());
     for (int32_t i0 = threadIdx.x; i0 < nr; i0 += 8 * kT) {
       F v[8];
 #pragma unroll

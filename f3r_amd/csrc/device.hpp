@@ -215,14 +215,15 @@ __device__ __forceinline__ void block_sum(T (&v)[NV], T *lds /* NV * kWavesPerBl
   __syncthreads();
 }
 
-// The sum of G partial sums in every thread of a block of at least kBlock
-// threads, the first of which add them, in the same order in every block (G a
-// few thousand at most: each block reads them all from L2).  The loads of a
+// The sum of G partial sums in every thread of a block of kBlock threads (WIDE:
+// of more, of which the first kBlock add), in the same order in every block (G
+// a few thousand at most: each block reads them all from L2).  The loads of a
 // round are issued together.
-template <class T> __device__ __forceinline__ T parts_sum(const T *__restrict__ p, int G) {
+template <class T, bool WIDE = false> __device__ __forceinline__ T parts_sum(const T *__restrict__ p, int G) {
   __shared__ T lds[kWavesPerBlock];
+  const bool adds = !WIDE || threadIdx.x < kBlock;
   T v = 0;
-  for (int b0 = threadIdx.x < kBlock ? threadIdx.x : G; b0 < G; b0 += 8 * kBlock) {
+  for (int b0 = adds ? threadIdx.x : G; b0 < G; b0 += 8 * kBlock) {
     T t[8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) t[q] = b0 + q * kBlock < G ? p[b0 + q * kBlock] : (T)0;
@@ -230,7 +231,7 @@ template <class T> __device__ __forceinline__ T parts_sum(const T *__restrict__ 
     for (int q = 0; q < 8; ++q) v += t[q];
   }
   v = wave_sum(v);
-  if (threadIdx.x < kBlock && (threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = v;
+  if (adds && (threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = v;
   __syncthreads();
   T s = lds[0];
 #pragma unroll

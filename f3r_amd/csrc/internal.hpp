@@ -86,13 +86,14 @@ template <class S, class F>
 void prec_entry(const MIo<S, F> &io, int64_t n, S *h, int num_cu, hipStream_t st);
 
 // the entry of one element (constructed by every thread of a block: the
-// block adds up the norm's partial sums)
+// block adds up the norm's partial sums; WIDE: a block of more than kBlock threads)
 template <class S, class F> struct MEntry {
   F iv, s;
   bool has_inv;
-  __device__ explicit MEntry(const MIo<S, F> &io) : iv(1), s(io.s), has_inv(io.npart != nullptr) {
+  template <class WIDE = std::false_type>
+  __device__ explicit MEntry(const MIo<S, F> &io, WIDE = WIDE()) : iv(1), s(io.s), has_inv(io.npart != nullptr) {
     if (!has_inv) return;
-    const F nv = sqrt(parts_sum<F>(io.npart, io.nparts));
+    const F nv = sqrt(parts_sum<F, WIDE::value>(io.npart, io.nparts));
     if (blockIdx.x == 0 && threadIdx.x == 0) *io.hnorm = nv;
     iv = (F)1 / nv;
   }
