@@ -481,13 +481,16 @@ template <class S, class F> struct EpiMExit {
 // less (9.7 and 7.5 us; the 7-point solve at 96^3 9.3 -> 7.9 ms).  A diagonal without an entry in a row holds a zero.
 // SYM: Z's diagonals are W's mirrored (W^T's pattern), so that one of the four
 // terms of each t is h_i itself.
+// SKIP: a zero entry takes no part, whatever it meets (0 times infinity is
+// NaN): for a caller's own vectors; in a solve one such number has reached
+// every row by the next dot.
 constexpr int kBand = 4;
 template <class S> struct Band {
   const S *w, *z;
   int32_t ow[kBand], oz[kBand];
   int32_t lo, hi;  // smallest and largest row reached from row 0
 };
-template <class S, class F, bool RAW, bool SYM>
+template <class S, class F, bool RAW, bool SYM, bool SKIP>
 __global__ __launch_bounds__(kBlock) void k_m_band(int32_t n, Band<S> bd, MIo<S, F> io) {
   using ACC = typename Acc<S>::type;
   using X = typename std::conditional<RAW, F, S>::type;
@@ -535,10 +538,15 @@ __global__ __launch_bounds__(kBlock) void k_m_band(int32_t n, Band<S> bd, MIo<S,
     ACC t = 0;
 #pragma unroll
     for (int b = 0; b < kBand; ++b) {
-      if constexpr (RAW) t = fma_<ACC>(to_acc(w[a].v[b]), (ACC)en(xv[a][b]), t);
-      else t = fma_<ACC>(to_acc(w[a].v[b]), to_acc(xv[a][b]), t);
+      ACC xe;
+      if constexpr (RAW) xe = (ACC)en(xv[a][b]);
+      else xe = to_acc(xv[a][b]);
+      if (SKIP && to_acc(w[a].v[b]) == 0) xe = 0;
+      t = fma_<ACC>(to_acc(w[a].v[b]), xe, t);
     }
-    acc = fma_<ACC>(to_acc(z.v[a]), to_acc(cvt<S>(t)), acc);
+    ACC te = to_acc(cvt<S>(t));
+    if (SKIP && to_acc(z.v[a]) == 0) te = 0;
+    acc = fma_<ACC>(to_acc(z.v[a]), te, acc);
   }
   if (row >= n) return;
   if constexpr (RAW) {
@@ -571,7 +579,7 @@ template <class A, class B> static bool apart(const A *p, const B *q, int64_t n)
   return !p || !q || a + n * sizeof(A) <= b || b + n * sizeof(B) <= a;
 }
 // rows gather x, so nothing that is written may lie over it
-template <class S, class F> static bool band_apply(Prec *P, const MIo<S, F> &io, hipStream_t st) {
+template <class S, class F> static bool band_apply(Prec *P, const MIo<S, F> &io, hipStream_t st, bool skip = false) {
   if (!P->bwz) return false;
   const int64_t n = P->n;
   const bool ok = io.raw ? apart(io.raw, io.out, n) && apart(io.raw, io.outf, n) && apart(io.raw, io.hin, n) &&
@@ -580,8 +588,9 @@ template <class S, class F> static bool band_apply(Prec *P, const MIo<S, F> &io,
   if (!ok) return false;
   bool sym = true;
   for (int k = 0; k < kBand; ++k) sym = sym && P->boz[k] == -P->bow[kBand - 1 - k];
-  auto kern = io.raw ? (sym ? k_m_band<S, F, true, true> : k_m_band<S, F, true, false>)
-                     : (sym ? k_m_band<S, F, false, true> : k_m_band<S, F, false, false>);
+  auto kern = io.raw ? (sym ? k_m_band<S, F, true, true, false> : k_m_band<S, F, true, false, false>)
+              : skip ? (sym ? k_m_band<S, F, false, true, true> : k_m_band<S, F, false, false, true>)
+                     : (sym ? k_m_band<S, F, false, true, false> : k_m_band<S, F, false, false, false>);
   hipLaunchKernelGGL(kern, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, (int32_t)n, band<S>(*P), io);
   return true;
 }
@@ -1549,7 +1558,7 @@ template <class S> static void sdainv_apply_t(Prec *P, const S *in, S *out, hipS
   MIo<S, ACC> io;
   io.in = in;
   io.out = out;
-  if (band_apply<S, ACC>(P, io, st)) return;
+  if (band_apply<S, ACC>(P, io, st, true)) return;
   S *tmp = P->tmp->as<S>();
   const bool wp = !P->W->sh->internal;
   SellArgs aw = sell_args(*P->W->sh, wp), az = sell_args(*P->Z->sh, wp);

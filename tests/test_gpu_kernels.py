@@ -641,3 +641,30 @@ def test_sdainv_band_form(ctx, dims, dtype):
     got, want = y.download(), x.download()
     assert np.all(np.isfinite(got.astype(np.float64))) and np.any(got != 0)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("dtype", ["f16", "f64"])
+def test_sdainv_band_form_with_nonfinite_input(ctx, dtype, bad):
+    """an element of the input that is not finite reaches the rows its factors
+    couple to it and no other: a diagonal's missing entries take no part"""
+    import f3r_amd as F
+    import scipy.sparse as sp
+    A = F.CSR.convdiff7(70, 5, 4, sigma=0.5, corr=4.0, peclet=0.0, seed=2)
+    F.algorithm.scaling(A)
+    P = F.SDAINV(A, 0.1, 1.0, dtype, ctx=ctx)
+    Z, W = (sp.csr_matrix((np.abs(v) + 1.0, i, r), shape=(A.n, A.n)) for r, i, v in P.factors())
+    x = F.uniform(A.n, -1.0, 1.0, seed=3).astype({"f16": np.float16, "f64": np.float64}[dtype])
+    y = F.vector(ctx, dtype, A.n)
+    P.operate(F.vector.from_numpy(ctx, x), y)
+    want = y.download()
+    for at in (0, 69, 70, 4 * 70 + 3, 5 * 70 - 1, 5 * 70, A.n // 2, A.n - 70, A.n - 1):
+        print(f"band form {dtype} {bad} at {at}", flush=True)
+        xb = x.copy()
+        xb[at] = bad
+        P.operate(F.vector.from_numpy(ctx, xb), y)
+        e = np.zeros(A.n)
+        e[at] = 1.0
+        reached = Z @ (W @ e) != 0
+        got = y.download()
+        assert not np.isfinite(got[reached]).any() and np.array_equal(got[~reached], want[~reached])
